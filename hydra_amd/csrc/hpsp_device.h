@@ -25,8 +25,15 @@ constexpr int waves_for(int N) { return N <= 4 ? 4 : (N <= 6 ? 3 : (N <= 10 ? 2 
 // is folded on the host (engine keys, final boost constants).
 struct DecayK {
   double m[HPSP_MAX_N];
+  double msum[HPSP_MAX_N];  // ((0 + m0) + m1) + ... + m[n], the chain's running sum
+  double msq[HPSP_MAX_N];   // m[n]^2
   double ecm;
   double maxw;
+  double mas0, masN;  // invMas[0] = 0 ecm + msum[0] and invMas[N-1] = 1 ecm + msum[N-1]
+  double rmasN;       // RN(1 / invMas[N-1])
+  // Every invMas lies in [2^-300, 2^300], where div_core divides exactly
+  // rounded: plain_m says so of the masses, plain of the masses and ecm.
+  int plain_m, plain;
   uint64_t key[4];  // engine key words, already splitmix-ed
   // Final boost of a single mother (Vector4R.inl:312-369) with its derived
   // constants, valid when do_boost != 0 (0 < b2 < 1).
@@ -357,6 +364,17 @@ __device__ __forceinline__ double to_unit(uint64_t w) {
     return (double)w * 0x1p-64;
 }
 
+// cos of the polar angle, 2 u - 1, of a word: exact for the 32-bit words
+// (w - 2^31 is w with its top bit flipped, read as signed).
+template <int ENGINE>
+__device__ __forceinline__ double to_cos(uint64_t w) {
+#pragma clang fp contract(off)
+  if constexpr (is_squares<ENGINE>())
+    return (double)(int32_t)((uint32_t)w ^ 0x80000000u) * 0x1p-31;
+  else
+    return 2 * to_unit<ENGINE>(w) - 1;
+}
+
 // In-register ascending sort of a small fixed-size array (odd-even
 // transposition network; any correct sort yields the same values).
 template <typename T, int K>
@@ -438,14 +456,11 @@ __device__ __forceinline__ void sincos_2pi_w32(uint32_t w, double& s, double& c)
 // contraction off itself, so the operation sequence holds in any translation
 // unit.
 
-// Correctly rounded FP64 square root: reciprocal-square-root estimate, one
-// Newton step on (g ~ sqrt(x), h ~ 1/(2 sqrt(x))), then two residual
-// corrections g += (x - g*g) * h (Markstein's scheme, as the AMDGPU backend
-// expands llvm.sqrt.f64).  The backend's rescaling of tiny inputs and its
-// zero/infinity fix-ups are replaced by sending inputs outside
-// [2^-767, 2^1000] to the library sqrt.
-__device__ __forceinline__ double sqrt_cr(double x) {
-  if (!(x >= 0x1p-767 && x <= 0x1p+1000)) return __builtin_sqrt(x);
+// Correctly rounded FP64 square root for x in [2^-767, 2^1000): reciprocal-
+// square-root estimate, one Newton step on (g ~ sqrt(x), h ~ 1/(2 sqrt(x))),
+// then two residual corrections g += (x - g*g) * h (Markstein's scheme).
+// Outside that range (sqrt_range) its value means nothing.
+__device__ __forceinline__ double sqrt_core(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y;
   double h = 0.5 * y;
@@ -456,6 +471,28 @@ __device__ __forceinline__ double sqrt_cr(double x) {
   g = __builtin_fma(d, h, g);
   d = __builtin_fma(-g, g, x);
   return __builtin_fma(d, h, g);
+}
+
+// 2^-767 <= x < 2^1000, from the high word: one unsigned compare (negative
+// values, zeros, NaN and infinities lie outside).
+__device__ __forceinline__ bool sqrt_range(double x) {
+  const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
+  return hi - 0x10000000u < 0x6E700000u;
+}
+
+// The square root of any x: the library's outside sqrt_core's range.
+__device__ __forceinline__ double sqrt_cr(double x) {
+  if (!sqrt_range(x)) return __builtin_sqrt(x);
+  return sqrt_core(x);
+}
+
+// x / a correctly rounded, from y = 1/a to within half an ulp (rcp_fast, or
+// RN(1/a) itself): quotient estimate and one residual correction (Markstein).
+// For a and x such that neither 1/a, the quotient nor the residual leaves the
+// normal range.
+__device__ __forceinline__ double div_core(double x, double a, double y) {
+  const double q = x * y;
+  return __builtin_fma(__builtin_fma(-a, q, x), y, q);
 }
 
 // Faithful (within about one ulp) square root for x >= 0 where only a
@@ -482,14 +519,25 @@ __device__ __forceinline__ double rcp_fast(double x) {
   return __builtin_fma(r, e, r);
 }
 
+// pdk's radicand (DecayMother.h / Decays.inl:245-248), in its order.
+__device__ __forceinline__ double pdk_radicand(double a, double b, double c) {
+#pragma clang fp contract(off)
+  return (a - b - c) * (a + b + c) * (a - b + c) * (a + b - c);
+}
+
 __device__ __forceinline__ double pdk(double a, double b, double c) {
 #pragma clang fp contract(off)
-  return sqrt_cr((a - b - c) * (a + b + c) * (a - b + c) * (a + b - c)) / (2 * a);
+  return sqrt_cr(pdk_radicand(a, b, c)) / (2 * a);
+}
+
+__device__ __forceinline__ double mass2_of(double e, double x, double y, double z) {
+#pragma clang fp contract(off)
+  return e * e - x * x - y * y - z * z;
 }
 
 __device__ __forceinline__ double mass_of(double e, double x, double y, double z) {
 #pragma clang fp contract(off)
-  const double m2 = e * e - x * x - y * y - z * z;
+  const double m2 = mass2_of(e, x, y, z);
   return (m2 > 0.0) ? sqrt_cr(m2) : 0.0;
 }
 
@@ -532,7 +580,7 @@ __device__ __forceinline__ void boost_folded(double (&v)[4], const DecayK& d) {
 // R + p_i of one iteration and R += p_i round identically, so the mass of the
 // running sum is computed once and reused as R.mass() of the next iteration.
 template <int N>
-__device__ __forceinline__ double event_weight_f64(const double (&p)[N][4], const double* m,
+__device__ __forceinline__ double event_weight_any(const double (&p)[N][4], const double* m,
                                                    double maxw) {
 #pragma clang fp contract(off)
   double R0 = p[0][0], R1 = p[0][1], R2 = p[0][2], R3 = p[0][3];
@@ -548,6 +596,39 @@ __device__ __forceinline__ double event_weight_f64(const double (&p)[N][4], cons
     w *= pdk(mS, m[i], mR);
     mR = mS;
   }
+  return w;
+}
+
+// The same bits, its common case without a branch per square root: every
+// radicand is taken to lie in sqrt_core's range (masses then lie in
+// [2^-384, 2^500], where div_core is exact too) and the events of which one
+// did not are formed again with event_weight_any.  2 a is written into the
+// division: RN(s / (2 a)) with 1 / (2 a).
+template <int N>
+__device__ __forceinline__ double event_weight_f64(const double (&p)[N][4], const double* m,
+                                                   double maxw) {
+#pragma clang fp contract(off)
+  double R0 = p[0][0], R1 = p[0][1], R2 = p[0][2], R3 = p[0][3];
+  double w = maxw;
+  const double m2 = mass2_of(R0, R1, R2, R3);
+  bool ok = sqrt_range(m2);
+  double mR = sqrt_core(m2);
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
+    R0 += p[i][0];
+    R1 += p[i][1];
+    R2 += p[i][2];
+    R3 += p[i][3];
+    const double s2 = mass2_of(R0, R1, R2, R3);
+    ok = ok & sqrt_range(s2);
+    const double mS = sqrt_core(s2);
+    const double x = pdk_radicand(mS, m[i], mR);
+    ok = ok & sqrt_range(x);
+    const double a2 = 2 * mS;
+    w *= div_core(sqrt_core(x), a2, rcp_fast(a2));
+    mR = mS;
+  }
+  if (__builtin_expect(!ok, 0)) w = event_weight_any<N>(p, m, maxw);
   return w;
 }
 

@@ -55,6 +55,19 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
   for (int i = 0; i < HPSP_MAX_N; ++i) k.m[i] = (i < d->n) ? d->masses[i] : 0.0;
   k.ecm = d->ecm;
   k.maxw = d->max_weight;
+  double sum = 0.0;
+  bool plain = true;
+  for (int i = 0; i < d->n; ++i) {
+    sum += d->masses[i];
+    k.msum[i] = sum;
+    k.msq[i] = d->masses[i] * d->masses[i];
+    plain = plain && d->masses[i] > 0.0;
+  }
+  k.mas0 = 0.0 * d->ecm + k.msum[0];
+  k.masN = 1.0 * d->ecm + sum;
+  k.rmasN = 1.0 / k.masN;
+  k.plain_m = plain && k.msum[0] >= 0x1p-300 && sum <= 0x1p+299;
+  k.plain = k.plain_m && d->ecm >= 0.0 && d->ecm <= 0x1p+299;
   engine_keys(d->engine, seed, k.key);
   // Vector4R::applyBoostTo(bx,by,bz) constants (Vector4R.inl:318-337).
   const double bx = d->beta[0], by = d->beta[1], bz = d->beta[2];

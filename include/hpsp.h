@@ -64,7 +64,7 @@ typedef enum {
 } hpsp_engine;
 
 typedef enum {
-  HPSP_FP64 = 0,  /* the reference's arithmetic, op for op */
+  HPSP_FP64 = 0,  /* the reference's arithmetic: weights bit for bit, momenta to rounding */
   HPSP_MIXED = 1  /* FP32 kinematics; FP64 pdk, weight product and sums */
 } hpsp_prec;
 
