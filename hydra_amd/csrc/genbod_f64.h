@@ -26,6 +26,7 @@
 
 #include <type_traits>
 
+#include "event_words.h"
 #include "hpsp_launch.h"
 
 namespace hpsp {
@@ -168,49 +169,6 @@ __device__ __forceinline__ void st(T* ptr, T v) {
   *glob(ptr) = v;
 }
 
-// Stream words of this lane's event: squares engines share the wave's 64+W
-// consecutive counters across lanes; Random123 engines evaluate per lane.
-template <int N, int ENGINE>
-struct EventWords {
-  static constexpr int W = 3 * N - 4;
-  std::conditional_t<is_squares<ENGINE>(), WaveWords, char> ww;
-  uint64_t y_hi;  // squares: key * counter of this lane's second word
-  uint64_t w[is_squares<ENGINE>() ? 1 : W];
-
-  __device__ __forceinline__ void init(const DecayK& d, uint64_t wave_first_evt, int lane) {
-    if constexpr (is_squares<ENGINE>()) {
-      // key * counter of this lane's two words, 64 counters apart: the
-      // second product is the first plus key * 64
-      const uint64_t c0 = wave_first_evt + 3 * (uint64_t)N;
-      ww.lane = lane;
-      const uint64_t y_lo = d.key[0] * (c0 + (uint64_t)lane);
-      y_hi = y_lo + (d.key[0] << 6);
-      ww.lo = squares_word_y<ENGINE>(d.key[0], y_lo);
-      ww.hi = squares_word_y<ENGINE>(d.key[0], y_hi);
-    } else {
-      r123_words<ENGINE, W>(d.key, wave_first_evt + (uint64_t)lane + 3 * (uint64_t)N, w);
-    }
-  }
-  // The next group: wave_first_evt is its first event, 64 after this
-  // group's.  With the squares engines its first 64 words are this group's
-  // second ones, so each lane evaluates one new word instead of two.
-  __device__ __forceinline__ void advance(const DecayK& d, uint64_t wave_first_evt, int lane) {
-    if constexpr (is_squares<ENGINE>()) {
-      ww.lo = ww.hi;
-      y_hi += d.key[0] << 6;  // counter + 64
-      ww.hi = squares_word_y<ENGINE>(d.key[0], y_hi);
-    } else {
-      init(d, wave_first_evt, lane);
-    }
-  }
-  __device__ __forceinline__ uint64_t operator()(int j) const {
-    if constexpr (is_squares<ENGINE>())
-      return ww.get(j);
-    else
-      return w[j];
-  }
-};
-
 // AverageOn's value of a described functor: divisions through reciprocals
 // (the result is compared within a tolerance, not bit for bit).  A user's
 // callable brings its own overload (found by argument-dependent lookup).
@@ -228,6 +186,7 @@ template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorK>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_average_f64(const AvgArgsT<FK> a) {
   __shared__ Stats sh[kBlock / kWave];
+  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
@@ -240,10 +199,7 @@ void k_average_f64(const AvgArgsT<FK> a) {
           c * kAvgChunk + ((uint64_t)wave * kGroupsPerWave + (uint64_t)it) * kWave;
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
-      if (it == 0)
-        words.init(a.d, a.first + k0, lane);
-      else
-        words.advance(a.d, a.first + k0, lane);
+      words.next(win[wave], a.d, a.first + k0, lane, it == 0);
       double p[N + (MOTHERS ? 1 : 0)][4];
       double f, wt;
       if constexpr (MOTHERS) {
@@ -314,6 +270,7 @@ struct LaneWords {
 template <int N, int ENGINE, bool MOTHERS, typename FS = DescSet>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_evaluate_f64(const EvalArgsT<FS> a) {
+  __shared__ typename EventWords<N, ENGINE>::Window win[MOTHERS ? 1 : kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
@@ -373,10 +330,7 @@ void k_evaluate_f64(const EvalArgsT<FS> a) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) p[0][c] = m4[c];
       } else {
-        if (g == g_first)
-          ewords.init(a.d, a.first + k0, lane);
-        else
-          ewords.advance(a.d, a.first + k0, lane);
+        ewords.next(win[wave], a.d, a.first + k0, lane, g == g_first);
         wt = genbod_f64<N, ENGINE>(a.d, ewords, p);
         if (a.d.do_boost) {
 #pragma unroll

@@ -12,15 +12,16 @@
 namespace hpsp {
 
 // Each wave takes runs of a.run consecutive groups of 64 events (grid-stride
-// over runs): with the squares engines a group's second 64 words are the next
-// group's first, so within a run each lane evaluates one word per group
-// instead of two.  COLS = false is the weights pass of a deferred Generate
+// over runs): a group's second 64 words (or Random123 blocks) are the next
+// group's first, so within a run each lane evaluates one per group instead of
+// two.  COLS = false is the weights pass of a deferred Generate
 // (no momentum columns): without the column stores' addresses and store
 // paths in its loop, the scalar registers it spills are reloaded outside the
 // loop only.
 template <int N, int ENGINE, bool MOTHERS, bool COLS = true>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_generate_f64(const GenArgs a) {
+  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
   const int lane = __lane_id();
   // wave index as a scalar so that column bases stay in SGPRs and every
   // store is (scalar base) + lane * 8
@@ -39,10 +40,7 @@ void k_generate_f64(const GenArgs a) {
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
 
-      if (g == g_first)
-        words.init(a.d, a.first + k0, lane);
-      else
-        words.advance(a.d, a.first + k0, lane);
+      words.next(win[wave], a.d, a.first + k0, lane, g == g_first);
       double p[N][4];
       const double wt = genbod_f64<N, ENGINE>(a.d, words, p);
 
@@ -96,9 +94,9 @@ void k_generate_f64(const GenArgs a) {
 // never read back: 32N bytes written per event (+16 with the weight column)
 // instead of 64N moved.
 //
-// One group of 64 events per wave (with the squares engines the block's
-// 256 + W - 1 engine words are evaluated once each and shared through LDS, so
-// an event costs one word, as in k_generate_f64's runs).  The block's 256
+// One group of 64 events per wave (the block's engine words are evaluated once
+// each and shared through LDS, so an event costs one word or Random123 block,
+// as in k_generate_f64's runs).  The block's 256
 // events fall into two contiguous runs of the output, its accepted events and
 // its rejected ones; for N <= 6 they are staged in LDS in partition order and
 // every column is written by all 256 threads as those two runs, so that only
@@ -108,14 +106,6 @@ void k_generate_f64(const GenArgs a) {
 // neighbouring blocks, which write neighbouring pieces of both runs, meet in
 // one L2.  A block's offset comes from the tile offset and a 16-lane scan of
 // the popcounts of its tile's flag words (block_part).
-// Squares words of one event from the block's words in LDS: thread t's own
-// word (counter c0 + t) and words j >= 1 at w[j], w = sw + t.
-struct BlockWords {
-  const uint32_t* w;
-  uint32_t own;
-  __device__ __forceinline__ uint64_t operator()(int j) const { return j == 0 ? own : w[j]; }
-};
-
 template <int N, int ENGINE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_uw_regen(const UnweightArgs a) {
@@ -125,9 +115,7 @@ void k_uw_regen(const UnweightArgs a) {
   // LDS (12 KB at N = 3) does not cap the waves in flight below the registers
   constexpr int CS = !kStage ? 1 : (C <= 8 ? C : C / 2);
   __shared__ double sh[CS][kStage ? kBlock : 1];
-  // squares engines: the block's engine words (see BlockWords)
-  constexpr int W = 3 * N - 4;
-  __shared__ uint32_t sw[is_squares<ENGINE>() ? kBlock + W - 1 : 1];
+  __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
   constexpr int kWavesPerBlock = kBlock / kWave;
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
   const uint64_t nblocks = (ngroups + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -146,29 +134,13 @@ void k_uw_regen(const UnweightArgs a) {
   const uint64_t k0 = g * kWave;
   const uint64_t k = k0 + (uint64_t)lane;
   const bool live_wave = g < ngroups;  // wave-uniform
-  uint32_t own = 0;
-  if constexpr (is_squares<ENGINE>()) {
-    // event kb + t reads the words at counters c0 + t + j, j < W: thread t
-    // evaluates the one at c0 + t, threads t < W - 1 also the one at c0 + 256 + t
-    const uint64_t c0 = a.gen_first + kb + 3 * (uint64_t)N;
-    const uint32_t t = threadIdx.x;
-    own = squares_word_y<ENGINE>(a.d.key[0], a.d.key[0] * (c0 + t));
-    sw[t] = own;
-    if (t < (uint32_t)(W - 1))
-      sw[kBlock + t] = squares_word_y<ENGINE>(a.d.key[0], a.d.key[0] * (c0 + kBlock + t));
-    __syncthreads();
-  }
+  BlockEventWords<N, ENGINE> words;
+  words.fill(sw, a.d, a.gen_first + kb);
   double p[N][4];
   uint32_t r = 0;  // the event's rank in the block's partition order
   if (live_wave) {
     const uint64_t fw = bp.fw;
-    if constexpr (is_squares<ENGINE>()) {
-      genbod_f64<N, ENGINE>(a.d, BlockWords{sw + threadIdx.x, own}, p);
-    } else {
-      EventWords<N, ENGINE> words;
-      words.init(a.d, a.gen_first + k0, lane);
-      genbod_f64<N, ENGINE>(a.d, words, p);
-    }
+    genbod_f64<N, ENGINE>(a.d, words, p);
     if (a.d.do_boost) {
 #pragma unroll
       for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);

@@ -11,6 +11,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "event_words.h"
 #include "genbod_mixed.h"
 #include "hpsp_launch.h"
 #include "uw_dst.h"
@@ -126,45 +127,6 @@ __device__ __forceinline__ void boost_general_f32(float (&v)[4], float bx, float
   }
 }
 
-template <int N, int ENGINE>
-struct EventWordsM {
-  static constexpr int W = 3 * N - 4;
-  std::conditional_t<is_squares<ENGINE>(), WaveWords, char> ww;
-  uint64_t y_hi;  // squares: key * counter of this lane's second word
-  uint64_t w[is_squares<ENGINE>() ? 1 : W];
-  __device__ __forceinline__ void init(const DecayK& d, uint64_t wave_first_evt, int lane) {
-    if constexpr (is_squares<ENGINE>()) {
-      // key * counter of this lane's two words, 64 counters apart: the
-      // second product is the first plus key * 64
-      const uint64_t c0 = wave_first_evt + 3 * (uint64_t)N;
-      ww.lane = lane;
-      const uint64_t y_lo = d.key[0] * (c0 + (uint64_t)lane);
-      y_hi = y_lo + (d.key[0] << 6);
-      ww.lo = squares_word_y<ENGINE>(d.key[0], y_lo);
-      ww.hi = squares_word_y<ENGINE>(d.key[0], y_hi);
-    } else {
-      r123_words<ENGINE, W>(d.key, wave_first_evt + (uint64_t)lane + 3 * (uint64_t)N, w);
-    }
-  }
-  // The next group (first event wave_first_evt): with the squares engines its
-  // first 64 words are this group's second ones.
-  __device__ __forceinline__ void advance(const DecayK& d, uint64_t wave_first_evt, int lane) {
-    if constexpr (is_squares<ENGINE>()) {
-      ww.lo = ww.hi;
-      y_hi += d.key[0] << 6;  // counter + 64
-      ww.hi = squares_word_y<ENGINE>(d.key[0], y_hi);
-    } else {
-      init(d, wave_first_evt, lane);
-    }
-  }
-  __device__ __forceinline__ uint64_t operator()(int j) const {
-    if constexpr (is_squares<ENGINE>())
-      return ww.get(j);
-    else
-      return w[j];
-  }
-};
-
 template <int N>
 __device__ __forceinline__ void final_boost_f32(float (&p)[N][4], const DecayK& d) {
   if (d.do_boost) {
@@ -174,9 +136,10 @@ __device__ __forceinline__ void final_boost_f32(float (&p)[N][4], const DecayK& 
 }
 
 // Runs of a.run consecutive groups of 64 events per wave, as in
-// k_generate_f64 (one squares word per lane and group within a run).
+// k_generate_f64 (one engine word or block per lane and group within a run).
 template <int N, int ENGINE, bool MOTHERS>
 __global__ __launch_bounds__(kBlock) void k_generate_mixed(const GenArgs a) {
+  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
@@ -187,15 +150,12 @@ __global__ __launch_bounds__(kBlock) void k_generate_mixed(const GenArgs a) {
        run += nwaves) {
     const uint64_t g_first = run * run_len;
     const uint64_t g_end = (g_first + run_len < ngroups) ? g_first + run_len : ngroups;
-    EventWordsM<N, ENGINE> words;
+    EventWords<N, ENGINE> words;
     for (uint64_t g = g_first; g < g_end; ++g) {
       const uint64_t k0 = g * kWave;
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
-      if (g == g_first)
-        words.init(a.d, a.first + k0, lane);
-      else
-        words.advance(a.d, a.first + k0, lane);
+      words.next(win[wave], a.d, a.first + k0, lane, g == g_first);
       float p[N][4];
       const double wt = genbod_mixed<N, ENGINE>(a.d, words, p);
       if constexpr (MOTHERS) {
@@ -267,6 +227,7 @@ struct ShiftedSums {
 template <int N, int ENGINE, bool MOTHERS>
 __global__ __launch_bounds__(kBlock) void k_average_mixed(const AvgArgs a) {
   __shared__ Stats sh[kBlock / kWave];
+  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
@@ -275,16 +236,13 @@ __global__ __launch_bounds__(kBlock) void k_average_mixed(const AvgArgs a) {
     // wave w folds groups 16w .. 16w+15 of the chunk in order (as the FP64
     // kernel), carrying the squares words from group to group
     constexpr int kGroupsPerWave = kAvgChunk / kBlock;
-    EventWordsM<N, ENGINE> words;
+    EventWords<N, ENGINE> words;
     for (int it = 0; it < kGroupsPerWave; ++it) {
       const uint64_t k0 =
           c * kAvgChunk + ((uint64_t)wave * kGroupsPerWave + (uint64_t)it) * kWave;
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
-      if (it == 0)
-        words.init(a.d, a.first + k0, lane);
-      else
-        words.advance(a.d, a.first + k0, lane);
+      words.next(win[wave], a.d, a.first + k0, lane, it == 0);
       float p[N + (MOTHERS ? 1 : 0)][4];
       double wt;
       if constexpr (MOTHERS) {
@@ -329,14 +287,6 @@ __global__ __launch_bounds__(kBlock) void k_average_mixed(const AvgArgs a) {
 // with the same code and so the same bits, at its place in the stable
 // partition.
 
-// Squares words of one event from the block's words in LDS (as k_uw_regen):
-// thread t's own word (counter c0 + t) and words j >= 1 at w[j], w = sw + t.
-struct BlockWordsM {
-  const uint32_t* w;
-  uint32_t own;
-  __device__ __forceinline__ uint64_t operator()(int j) const { return j == 0 ? own : w[j]; }
-};
-
 // The regenerating scatter of k_uw_regen with the mixed GENBOD: one group of
 // 64 events per wave, the block's 256 events staged in LDS in partition
 // order (all 4N FP32 columns at once: 12 KB at N = 3) and each column written
@@ -349,8 +299,7 @@ void k_uw_regen_mixed(const UnweightArgs a) {
   constexpr int C = 4 * N;
   constexpr int CS = C <= 24 ? C : C / 2;  // columns staged at once
   __shared__ float sh[CS][kBlock];
-  constexpr int W = 3 * N - 4;
-  __shared__ uint32_t sw[is_squares<ENGINE>() ? kBlock + W - 1 : 1];
+  __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
   constexpr int kWavesPerBlock = kBlock / kWave;
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
   const uint64_t nblocks = (ngroups + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -369,28 +318,14 @@ void k_uw_regen_mixed(const UnweightArgs a) {
   const uint64_t k0 = g * kWave;
   const uint64_t k = k0 + (uint64_t)lane;
   const bool live_wave = g < ngroups;  // wave-uniform
-  uint32_t own = 0;
-  if constexpr (is_squares<ENGINE>()) {
-    const uint64_t c0 = a.gen_first + kb + 3 * (uint64_t)N;
-    const uint32_t t = threadIdx.x;
-    own = squares_word_y<ENGINE>(a.d.key[0], a.d.key[0] * (c0 + t));
-    sw[t] = own;
-    if (t < (uint32_t)(W - 1))
-      sw[kBlock + t] = squares_word_y<ENGINE>(a.d.key[0], a.d.key[0] * (c0 + kBlock + t));
-    __syncthreads();
-  }
+  BlockEventWords<N, ENGINE> words;
+  words.fill(sw, a.d, a.gen_first + kb);
   float p[N][4];
   double wt = 0.0;
   uint32_t r = 0;  // the event's rank in the block's partition order
   if (live_wave) {
     const uint64_t fw = bp.fw;
-    if constexpr (is_squares<ENGINE>()) {
-      wt = genbod_mixed<N, ENGINE>(a.d, BlockWordsM{sw + threadIdx.x, own}, p);
-    } else {
-      EventWordsM<N, ENGINE> words;
-      words.init(a.d, a.gen_first + k0, lane);
-      wt = genbod_mixed<N, ENGINE>(a.d, words, p);
-    }
+    wt = genbod_mixed<N, ENGINE>(a.d, words, p);
     final_boost_f32<N>(p, a.d);
     const uint64_t below = (lane == 0) ? 0ULL : (~0ULL >> (64 - lane));
     const uint32_t acc_below = acc_wave + (uint32_t)__popcll(fw & below);

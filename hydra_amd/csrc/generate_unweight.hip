@@ -44,6 +44,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "event_words.h"
 #include "genbod_f64.h"
 #include "genbod_mixed.h"
 #include "uw_dst.h"
@@ -291,8 +292,9 @@ __device__ __forceinline__ double chain3_q2(const DecayK& d, const WordFn& word,
 
 }  // namespace
 
-// One 1024-event tile per block, items as k_uw_flags: thread item j is event
-// tile * 1024 + j * 256 + wave * 64 + lane of the container (generation
+// One 1024-event tile per block, four consecutive groups of 64 events per
+// wave (so that they share engine words): thread item j is event
+// tile * 1024 + (wave * 4 + j) * 64 + lane of the container (generation
 // index a.gen_first + that); flags as 64-bit ballots, counts per tile.  The
 // events the chain leaves in doubt get the chain's flag for now, and each
 // group with any is appended to the list dl as (group, mask of those events),
@@ -305,6 +307,10 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
 #pragma clang fp contract(off)
   __shared__ uint32_t cnt[kBlock / kWave];
   __shared__ uint64_t dm[kUwTile / kWave];  // doubt mask of each group of the tile
+  // the squares engines' bound needs the mass words alone, the Random123 ones'
+  // also the polar angles
+  using Words = EventWords<N, ENGINE, is_squares<ENGINE>() ? N - 2 : 3 * N - 4>;
+  __shared__ typename Words::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
@@ -312,19 +318,20 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
   if (tile >= ntiles) return;  // whole block
   // 3 bodies: the table, bins of (X, Y) pairs
   [[maybe_unused]] const double2* XY3 = reinterpret_cast<const double2*>(tab3);
-  const uint64_t off = (uint64_t)wave * kWave + (uint64_t)lane;
+  const uint64_t off = (uint64_t)wave * (kItems * kWave) + (uint64_t)lane;
   // key * (jump + k) of item 0 for the accept word and key * (gen_first + k +
   // 3N) for the generation word; item j + 1 is kBlock events on
   uint64_t ykey = a.uw_key * (a.jump + tile * kUwTile + off);
-  const uint64_t ystep = a.uw_key * (uint64_t)kBlock;
+  const uint64_t ystep = a.uw_key * (uint64_t)kWave;
   uint64_t ygen = a.d.key[0] * (a.gen_first + tile * kUwTile + off + 3 * (uint64_t)N);
-  const uint64_t gstep = a.d.key[0] * (uint64_t)kBlock;
+  const uint64_t gstep = a.d.key[0] * (uint64_t)kWave;
   uint32_t c = 0;
   // unrolled where the body is small enough for it
   constexpr int kUnroll = N <= 6 || is_squares<ENGINE>() ? kItems : 1;
+  [[maybe_unused]] Words words;
 #pragma unroll kUnroll
   for (int j = 0; j < kItems; ++j, ykey += ystep, ygen += gstep) {
-    const uint64_t g = tile * (kUwTile / kWave) + (uint64_t)j * (kBlock / kWave) + wave;
+    const uint64_t g = tile * (kUwTile / kWave) + (uint64_t)wave * kItems + j;
     const uint64_t k0 = g * kWave;
     const uint64_t k = k0 + (uint64_t)lane;
     double B, q2;
@@ -335,13 +342,11 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
       q2 = chain3_q2<ENGINE>(a.d, w, ck, XY3, B);
       sure = B < 0x1p-10;  // false for NaN
     } else if constexpr (N == 3) {
-      EventWords<N, ENGINE> words;
-      words.init(a.d, a.gen_first + k0, lane);
+      words.next(win[wave], a.d, a.gen_first + k0, lane, j == 0);
       q2 = chain3_q2<ENGINE>(a.d, words, ck, XY3, B);
       sure = B < 0x1p-10;
     } else {
-      EventWords<N, ENGINE> words;
-      words.init(a.d, a.gen_first + k0, lane);
+      words.next(win[wave], a.d, a.gen_first + k0, lane, j == 0);
       q2 = chain_q2<N, ENGINE>(a.d, words, ck.C, ck.ks_fixed, ck.ks_unit, ck.ic2_0, B, sure);
     }
     const bool live = k < a.n;
@@ -354,7 +359,7 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
     const uint64_t doubt = __ballot(live && !sure);
     if (lane == 0) {
       *(glob(a.flags) + g) = ball;
-      dm[j * (kBlock / kWave) + wave] = doubt;
+      dm[wave * kItems + j] = doubt;
     }
     c += (uint32_t)__popcll(ball);
   }
@@ -446,22 +451,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_fo
 void k_uw_flags_mixed(const UnweightArgs a, const ChainK ck, const double* tab3) {
 #pragma clang fp contract(off)
   __shared__ uint32_t cnt[kBlock / kWave];
+  using Words = EventWords<N, ENGINE, N - 2>;
+  __shared__ typename Words::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
   const uint64_t tile = xcd_tile(ntiles);
   if (tile >= ntiles) return;  // whole block
   [[maybe_unused]] const double2* XY3 = reinterpret_cast<const double2*>(tab3);
-  const uint64_t off = (uint64_t)wave * kWave + (uint64_t)lane;
+  const uint64_t off = (uint64_t)wave * (kItems * kWave) + (uint64_t)lane;
   uint64_t ykey = a.uw_key * (a.jump + tile * kUwTile + off);
-  const uint64_t ystep = a.uw_key * (uint64_t)kBlock;
+  const uint64_t ystep = a.uw_key * (uint64_t)kWave;
   uint64_t ygen = a.d.key[0] * (a.gen_first + tile * kUwTile + off + 3 * (uint64_t)N);
-  const uint64_t gstep = a.d.key[0] * (uint64_t)kBlock;
+  const uint64_t gstep = a.d.key[0] * (uint64_t)kWave;
   uint32_t c = 0;
   constexpr int kUnroll = N <= 6 || is_squares<ENGINE>() ? kItems : 1;
+  [[maybe_unused]] Words words;
 #pragma unroll kUnroll
   for (int j = 0; j < kItems; ++j, ykey += ystep, ygen += gstep) {
-    const uint64_t g = tile * (kUwTile / kWave) + (uint64_t)j * (kBlock / kWave) + wave;
+    const uint64_t g = tile * (kUwTile / kWave) + (uint64_t)wave * kItems + j;
     const uint64_t k0 = g * kWave;
     const uint64_t k = k0 + (uint64_t)lane;
     // the event's mass words, from the wave's shared words where they are
@@ -470,8 +478,7 @@ void k_uw_flags_mixed(const UnweightArgs a, const ChainK ck, const double* tab3)
     if constexpr (N == 3 && is_squares<ENGINE>()) {
       mw.w[0] = squares_word_y<ENGINE>(a.d.key[0], ygen);  // counter gen_first + k + 3N
     } else if constexpr (N > 2) {
-      EventWords<N, ENGINE> words;
-      words.init(a.d, a.gen_first + k0, lane);
+      words.next(win[wave], a.d, a.gen_first + k0, lane, j == 0);
 #pragma unroll
       for (int i = 0; i < N - 2; ++i) mw.w[i] = words(i);
     }

@@ -343,6 +343,7 @@ __host__ __device__ __forceinline__ uint32_t minstd_seed(uint32_t s) {
 }
 
 constexpr int kMinstd = HPSP_MINSTD_RAND;
+constexpr double kMinstdInv = 1.0 / 2147483646.0;
 
 // Engines whose words fit 32 bits.
 template <int ENGINE>
@@ -356,9 +357,14 @@ constexpr bool narrow_words() {
 template <int ENGINE>
 __device__ __forceinline__ double to_unit(uint64_t w) {
 #pragma clang fp contract(off)
-  if constexpr (ENGINE == kMinstd)
-    return (double)((uint32_t)w - 1u) / 2147483646.0;
-  else if constexpr (is_squares<ENGINE>())
+  if constexpr (ENGINE == kMinstd) {
+    // the quotient from RN(1 / 2147483646) and one residual correction: equal
+    // to the rounded division for every state (checked for all 2^31)
+    const double x = (double)((uint32_t)w - 1u);
+    const double q = x * kMinstdInv;
+    return __builtin_fma(__builtin_fma(-2147483646.0, q, x), kMinstdInv, q);
+  }
+  if constexpr (is_squares<ENGINE>())
     return (double)(uint32_t)w * 0x1p-32;
   else
     return (double)w * 0x1p-64;
@@ -375,36 +381,32 @@ __device__ __forceinline__ double to_cos(uint64_t w) {
     return 2 * to_unit<ENGINE>(w) - 1;
 }
 
-// In-register ascending sort of a small fixed-size array (odd-even
-// transposition network; any correct sort yields the same values).
+// In-register ascending sort of a small fixed-size array (any correct sort
+// yields the same values): Batcher's merge exchange (Knuth, The Art of
+// Computer Programming 3, 5.2.2, algorithm M), which takes 19 exchanges for 8
+// values where an odd-even transposition takes 28.
 template <typename T, int K>
 __device__ __forceinline__ void sort_net(T (&v)[K]) {
+  constexpr int t = K > 8 ? 4 : (K > 4 ? 3 : (K > 2 ? 2 : 1));  // 2^t >= K
+  static_assert(K <= 16, "2^t >= K");
 #pragma unroll
-  for (int r = 0; r < K; ++r) {
+  for (int pp = t - 1; pp >= 0; --pp) {
+    const int p = 1 << pp;
 #pragma unroll
-    for (int i = (r & 1); i + 1 < K; i += 2) {
-      T a = v[i], b = v[i + 1];
-      v[i] = a < b ? a : b;
-      v[i + 1] = a < b ? b : a;
+    for (int qq = t - 1; qq >= pp; --qq) {
+      const int r = qq == t - 1 ? 0 : p;
+      const int d = qq == t - 1 ? p : (2 << qq) - p;
+#pragma unroll
+      for (int i = 0; i + d < K; ++i) {
+        if ((i & p) == r) {
+          const T a = v[i], b = v[i + d];
+          v[i] = a < b ? a : b;
+          v[i + d] = a < b ? b : a;
+        }
+      }
     }
   }
 }
-
-// Wave-level sharing of squares words.  Lane L's event e0+L needs the words
-// at counters c0 + L + k, k = 0..W-1 (W <= 64).  Each lane evaluates the two
-// words at c0 + L ("lo") and c0 + 64 + L ("hi").  For word k, lane L reads
-// source lane s = (L+k) mod 64; if L+k < 64 it needs lo[s] and then s >= k,
-// otherwise hi[s] and then s < k.  So each source lane offers
-// (s >= k ? lo : hi) and one ds_bpermute per word suffices.
-struct WaveWords {
-  uint32_t lo, hi;
-  int lane;
-  __device__ __forceinline__ uint32_t get(int k) const {
-    if (k == 0) return lo;
-    const uint32_t src = (lane >= k) ? lo : hi;
-    return (uint32_t)__builtin_amdgcn_ds_bpermute(((lane + k) & (kWave - 1)) << 2, (int)src);
-  }
-};
 
 // ---------------------------------------------------------------------------
 // sin and cos of 2*pi*u for u in [0, 1].  u = (j + d) / 256 with j = floor(256 u)

@@ -139,7 +139,8 @@ struct HistArgs {
 struct RangeArgs {
   DecayK d;            // key words unused
   uint32_t x_start;
-  uint32_t a_stride;   // 48271^(grid * kBlock): the state advance of one grid pass
+  uint32_t run;        // consecutive groups of 64 elements per wave (set by the launcher)
+  uint32_t a_stride;   // 48271^(elements from a wave's run to its next; set by the launcher)
   uint64_t n;
   double* cols;        // generate: 4N momentum columns of ld doubles
   uint64_t ld;

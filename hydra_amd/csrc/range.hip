@@ -5,12 +5,12 @@
 // -ffp-contract=off.
 //
 // Engine words.  minstd_rand's word j of element first + k is
-// x_start * a^(k + j) mod m (a = 48271, m = 2^31 - 1).  A wave's 64 elements
-// need the words at offsets k0 + 0 .. k0 + 63 + 3N - 5: each lane holds the
-// two words at k0 + lane and k0 + 64 + lane and the wave shares them with
-// ds_bpermute (WaveWords), as the squares engines' counters are shared.  A
-// lane's first pair costs one power of a (uniform across the wave) and a
-// table lookup; each further grid pass multiplies both by a^(grid size).
+// x_start * a^(k + j) mod m (a = 48271, m = 2^31 - 1).  A wave takes runs of
+// consecutive groups of 64 elements, whose words it shares through LDS
+// (WindowView): a lane evaluates the word 64 after its last one, one product
+// with a^64, for each further group.  A run's first words cost one power of
+// a, formed on the scalar unit, and a table lookup; a wave's next run one
+// product with a^(the events between).
 //
 // Kernels:
 //   k_range_generate<N>  elements into SoA momentum columns and a weight column
@@ -21,6 +21,7 @@
 #include <array>
 #include <utility>
 
+#include "event_words.h"
 #include "genbod_f64.h"
 #include "hist_key.h"
 
@@ -41,28 +42,42 @@ constexpr MinstdPowers minstd_powers() {
 }
 __constant__ MinstdPowers kPow = minstd_powers();
 
-// This lane's two stream words and the wave view genbod_f64 reads.
+constexpr uint32_t kMinstdA64 = minstd_powers().v[kWave];  // a^64 mod m
+
+// The words of a wave's groups of elements.
+template <int N>
 struct RangeWords {
-  uint32_t lo, hi;
-  int lane;
-  // words at offsets k0 + lane and k0 + 64 + lane
-  __device__ __forceinline__ void init(uint32_t x_start, uint64_t k0, int l) {
-    lane = l;
+  static constexpr int W = 3 * N - 4;
+  using View = WindowView<uint32_t, 1, W>;
+  using Window = typename View::Win;
+  View v;
+  uint32_t x0;  // the lane's word at the run's first group
+  uint32_t x;   // its last word
+
+  // the first run, whose first element is k0
+  __device__ __forceinline__ void first(uint32_t x_start, uint64_t k0, int lane) {
     const uint32_t xw = minstd_mul(x_start, minstd_pow(k0));
-    lo = minstd_mul(xw, kPow.v[l]);
-    hi = minstd_mul(xw, kPow.v[kWave + l]);
+    x0 = minstd_mul(xw, kPow.v[lane]);
   }
-  __device__ __forceinline__ void step(uint32_t a) {
-    lo = minstd_mul(lo, a);
-    hi = minstd_mul(hi, a);
+  // the run's first group, or the group after the last
+  __device__ __forceinline__ void next(Window& win, int lane, bool restart) {
+    if (restart) {
+      x = minstd_mul(x0, kMinstdA64);
+      const uint32_t lo[1] = {x0}, hi[1] = {x};
+      v.start(win, lane, 0, lo, hi);
+    } else {
+      x = minstd_mul(x, kMinstdA64);
+      const uint32_t hi[1] = {x};
+      v.shift(hi);
+    }
   }
-  __device__ __forceinline__ uint64_t operator()(int j) const {
-    return WaveWords{lo, hi, lane}.get(j);
-  }
+  // the wave's next run
+  __device__ __forceinline__ void skip(uint32_t a_stride) { x0 = minstd_mul(x0, a_stride); }
+  __device__ __forceinline__ uint64_t operator()(int j) const { return v.get(j); }
 };
 
 template <int N>
-__device__ __forceinline__ double range_event(const DecayK& d, const RangeWords& w,
+__device__ __forceinline__ double range_event(const DecayK& d, const RangeWords<N>& w,
                                               double (&p)[N][4]) {
   const double wt = genbod_f64<N, kMinstd>(d, w, p);
   if (d.do_boost) {
@@ -75,27 +90,34 @@ __device__ __forceinline__ double range_event(const DecayK& d, const RangeWords&
 template <int N>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_range_generate(const RangeArgs a) {
+  __shared__ typename RangeWords<N>::Window win[kBlock / kWave];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  uint64_t base = (uint64_t)blockIdx.x * kBlock;
-  if (base >= a.n) return;
-  RangeWords words;
-  words.init(a.x_start, base + (uint64_t)wave * kWave, lane);
-  for (; base < a.n; base += stride) {
-    const uint64_t k0 = base + (uint64_t)wave * kWave;
-    double p[N][4];
-    const double wt = range_event<N>(a.d, words, p);
-    if (k0 + (uint64_t)lane < a.n) {
-      double* c = a.cols + k0;
+  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
+  const uint64_t nruns = (ngroups + a.run - 1) / a.run;
+  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
+  uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  RangeWords<N> words;
+  words.first(a.x_start, run * a.run * kWave, lane);
+  for (; run < nruns; run += nwaves) {
+    const uint64_t g_first = run * a.run;
+    const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
+    for (uint64_t g = g_first; g < g_end; ++g) {
+      const uint64_t k0 = g * kWave;
+      words.next(win[wave], lane, g == g_first);
+      double p[N][4];
+      const double wt = range_event<N>(a.d, words, p);
+      if (k0 + (uint64_t)lane < a.n) {
+        double* c = a.cols + k0;
 #pragma unroll
-      for (int i = 0; i < N; ++i)
+        for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, p[i][q]);
-      if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
+          for (int q = 0; q < 4; ++q)
+            st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, p[i][q]);
+        if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
+      }
     }
-    words.step(a.a_stride);
+    words.skip(a.a_stride);
   }
 }
 
@@ -103,6 +125,7 @@ template <int N>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_range_hist(const RangeArgs a) {
   extern __shared__ double bins[];
+  __shared__ typename RangeWords<N>::Window win[kBlock / kWave];
   const uint64_t nslots = a.h.nbins + 2;
   if (a.use_lds) {
     for (uint64_t b = threadIdx.x; b < nslots; b += kBlock) bins[b] = 0.0;
@@ -110,30 +133,37 @@ void k_range_hist(const RangeArgs a) {
   }
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  uint64_t base = (uint64_t)blockIdx.x * kBlock;
-  RangeWords words;
-  words.init(a.x_start, base + (uint64_t)wave * kWave, lane);
-  for (; base < a.n; base += stride) {
-    const uint64_t k = base + (uint64_t)wave * kWave + (uint64_t)lane;
-    double p[N][4];
-    const double wt = range_event<N>(a.d, words, p);
-    words.step(a.a_stride);
-    if (k >= a.n) continue;
-    double x[HPSP_HIST_MAX_DIM];
+  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
+  const uint64_t nruns = (ngroups + a.run - 1) / a.run;
+  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
+  uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  RangeWords<N> words;
+  words.first(a.x_start, run * a.run * kWave, lane);
+  for (; run < nruns; run += nwaves) {
+    const uint64_t g_first = run * a.run;
+    const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
+    for (uint64_t g = g_first; g < g_end; ++g) {
+      const uint64_t k = g * kWave + (uint64_t)lane;
+      words.next(win[wave], lane, g == g_first);
+      double p[N][4];
+      const double wt = range_event<N>(a.d, words, p);
+      if (k >= a.n) continue;
+      double x[HPSP_HIST_MAX_DIM];
 #pragma unroll
-    for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
-      x[d] = (d < a.h.ndim) ? functor_eval<double>(a.axes[d], p) : 0.0;
-    const double w = a.weight_mode == HPSP_HIST_WEIGHT_GENERATION ? wt
-                     : a.weight_mode == HPSP_HIST_WEIGHT_PHSP
-                         ? event_weight_f64<N>(p, a.d.m, a.d.maxw)
-                         : 1.0;
-    const uint64_t key = hist_key(a.h, x);
-    if (key == kDrop) continue;
-    if (a.use_lds)
-      atomicAdd(&bins[key], w);
-    else
-      unsafeAtomicAdd(&a.contents[key], w);
+      for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
+        x[d] = (d < a.h.ndim) ? functor_eval<double>(a.axes[d], p) : 0.0;
+      const double w = a.weight_mode == HPSP_HIST_WEIGHT_GENERATION ? wt
+                       : a.weight_mode == HPSP_HIST_WEIGHT_PHSP
+                           ? event_weight_f64<N>(p, a.d.m, a.d.maxw)
+                           : 1.0;
+      const uint64_t key = hist_key(a.h, x);
+      if (key == kDrop) continue;
+      if (a.use_lds)
+        atomicAdd(&bins[key], w);
+      else
+        unsafeAtomicAdd(&a.contents[key], w);
+    }
+    words.skip(a.a_stride);
   }
   if (a.use_lds) {
     __syncthreads();
@@ -146,13 +176,15 @@ void k_range_hist(const RangeArgs a) {
 
 // ---------------------------------------------------------------------------
 
-// A lane's first word pair costs a power of a by square-and-multiply over the
-// bits of its offset (some 30 steps); later grid passes step by one multiply.
-// The grid is capped so that each lane runs many passes.
+// Runs of the generation kernel as k_generate_f64's, dispatched in order
+// (bound by its stores up to 3 daughters); the events from a wave's run to its
+// next one are a power of a formed here.
 template <int N>
 static void gen_one(RangeArgs a, hipStream_t s) {
-  const unsigned g = grid_for(a.n, 8192u);
-  a.a_stride = minstd_pow((uint64_t)g * kBlock);
+  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
+  a.run = run_groups(ngroups, N <= 3 ? kRunMaxStores : kRunMax);
+  const unsigned g = grid_for_runs((ngroups + a.run - 1) / a.run);
+  a.a_stride = minstd_pow((uint64_t)g * (kBlock / kWave) * a.run * kWave);
   hipLaunchKernelGGL(k_range_generate<N>, dim3(g), dim3(kBlock), 0, s, a);
 }
 
@@ -165,7 +197,12 @@ static void hist_one(RangeArgs a, hipStream_t s) {
   // merge costs nslots atomics
   const unsigned cap = (a.use_lds && lds > 32768) ? 512u : 2048u;
   const unsigned g = grid_for(a.n, cap);
-  a.a_stride = minstd_pow((uint64_t)g * kBlock);
+  // one run per wave: nothing is stored on the way
+  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
+  const uint64_t nwaves = (uint64_t)g * (kBlock / kWave);
+  const uint64_t per = (ngroups + nwaves - 1) / nwaves;
+  a.run = (uint32_t)(per < 1 ? 1 : (per < (1u << 20) ? per : (1u << 20)));
+  a.a_stride = minstd_pow(nwaves * a.run * kWave);
   hipLaunchKernelGGL(k_range_hist<N>, dim3(g), dim3(kBlock), lds, s, a);
 }
 
