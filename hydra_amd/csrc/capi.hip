@@ -861,14 +861,16 @@ static int average_common(const hpsp_decay* d, const hpsp_functor* f, uint64_t s
   a.n = n;
   a.mothers = mothers;
   a.mld = mld;
-  a.partials = static_cast<Stats*>(ws);
   hipStream_t s = as_stream(stream);
   const uint64_t m = (n + kAvgChunk - 1) / kAvgChunk;
+  // one chunk's partial is the result
+  a.partials = m == 1 ? reinterpret_cast<Stats*>(out_dev) : static_cast<Stats*>(ws);
   if (n > 0) {
     const int e = (prec == HPSP_FP64) ? launch_average_f64(d->n, d->engine, a, s)
                                       : launch_average_mixed(d->n, d->engine, a, s);
     if (e) return HPSP_ERR_HIP;
   }
+  if (m == 1) return HPSP_OK;
   return hip_status(launch_stats_finalize(a.partials, m, reinterpret_cast<Stats*>(out_dev), s));
 }
 

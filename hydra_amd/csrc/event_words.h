@@ -10,10 +10,10 @@
 // block once and puts it into LDS; the event in lane l reads word j at slot
 // l + j / A, an immediate offset from one address.  The kernels that read them
 // are bound by their vector instructions: evaluating every block in every lane
-// (Random123) took Generate of 3e6 4-body Threefry events 118 us against 102
-// us, 5e5 12-body ones 52 us against 42; one ds_bpermute, a select and its
-// address per word (squares engines) took the 10-body Generate of 2^24 events
-// 1.57 ms against 1.51 ms, the mixed one 685 us against 659 us.
+// (Random123) took Generate of 3e6 4-body Threefry events 118 us against 102,
+// Evaluate of 6e5 8-body Threefry4x64 ones 52 against 42; one ds_bpermute, a
+// select and its address per word (squares engines) took the 10-body Generate
+// of 2^24 events 1.57 ms against 1.51, the mixed one 685 us against 659.
 //
 // The counter of a Random123 block is two 64-bit words: e + 3N wraps in 64
 // bits, the steps from there carry into the second.  In the one group of

@@ -178,27 +178,44 @@ __device__ __forceinline__ double avg_value(const FunctorK& f, const double (&p)
 }
 
 // AverageOn: chunks of kAvgChunk consecutive events, one partial per chunk.
-// Within a chunk wave w folds its own run of consecutive groups of 64 events
-// (groups 16w .. 16w+15), lane l event l of each, in order, so the squares
-// words carry from group to group; the four wave results merge in a fixed
-// tree, so a partial depends only on its event range.
-template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorK>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+// Within a chunk accumulating wave w folds its own run of consecutive groups
+// of 64 events (groups 16w .. 16w+15), lane l event l of each, in order; the
+// four wave results merge in a fixed tree, so a partial depends only on its
+// event range.
+//
+// WAVES = 4: each wave generates the groups it folds, the engine words
+// carrying from group to group.  With fewer chunks than the chip holds blocks,
+// the 16 groups in series set the time (a 5-body chunk in mixed precision: 33
+// us), so for those WAVES = 16 or 8 waves generate the chunk's groups, stage
+// every event's functor value and weight in LDS, and four of them fold the
+// staged values in the same order: the same partial, bit for bit.
+constexpr int avg_wide_waves(int N) { return N <= 6 ? 16 : 8; }  // 128 or 256 registers
+
+template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorK, int WAVES = kBlock / kWave>
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_average_f64(const AvgArgsT<FK> a) {
-  __shared__ Stats sh[kBlock / kWave];
-  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
+  constexpr int kFold = kBlock / kWave;  // waves that fold
+  constexpr bool kWide = WAVES > kFold;
+  constexpr int kGroups = kAvgChunk / kWave;
+  __shared__ Stats sh[kFold];
+  __shared__ double staged[2][kWide ? kAvgChunk : 1];  // functor values, weights
+  __shared__ typename EventWords<N, ENGINE>::Window win[WAVES];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
   for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
     Stats acc = {0.0, 0.0, 0.0};
-    constexpr int kGroupsPerWave = kAvgChunk / kBlock;
+    // a chunk with few events spreads them over all its waves
+    const uint64_t left = (a.n - c * kAvgChunk + kWave - 1) / kWave;
+    const int groups = kWide && left < kGroups ? (int)left : kGroups;
+    const int per_wave = (groups + WAVES - 1) / WAVES;
     EventWords<N, ENGINE> words;
-    for (int it = 0; it < kGroupsPerWave; ++it) {
-      const uint64_t k0 =
-          c * kAvgChunk + ((uint64_t)wave * kGroupsPerWave + (uint64_t)it) * kWave;
+    for (int it = 0; it < per_wave; ++it) {
+      const int g = wave * per_wave + it;
+      const uint64_t k0 = c * kAvgChunk + (uint64_t)g * kWave;
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
+      if (kWide && g >= groups) break;  // wave-uniform
       words.next(win[wave], a.d, a.first + k0, lane, it == 0);
       double p[N + (MOTHERS ? 1 : 0)][4];
       double f, wt;
@@ -226,13 +243,28 @@ void k_average_f64(const AvgArgsT<FK> a) {
         }
       }
       f = avg_value(a.f, p);
-      if (live) stats_push(acc, f, wt);
+      if constexpr (kWide) {
+        staged[0][g * kWave + lane] = f;
+        staged[1][g * kWave + lane] = wt;
+      } else {
+        if (live) stats_push(acc, f, wt);
+      }
     }
-    acc = wave_reduce_stats(acc);
-    if (lane == 0) sh[wave] = acc;
+    if constexpr (kWide) __syncthreads();
+    if (!kWide || wave < kFold) {
+      if constexpr (kWide) {
+        for (int it = 0; it < kGroups / kFold; ++it) {
+          const int t = (wave * (kGroups / kFold) + it) * kWave + lane;
+          if (c * kAvgChunk + (uint64_t)t < a.n) stats_push(acc, staged[0][t], staged[1][t]);
+        }
+      }
+      acc = wave_reduce_stats(acc);
+      if (lane == 0) sh[wave] = acc;
+    }
     __syncthreads();
     if (threadIdx.x == 0)
-      a.partials[c] = stats_merge(stats_merge(sh[0], sh[1]), stats_merge(sh[2], sh[3]));
+      a.partials[c] =
+          stats_or_zero(stats_merge(stats_merge(sh[0], sh[1]), stats_merge(sh[2], sh[3])));
     __syncthreads();
   }
 }

@@ -189,19 +189,31 @@ void k_uw_regen(const UnweightArgs a) {
 }
 
 // Merge m partials in a fixed order: thread t folds a contiguous slice, then
-// a pairwise tree over the 256 slice results.
-__global__ __launch_bounds__(kBlock) void k_stats_finalize(const Stats* part, uint64_t m,
-                                                           Stats* out) {
-  __shared__ Stats sh[kBlock];
-  const uint64_t per = (m + kBlock - 1) / kBlock;
+// a pairwise tree over the slice results, the lanes of a wave first.  One block
+// bound by its chain of dependent merges (0.25 us each): 1024 threads fold
+// 4096 partials (2^24 events) in 4 + 10 steps, 256 took 16 + 8.
+constexpr int kMergeThreads = 1024;
+__global__ __launch_bounds__(kMergeThreads) void k_stats_finalize(const Stats* part, uint64_t m,
+                                                                  Stats* out) {
+  __shared__ Stats sh[kMergeThreads / kWave];
+  const uint64_t per = (m + kMergeThreads - 1) / kMergeThreads;
   const uint64_t b = (uint64_t)threadIdx.x * per;
   const uint64_t e = (b + per < m) ? b + per : m;
   Stats acc = {0.0, 0.0, 0.0};
-  for (uint64_t i = b; i < e; ++i) acc = stats_merge(acc, part[i]);
-  sh[threadIdx.x] = acc;
+  Stats next = acc;
+  if (b < e) next = part[b];
+  for (uint64_t i = b; i < e; ++i) {
+    const Stats cur = next;
+    if (i + 1 < e) next = part[i + 1];
+    acc = stats_merge(acc, cur);
+  }
+  acc = wave_reduce_stats(acc);
+  if (__lane_id() == 0) sh[threadIdx.x / kWave] = acc;
   __syncthreads();
-  for (int off = 1; off < kBlock; off <<= 1) {
-    if ((threadIdx.x & (2 * off - 1)) == 0) sh[threadIdx.x] = stats_merge(sh[threadIdx.x], sh[threadIdx.x + off]);
+  constexpr int W = kMergeThreads / kWave;
+  for (int off = 1; off < W; off <<= 1) {
+    if (threadIdx.x < W && (threadIdx.x & (2 * off - 1)) == 0)
+      sh[threadIdx.x] = stats_merge(sh[threadIdx.x], sh[threadIdx.x + off]);
     __syncthreads();
   }
   if (threadIdx.x == 0) *out = sh[0];
@@ -292,12 +304,23 @@ static void gen_one(const GenArgs& in, hipStream_t s) {
 
 template <int N, int E>
 static void avg_one(const AvgArgs& a, hipStream_t s) {
-  const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
-  const unsigned g = (unsigned)(nchunks < 8192 ? (nchunks ? nchunks : 1) : 8192);
-  if (a.mothers)
-    hipLaunchKernelGGL((k_average_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_average_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+  constexpr int kWaves = avg_wide_waves(N);
+  launch_avg(
+      a.n, kWaves,
+      [&](unsigned g) {
+        if (a.mothers)
+          hipLaunchKernelGGL((k_average_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
+        else
+          hipLaunchKernelGGL((k_average_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+      },
+      [&](unsigned g, unsigned threads) {
+        if (a.mothers)
+          hipLaunchKernelGGL((k_average_f64<N, E, true, FunctorK, kWaves>), dim3(g), dim3(threads),
+                             0, s, a);
+        else
+          hipLaunchKernelGGL((k_average_f64<N, E, false, FunctorK, kWaves>), dim3(g),
+                             dim3(threads), 0, s, a);
+      });
 }
 
 template <int N, int E>
@@ -348,7 +371,7 @@ int launch_average_f64(int N, int engine, const AvgArgs& a, hipStream_t s) {
 }
 
 int launch_stats_finalize(const Stats* partials, uint64_t m, Stats* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_stats_finalize, dim3(1), dim3(kBlock), 0, s, partials, m, out);
+  hipLaunchKernelGGL(k_stats_finalize, dim3(1), dim3(kMergeThreads), 0, s, partials, m, out);
   return (int)hipGetLastError();
 }
 

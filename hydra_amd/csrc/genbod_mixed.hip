@@ -224,24 +224,33 @@ struct ShiftedSums {
   }
 };
 
-template <int N, int ENGINE, bool MOTHERS>
-__global__ __launch_bounds__(kBlock) void k_average_mixed(const AvgArgs a) {
-  __shared__ Stats sh[kBlock / kWave];
-  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
+// The chunks, groups and wide form of k_average_f64.
+constexpr int kAvgWideWaves = 16;
+
+template <int N, int ENGINE, bool MOTHERS, int WAVES = kBlock / kWave>
+__global__ __launch_bounds__(WAVES * kWave) void k_average_mixed(const AvgArgs a) {
+  constexpr int kFold = kBlock / kWave;  // waves that fold
+  constexpr bool kWide = WAVES > kFold;
+  constexpr int kGroups = kAvgChunk / kWave;
+  __shared__ Stats sh[kFold];
+  __shared__ double staged[2][kWide ? kAvgChunk : 1];  // functor values, weights
+  __shared__ typename EventWords<N, ENGINE>::Window win[WAVES];
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
   for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
     ShiftedSums acc;
-    // wave w folds groups 16w .. 16w+15 of the chunk in order (as the FP64
-    // kernel), carrying the squares words from group to group
-    constexpr int kGroupsPerWave = kAvgChunk / kBlock;
+    // a chunk with few events spreads them over all its waves
+    const uint64_t left = (a.n - c * kAvgChunk + kWave - 1) / kWave;
+    const int groups = kWide && left < kGroups ? (int)left : kGroups;
+    const int per_wave = (groups + WAVES - 1) / WAVES;
     EventWords<N, ENGINE> words;
-    for (int it = 0; it < kGroupsPerWave; ++it) {
-      const uint64_t k0 =
-          c * kAvgChunk + ((uint64_t)wave * kGroupsPerWave + (uint64_t)it) * kWave;
+    for (int it = 0; it < per_wave; ++it) {
+      const int g = wave * per_wave + it;
+      const uint64_t k0 = c * kAvgChunk + (uint64_t)g * kWave;
       const uint64_t k = k0 + (uint64_t)lane;
       const bool live = k < a.n;
+      if (kWide && g >= groups) break;  // wave-uniform
       words.next(win[wave], a.d, a.first + k0, lane, it == 0);
       float p[N + (MOTHERS ? 1 : 0)][4];
       double wt;
@@ -267,13 +276,28 @@ __global__ __launch_bounds__(kBlock) void k_average_mixed(const AvgArgs a) {
         final_boost_f32<N>(p, a.d);
       }
       const double f = functor_eval<float, false>(a.f, p);
-      if (live) acc.push(f, wt);
+      if constexpr (kWide) {
+        staged[0][g * kWave + lane] = f;
+        staged[1][g * kWave + lane] = wt;
+      } else {
+        if (live) acc.push(f, wt);
+      }
     }
-    const Stats st = wave_reduce_stats(acc.stats());
-    if (lane == 0) sh[wave] = st;
+    if constexpr (kWide) __syncthreads();
+    if (!kWide || wave < kFold) {
+      if constexpr (kWide) {
+        for (int it = 0; it < kGroups / kFold; ++it) {
+          const int t = (wave * (kGroups / kFold) + it) * kWave + lane;
+          if (c * kAvgChunk + (uint64_t)t < a.n) acc.push(staged[0][t], staged[1][t]);
+        }
+      }
+      const Stats st = wave_reduce_stats(acc.stats());
+      if (lane == 0) sh[wave] = st;
+    }
     __syncthreads();
     if (threadIdx.x == 0)
-      a.partials[c] = stats_merge(stats_merge(sh[0], sh[1]), stats_merge(sh[2], sh[3]));
+      a.partials[c] =
+          stats_or_zero(stats_merge(stats_merge(sh[0], sh[1]), stats_merge(sh[2], sh[3])));
     __syncthreads();
   }
 }
@@ -388,12 +412,22 @@ static void gen_one(const GenArgs& in, hipStream_t s) {
 
 template <int N, int E>
 static void avg_one(const AvgArgs& a, hipStream_t s) {
-  const uint64_t nchunks = (a.n + kAvgChunk - 1) / kAvgChunk;
-  const unsigned g = (unsigned)(nchunks < 8192 ? (nchunks ? nchunks : 1) : 8192);
-  if (a.mothers)
-    hipLaunchKernelGGL((k_average_mixed<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_average_mixed<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+  launch_avg(
+      a.n, kAvgWideWaves,
+      [&](unsigned g) {
+        if (a.mothers)
+          hipLaunchKernelGGL((k_average_mixed<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
+        else
+          hipLaunchKernelGGL((k_average_mixed<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+      },
+      [&](unsigned g, unsigned threads) {
+        if (a.mothers)
+          hipLaunchKernelGGL((k_average_mixed<N, E, true, kAvgWideWaves>), dim3(g), dim3(threads),
+                             0, s, a);
+        else
+          hipLaunchKernelGGL((k_average_mixed<N, E, false, kAvgWideWaves>), dim3(g), dim3(threads),
+                             0, s, a);
+      });
 }
 
 template <int I>

@@ -933,6 +933,11 @@ __device__ __forceinline__ Stats stats_merge(const Stats& x, const Stats& y) {
   return r;
 }
 
+// A partial without weight says nothing (every merge passes it over): zeros.
+__device__ __forceinline__ Stats stats_or_zero(const Stats& x) {
+  return x.w == 0.0 ? Stats{0.0, 0.0, 0.0} : x;
+}
+
 // Fold one event {f, wt, 0} into a running accumulator (weighted West
 // update; equal to AddStatsPHSP with a single-point right side).
 __device__ __forceinline__ void stats_push(Stats& s, double f, double wt) {
