@@ -641,6 +641,7 @@ int hpsp_unweight_regenerate(const hpsp_decay* d, uint64_t gen_seed, uint64_t fi
   a.n_acc = n_acc_dev;
   a.regen = 1;
   a.gen_first = first;
+  a.scan_here = use_scan_here(a) ? kScanTiles : 0;
   rc = hip_status(launch_unweight(d->n, a, s));  // flags and offsets
   if (rc) return rc;
   if (!cols_out && !idx_out && !w_out) return HPSP_OK;
@@ -659,6 +660,13 @@ size_t hpsp_generate_unweight_workspace_size(uint64_t n) {
   if (too_many(n)) return SIZE_MAX;
   return gu_table_offset(n) + align_up(2 * kBin3 * sizeof(double));
 }
+
+// Events up to which hpsp_generate_unweight forms every event's momenta for its
+// flag: it costs less than the chain's three further launches (11 us) up to
+// about 7e5 events for 3 bodies (524288: 22.1 us against 26.7; 1e6: 38.5 against
+// 33.3), 5e5 for 5 (524288: 36.3 against 35.9) and 4e5 for 12 (262144: 54
+// against 59; 524288: 98 against 86).
+constexpr uint64_t kExactEvents = 3 << 17;
 
 // The chain flags kernels' constants, formed once here instead of by every
 // wave (FP64 divisions); scale2 bounds E^2 + p^2 of any subsystem; K of the
@@ -723,6 +731,7 @@ int hpsp_generate_unweight(const hpsp_decay* d, uint64_t gen_seed, uint64_t firs
   a.regen = 1;
   a.gen_first = first;
   if (n == 0) return hip_status(launch_unweight(d->n, a, s));  // the count: 0
+  a.scan_here = use_scan_here(a) ? kScanTiles : 0;
   // E^2 + |p|^2 of any subsystem is at most (M gamma (1 + beta))^2, M = the
   // decay's fECM + sum of masses; the momenta's error constant 2K + 4
   double M = d->ecm;
@@ -734,8 +743,13 @@ int hpsp_generate_unweight(const hpsp_decay* d, uint64_t gen_seed, uint64_t firs
     const double f = a.d.gamma * (1.0 + b);
     scale2 *= f * f;
   }
-  const ChainK ck = make_chaink(d, scale2);
-  rc = hip_status(launch_flags_chain(d->n, d->engine, a, dl_count, dl, tab3, ck, s));
+  if (a.scan_here && n <= kExactEvents) {
+    a.scan_here = kScanBlocks;
+    rc = hip_status(launch_flags_exact(d->n, d->engine, a, s));
+  } else {
+    rc = hip_status(launch_flags_chain(d->n, d->engine, a, dl_count, dl, tab3,
+                                       make_chaink(d, scale2), s));
+  }
   if (rc) return rc;
   rc = hip_status(launch_uw_scans(a, s));
   if (rc) return rc;
@@ -779,8 +793,14 @@ int hpsp_generate_unweight_mixed(const hpsp_decay* d, uint64_t gen_seed, uint64_
   a.regen = 1;
   a.gen_first = first;
   if (n == 0) return hip_status(launch_unweight(d->n, a, s));  // the count: 0
+  a.scan_here = use_scan_here(a) ? kScanTiles : 0;
   // no momenta are involved in the mixed flags' bound: no scale
-  rc = hip_status(launch_flags_mixed(d->n, d->engine, a, tab3, make_chaink(d, 0.0), s));
+  if (a.scan_here) {
+    a.scan_here = kScanBlocks;
+    rc = hip_status(launch_flags_direct(d->n, d->engine, a, s));
+  } else {
+    rc = hip_status(launch_flags_mixed(d->n, d->engine, a, tab3, make_chaink(d, 0.0), s));
+  }
   if (rc) return rc;
   rc = hip_status(launch_uw_scans(a, s));
   if (rc) return rc;

@@ -106,7 +106,7 @@ void k_generate_f64(const GenArgs a) {
 // neighbouring blocks, which write neighbouring pieces of both runs, meet in
 // one L2.  A block's offset comes from the tile offset and a 16-lane scan of
 // the popcounts of its tile's flag words (block_part).
-template <int N, int ENGINE>
+template <int N, int ENGINE, bool HERE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_uw_regen(const UnweightArgs a) {
   constexpr int C = 4 * N;
@@ -125,10 +125,12 @@ void k_uw_regen(const UnweightArgs a) {
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t g0 = blk * kWavesPerBlock;  // the block's first group
-  const BlockPart bp = block_part(a, g0, wave, ngroups);
+  __shared__ TileSums sums;
+  const TilePlace at = tile_place<HERE>(a, g0 / (kUwTile / kWave), sums);
+  const BlockPart bp = block_part(a, g0, wave, ngroups, at.off);
   const uint64_t goff = bp.goff;  // accepted events before the block
   const uint32_t acc_wave = bp.acc_wave, a_blk = bp.a_blk;
-  const uint64_t nacc = *a.n_acc;
+  const uint64_t nacc = at.nacc;
   const uint64_t kb = g0 * kWave;  // the block's first event
   const uint64_t g = g0 + (uint64_t)wave;
   const uint64_t k0 = g * kWave;
@@ -186,6 +188,42 @@ void k_uw_regen(const UnweightArgs a) {
       }
     }
   }
+}
+
+// The flags of a Generate's events, few enough that launches and the chains of
+// dependent operations, not throughput, set the time: each event's momenta and
+// PhaseSpaceWeight formed and the reference's test applied (FlagDaugthers,
+// Decays.inl:75-89), one group of 64 per wave.  In place of the weight chain's
+// four launches (its list's counter, table, flags, doubtful events): the 3-body
+// call of 1e5 events 25 us -> 12, the 10-body one of 4e4 42 -> 25.
+template <int N, int ENGINE>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+void k_uw_flags_exact(const UnweightArgs a) {
+#pragma clang fp contract(off)
+  __shared__ uint32_t cnt[kBlock / kWave];
+  __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
+  const int lane = __lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t g = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  const uint64_t k = g * kWave + (uint64_t)lane;
+  const double rmax = 1.0 / a.maxv;
+  const bool rmax_ok = __builtin_fabs(rmax) >= 0x1p-1000 && __builtin_fabs(rmax) <= 0x1p+1000;
+  BlockEventWords<N, ENGINE> words;
+  words.fill(sw, a.d, a.gen_first + (uint64_t)blockIdx.x * kBlock);
+  uint64_t ball = 0;
+  if (g * kWave < a.n) {  // wave-uniform
+    double p[N][4];
+    genbod_f64<N, ENGINE>(a.d, words, p);
+    if (a.d.do_boost) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);
+    }
+    const double u = (double)squares3(a.uw_key, a.jump + k) * 0x1p-32;
+    ball = __ballot(k < a.n && ratio_above(event_weight_f64<N>(p, a.d.m, a.d.maxw), a.maxv, rmax,
+                                           rmax_ok, u));
+    if (lane == 0) *(glob(a.flags) + g) = ball;
+  }
+  put_block_count(a, (uint32_t)__popcll(ball), cnt);
 }
 
 // Merge m partials in a fixed order: thread t folds a contiguous slice, then
@@ -327,9 +365,20 @@ template <int N, int E>
 static void regen_one(const UnweightArgs& a, hipStream_t s) {
   const uint64_t nblocks = (a.n + kBlock - 1) / kBlock;
   const uint64_t grid = (nblocks + kXcds - 1) / kXcds * kXcds;
-  hipLaunchKernelGGL((k_uw_regen<N, E>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+  if (a.scan_here)
+    hipLaunchKernelGGL((k_uw_regen<N, E, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_uw_regen<N, E, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
 }
 
+template <int N, int E>
+static void exact_one(const UnweightArgs& a, hipStream_t s) {
+  const unsigned ntiles = (unsigned)((a.n + kUwTile - 1) / kUwTile);
+  hipLaunchKernelGGL((k_uw_flags_exact<N, E>), dim3(ntiles * kItems), dim3(kBlock), 0, s, a);
+}
+
+template <int I>
+static constexpr auto exact_at = &exact_one<2 + I / kNumE, I % kNumE>;
 template <int I>
 static constexpr auto gen_at = &gen_one<2 + I / kNumE, I % kNumE>;
 template <int I>
@@ -346,17 +395,27 @@ static constexpr auto regen_table(std::integer_sequence<int, I...>) {
   return std::array<void (*)(const UnweightArgs&, hipStream_t), sizeof...(I)>{regen_at<I>...};
 }
 template <int... I>
+static constexpr auto exact_table(std::integer_sequence<int, I...>) {
+  return std::array<void (*)(const UnweightArgs&, hipStream_t), sizeof...(I)>{exact_at<I>...};
+}
+template <int... I>
 static constexpr auto avg_table(std::integer_sequence<int, I...>) {
   return std::array<void (*)(const AvgArgs&, hipStream_t), sizeof...(I)>{avg_at<I>...};
 }
 
 static const auto kGen = gen_table(std::make_integer_sequence<int, kNumN * kNumE>{});
 static const auto kAvg = avg_table(std::make_integer_sequence<int, kNumN * kNumE>{});
+static const auto kExact = exact_table(std::make_integer_sequence<int, kNumN * kNumE>{});
 static const auto kRegen = regen_table(std::make_integer_sequence<int, kNumN * kNumE>{});
 
 int launch_unweight_regen(int N, int engine, const UnweightArgs& a, hipStream_t s) {
   if (a.n == 0) return (int)hipSuccess;
   kRegen[(N - 2) * kNumE + engine](a, s);
+  return (int)hipGetLastError();
+}
+
+int launch_flags_exact(int N, int engine, const UnweightArgs& a, hipStream_t s) {
+  kExact[(N - 2) * kNumE + engine](a, s);
   return (int)hipGetLastError();
 }
 

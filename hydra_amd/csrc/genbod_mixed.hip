@@ -311,13 +311,42 @@ __global__ __launch_bounds__(WAVES * kWave) void k_average_mixed(const AvgArgs a
 // with the same code and so the same bits, at its place in the stable
 // partition.
 
+// The flags for few events (as k_uw_flags_exact): every event's FP64 weight
+// chain, one group of 64 events per wave, without the table that
+// k_uw_flags_mixed's bound takes a launch for.
+template <int N, int ENGINE>
+__global__ __launch_bounds__(kBlock) void k_uw_flags_direct(const UnweightArgs a) {
+#pragma clang fp contract(off)
+  __shared__ uint32_t cnt[kBlock / kWave];
+  using Words = EventWords<N, ENGINE, N - 2>;
+  __shared__ typename Words::Window win[kBlock / kWave];
+  const int lane = __lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t g = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  const uint64_t k = g * kWave + (uint64_t)lane;
+  uint64_t ball = 0;
+  if (g * kWave < a.n) {  // wave-uniform
+    const double rmax = 1.0 / a.maxv;
+    const bool rmax_ok = __builtin_fabs(rmax) >= 0x1p-1000 && __builtin_fabs(rmax) <= 0x1p+1000;
+    Words words;
+    words.next(win[wave], a.d, a.gen_first + g * kWave, lane, true);
+    double invMas[N];
+    float pd[N - 1];
+    const double w = weight_chain<N, ENGINE>(a.d, words, invMas, pd);
+    const double u = (double)squares3(a.uw_key, a.jump + k) * 0x1p-32;
+    ball = __ballot(k < a.n && ratio_above(w, a.maxv, rmax, rmax_ok, u));
+    if (lane == 0) *(glob(a.flags) + g) = ball;
+  }
+  put_block_count(a, (uint32_t)__popcll(ball), cnt);
+}
+
 // The regenerating scatter of k_uw_regen with the mixed GENBOD: one group of
 // 64 events per wave, the block's 256 events staged in LDS in partition
 // order (all 4N FP32 columns at once: 12 KB at N = 3) and each column written
 // as the block's two runs; cols_out holds FP32 columns (UnweightArgs carries
 // it as a double pointer).  w_out receives each output row's weight column
 // value, the FP64 generation weight.
-template <int N, int ENGINE>
+template <int N, int ENGINE, bool HERE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_uw_regen_mixed(const UnweightArgs a) {
   constexpr int C = 4 * N;
@@ -333,10 +362,12 @@ void k_uw_regen_mixed(const UnweightArgs a) {
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t g0 = blk * kWavesPerBlock;
-  const BlockPart bp = block_part(a, g0, wave, ngroups);
+  __shared__ TileSums sums;
+  const TilePlace at = tile_place<HERE>(a, g0 / (kUwTile / kWave), sums);
+  const BlockPart bp = block_part(a, g0, wave, ngroups, at.off);
   const uint64_t goff = bp.goff;
   const uint32_t acc_wave = bp.acc_wave, a_blk = bp.a_blk;
-  const uint64_t nacc = *a.n_acc;
+  const uint64_t nacc = at.nacc;
   const uint64_t kb = g0 * kWave;
   const uint64_t g = g0 + (uint64_t)wave;
   const uint64_t k0 = g * kWave;
@@ -390,7 +421,10 @@ template <int N, int E>
 static void regen_mixed_one(const UnweightArgs& a, hipStream_t s) {
   const uint64_t nblocks = (a.n + kBlock - 1) / kBlock;
   const uint64_t grid = (nblocks + kXcds - 1) / kXcds * kXcds;
-  hipLaunchKernelGGL((k_uw_regen_mixed<N, E>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+  if (a.scan_here)
+    hipLaunchKernelGGL((k_uw_regen_mixed<N, E, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_uw_regen_mixed<N, E, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
 }
 
 template <int N, int E>
@@ -442,6 +476,24 @@ static constexpr auto gen_table(std::integer_sequence<int, I...>) {
 template <int... I>
 static constexpr auto avg_table(std::integer_sequence<int, I...>) {
   return std::array<void (*)(const AvgArgs&, hipStream_t), sizeof...(I)>{avg_at<I>...};
+}
+
+template <int N, int E>
+static void direct_one(const UnweightArgs& a, hipStream_t s) {
+  const unsigned ntiles = (unsigned)((a.n + kUwTile - 1) / kUwTile);
+  hipLaunchKernelGGL((k_uw_flags_direct<N, E>), dim3(ntiles * kItems), dim3(kBlock), 0, s, a);
+}
+template <int I>
+static constexpr auto direct_at = &direct_one<2 + I / kNumE, I % kNumE>;
+template <int... I>
+static constexpr auto direct_table(std::integer_sequence<int, I...>) {
+  return std::array<void (*)(const UnweightArgs&, hipStream_t), sizeof...(I)>{direct_at<I>...};
+}
+static const auto kDirect = direct_table(std::make_integer_sequence<int, kNumN * kNumE>{});
+
+int launch_flags_direct(int N, int engine, const UnweightArgs& a, hipStream_t s) {
+  kDirect[(N - 2) * kNumE + engine](a, s);
+  return (int)hipGetLastError();
 }
 
 template <int I>

@@ -203,9 +203,12 @@ __device__ __forceinline__ int bin3(uint32_t v) {
   return (int)side * kBin3Side + idx;
 }
 
-__global__ __launch_bounds__(kBlock) void k_chain_table3(const DecayK d, double2* XY) {
+// count, where given, is cleared (the chain's list, filled by the next kernel).
+__global__ __launch_bounds__(kBlock) void k_chain_table3(const DecayK d, double2* XY,
+                                                         uint64_t* count) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i == 0 && count) *count = 0;
   if (i >= kBin3) return;
   const int side = i / kBin3Side, idx = i % kBin3Side;
   uint64_t tlo, thi;
@@ -526,7 +529,7 @@ static void flags_mixed_one(const UnweightArgs& a, double* tab3, const ChainK& c
   const unsigned grid = (unsigned)((ntiles + kXcds - 1) / kXcds * kXcds);
   if constexpr (N == 3)
     hipLaunchKernelGGL(k_chain_table3, dim3((kBin3 + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                       a.d, reinterpret_cast<double2*>(tab3));
+                       a.d, reinterpret_cast<double2*>(tab3), (uint64_t*)nullptr);
   hipLaunchKernelGGL((k_uw_flags_mixed<N, E>), dim3(grid), dim3(kBlock), 0, s, a, ck,
                      (const double*)tab3);
 }
@@ -556,10 +559,11 @@ static void chain_one(const UnweightArgs& a, uint64_t* dl_count, uint64_t* dl, d
                       const ChainK& ck, hipStream_t s) {
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
   const unsigned grid = (unsigned)((ntiles + kXcds - 1) / kXcds * kXcds);
-  hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, s, dl_count);
   if constexpr (N == 3)
     hipLaunchKernelGGL(k_chain_table3, dim3((kBin3 + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                       a.d, reinterpret_cast<double2*>(tab3));
+                       a.d, reinterpret_cast<double2*>(tab3), dl_count);
+  else
+    hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, s, dl_count);
   hipLaunchKernelGGL((k_uw_flags_chain<N, E>), dim3(grid), dim3(kBlock), 0, s, a, dl_count, dl,
                      ck, (const double*)tab3);
   const unsigned pgrid = (unsigned)(ntiles < kPatchBlocks ? ntiles : kPatchBlocks);

@@ -187,7 +187,21 @@ struct UnweightArgs {
   uint64_t* tidx;       // order 1: original index of the r-th kept sample
   int regen;            // events regenerated at their destinations, not moved
   uint64_t gen_first;   // regen: generation index of the container's row 0
+  int scan_here;        // the scatter sums the counts itself (use_scan_here): kScanTiles
+                        // from tile_count, kScanBlocks from a 16-bit count per 256 events
+                        // at tile_off (four in the place of one offset)
 };
+constexpr int kScanTiles = 1, kScanBlocks = 2;
+
+// Up to kScanHereTiles tiles (2^20 events) the scatter's blocks sum the counts
+// themselves, at most four per thread, instead of reading offsets that a kernel
+// of its own wrote: a launch (about 4 us) less, for two shuffle sums per block.
+// For calls with outputs; block 0 writes the accepted total.
+constexpr uint64_t kScanHereTiles = 4 * kBlock;
+inline bool use_scan_here(const UnweightArgs& a) {
+  return (a.cols_out || a.idx_out || a.w_out) && a.order == 0 &&
+         (a.n + kUwTile - 1) / kUwTile <= kScanHereTiles;
+}
 
 // Kernel launchers; each returns a hipError_t value.
 int launch_generate_f64(int N, int engine, const GenArgs& a, hipStream_t s);
@@ -203,7 +217,8 @@ int launch_range_generate(int N, const RangeArgs& a, hipStream_t s);
 int launch_range_histogram(int N, const RangeArgs& a, hipStream_t s);
 int launch_stats_finalize(const Stats* partials, uint64_t m, Stats* out, hipStream_t s);
 int launch_event_weight(int N, const WeightArgs& a, hipStream_t s);
-// Exclusive scan of the tile counts into a.tile_off, the total into *a.n_acc.
+// Exclusive scan of the tile counts into a.tile_off, the total into *a.n_acc
+// (nothing where a.scan_here is set).
 int launch_uw_scans(const UnweightArgs& a, hipStream_t s);
 // Flags of Decays::Unweight for events a.gen_first.. of a Generate with decay
 // a.d, decided from each event's generation weight where it is far enough
@@ -225,12 +240,18 @@ struct ChainK {
   double rmax;      // RN(1 / max) and whether it is normal (ratio_above)
   int rmax_ok;
 };
+// For few events with outputs (a.scan_here) instead: every event's momenta,
+// PhaseSpaceWeight and test in one kernel (genbod_f64.hip; kScanBlocks).
+int launch_flags_exact(int N, int engine, const UnweightArgs& a, hipStream_t s);
 int launch_flags_chain(int N, int engine, const UnweightArgs& a, uint64_t* dl_count, uint64_t* dl,
                        double* tab3, const ChainK& ck, hipStream_t s);
 // The mixed form: flags from each event's FP64 weight chain, the mixed
 // Generate's weight column (generate_unweight.hip; tab3 and ck as for
 // launch_flags_chain); then every event generated again at its place, FP32
 // columns in a.cols_out, carried as a double pointer (genbod_mixed.hip).
+// (for few events with outputs, a.scan_here, instead: every event's weight chain
+// and test in one kernel, launch_flags_direct; kScanBlocks)
+int launch_flags_direct(int N, int engine, const UnweightArgs& a, hipStream_t s);
 int launch_flags_mixed(int N, int engine, const UnweightArgs& a, double* tab3, const ChainK& ck,
                        hipStream_t s);
 int launch_unweight_regen_mixed(int N, int engine, const UnweightArgs& a, hipStream_t s);

@@ -7,8 +7,8 @@
 //                      default engine's word for the container index, the
 //                      test  w / max > u; a 64-bit __ballot per wave gives
 //                      the flag word, popcounts give the tile count.
-//   2. k_uw_scan    -- one block: exclusive prefix of the tile counts and
-//                      the accepted total.
+//   2. k_uw_scan    -- exclusive prefix of the tile counts and the accepted
+//                      total (for few tiles the scatter sums them itself).
 //   3. k_uw_scatter -- each event's destination from its tile offset and the
 //                      popcount of the lower lanes of its ballot word:
 //                      accepted -> off_acc, rejected -> n_acc + (k - off_acc);
@@ -92,6 +92,53 @@ __global__ __launch_bounds__(kBlock) void k_uw_flags(const UnweightArgs a) {
   if (lane == 0) cnt[wave] = c;
   __syncthreads();
   if (threadIdx.x == 0) a.tile_count[tile] = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+}
+
+// Exclusive scan of the tile counts in one kernel: each block takes a run of
+// kScanThreads tiles, sums the counts before them itself (four per load) and
+// scans its own.  At 2^27 events (128 runs) its longest block reads 0.5 MB, a
+// few us, where three kernels (below) take three launches, 14 us at 10^7 events;
+// beyond kScanOneRuns runs the reads would grow with the
+// square and the three kernels take over.
+constexpr int kScanThreads = 1024;
+constexpr uint64_t kScanOneRuns = 256;
+__global__ __launch_bounds__(kScanThreads) void k_uw_scan(const uint32_t* tile_count,
+                                                          uint64_t ntiles, uint64_t* tile_off,
+                                                          uint64_t* n_acc) {
+  constexpr int W = kScanThreads / kWave;
+  __shared__ uint64_t sh[2][W];
+  const int lane = __lane_id();
+  const int wave = threadIdx.x / kWave;
+  const uint64_t base = (uint64_t)blockIdx.x * kScanThreads;
+  uint64_t before = 0;
+  const uint4* v = reinterpret_cast<const uint4*>(tile_count);
+#pragma unroll 4
+  for (uint64_t i = threadIdx.x; i < base / 4; i += kScanThreads) {
+    const uint4 c = v[i];
+    before += (uint64_t)c.x + c.y + c.z + c.w;
+  }
+  const uint64_t t = base + threadIdx.x;
+  const uint64_t own = t < ntiles ? tile_count[t] : 0u;
+  uint64_t x = own;  // inclusive over the wave
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t o = __shfl_up(x, off, kWave);
+    if (lane >= off) x += o;
+    before += __shfl_xor(before, off, kWave);
+  }
+  if (lane == kWave - 1) {
+    sh[0][wave] = x;
+    sh[1][wave] = before;
+  }
+  __syncthreads();
+  uint64_t off = x - own, total = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    off += sh[1][w] + (w < wave ? sh[0][w] : 0);
+    total += sh[1][w] + sh[0][w];
+  }
+  if (t < ntiles) tile_off[t] = off;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *n_acc = total;
 }
 
 // Exclusive scan of the tile counts in three fully parallel steps:
@@ -180,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_uw_scan_tiles(const uint32_t* tile_c
 // threads as the block's two runs (accepted, rejected), so that only the ends
 // of a block's runs are partial cache lines.  Blocks are dealt to XCDs in
 // contiguous ranges.
-template <int N>
+template <int N, bool HERE>
 __global__ __launch_bounds__(kBlock) void k_uw_scatter_staged(const UnweightArgs a) {
   constexpr int C = 4 * N;
   // all columns staged at once: staging half of them (more waves in flight)
@@ -196,10 +243,12 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter_staged(const UnweightArgs
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t g0 = blk * kWavesPerBlock;
-  const BlockPart bp = block_part(a, g0, wave, ngroups);
+  __shared__ TileSums sums;
+  const TilePlace at = tile_place<HERE>(a, g0 / (kUwTile / kWave), sums);
+  const BlockPart bp = block_part(a, g0, wave, ngroups, at.off);
   const uint64_t goff = bp.goff;
   const uint32_t acc_wave = bp.acc_wave, a_blk = bp.a_blk;
-  const uint64_t nacc = *a.n_acc;
+  const uint64_t nacc = at.nacc;
   const uint64_t kb = g0 * kWave;
   const uint64_t g = g0 + (uint64_t)wave;
   const uint64_t k0 = g * kWave;
@@ -242,7 +291,7 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter_staged(const UnweightArgs
   }
 }
 
-template <int N>
+template <int N, bool HERE>
 __global__ __launch_bounds__(kBlock) void k_uw_scatter(const UnweightArgs a) {
   __shared__ uint64_t goff[kUwTile / kWave];
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
@@ -252,8 +301,10 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter(const UnweightArgs a) {
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = kUwTile / kWave;
-  const uint64_t tile_base = a.tile_off[tile];
-  const uint64_t nacc = *a.n_acc;
+  __shared__ TileSums sums;
+  const TilePlace at = tile_place<HERE>(a, tile, sums);
+  const uint64_t tile_base = at.off;
+  const uint64_t nacc = at.nacc;
   // group offsets inside the tile: lanes 0..15 of wave 0 each load one flag
   // word and an inclusive shuffle scan turns the popcounts into offsets
   if (wave == 0) {
@@ -360,6 +411,7 @@ __device__ __forceinline__ uint64_t swap_chain_dst(const UnweightArgs& a, uint64
 // hydra::unweight's scatter of ncols value columns (any count): the same
 // destinations as k_uw_scatter (or the sequential-partition ones), columns
 // moved in batches of eight with all four groups' loads of a batch in flight.
+template <bool HERE>
 __global__ __launch_bounds__(kBlock) void k_uw_scatter_cols(const UnweightArgs a, int ncols) {
   __shared__ uint64_t goff[kUwTile / kWave];
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
@@ -369,8 +421,10 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter_cols(const UnweightArgs a
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = kUwTile / kWave;
-  const uint64_t tile_base = a.tile_off[tile];
-  const uint64_t nacc = *a.n_acc;
+  __shared__ TileSums sums;
+  const TilePlace at = tile_place<HERE>(a, tile, sums);
+  const uint64_t tile_base = at.off;
+  const uint64_t nacc = at.nacc;
   if (wave == 0) {
     const uint64_t gi = tile * ngroups + (uint64_t)lane;
     const uint32_t own =
@@ -495,7 +549,14 @@ constexpr int kNumN = HPSP_MAX_N - 1;
 static void launch_flags(int N, const UnweightArgs& a, uint64_t ntiles, hipStream_t s);
 
 int launch_uw_scans(const UnweightArgs& a, hipStream_t s) {
+  if (a.scan_here) return (int)hipSuccess;
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
+  const uint64_t nblocks = (ntiles + kScanThreads - 1) / kScanThreads;
+  if (nblocks <= kScanOneRuns) {
+    hipLaunchKernelGGL(k_uw_scan, dim3((unsigned)nblocks), dim3(kScanThreads), 0, s, a.tile_count,
+                       ntiles, a.tile_off, a.n_acc);
+    return (int)hipGetLastError();
+  }
   const uint64_t nruns = (ntiles + kScanRun - 1) / kScanRun;
   hipLaunchKernelGGL(k_uw_scan_blocks, dim3((unsigned)nruns), dim3(kBlock), 0, s, a.tile_count,
                      ntiles, a.run_sum);
@@ -506,7 +567,9 @@ int launch_uw_scans(const UnweightArgs& a, hipStream_t s) {
 }
 
 template <int N>
-static void uw_one(const UnweightArgs& a, hipStream_t s) {
+static void uw_one(const UnweightArgs& in, hipStream_t s) {
+  UnweightArgs a = in;
+  a.scan_here = use_scan_here(a) ? kScanTiles : 0;
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
   if (a.w_in && !a.use_f)
     launch_flags(0, a, ntiles, s);
@@ -517,10 +580,18 @@ static void uw_one(const UnweightArgs& a, hipStream_t s) {
     if constexpr (N <= 6) {
       const uint64_t nblocks = (a.n + kBlock - 1) / kBlock;
       const uint64_t grid = (nblocks + kXcds - 1) / kXcds * kXcds;
-      hipLaunchKernelGGL(k_uw_scatter_staged<N>, dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+      if (a.scan_here)
+        hipLaunchKernelGGL((k_uw_scatter_staged<N, true>), dim3((unsigned)grid), dim3(kBlock), 0,
+                           s, a);
+      else
+        hipLaunchKernelGGL((k_uw_scatter_staged<N, false>), dim3((unsigned)grid), dim3(kBlock), 0,
+                           s, a);
     } else {
       const uint64_t grid = (ntiles + kXcds - 1) / kXcds * kXcds;
-      hipLaunchKernelGGL(k_uw_scatter<N>, dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+      if (a.scan_here)
+        hipLaunchKernelGGL((k_uw_scatter<N, true>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
+      else
+        hipLaunchKernelGGL((k_uw_scatter<N, false>), dim3((unsigned)grid), dim3(kBlock), 0, s, a);
     }
   }
 }
@@ -538,6 +609,7 @@ int launch_unweight_sample(int ncols, const UnweightArgs& in, double* block_max,
     return (int)hipGetLastError();
   }
   UnweightArgs a = in;
+  a.scan_here = use_scan_here(a) ? kScanTiles : 0;
   if (max_dev) {  // max_element of the weights
     hipLaunchKernelGGL(k_max_column, dim3((unsigned)nblocks), dim3(kBlock), 0, s, a.w_in, a.n,
                        block_max);
@@ -546,18 +618,17 @@ int launch_unweight_sample(int ncols, const UnweightArgs& in, double* block_max,
   }
   const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
   launch_flags(0, a, ntiles, s);
-  const uint64_t nruns = (ntiles + kScanRun - 1) / kScanRun;
-  hipLaunchKernelGGL(k_uw_scan_blocks, dim3((unsigned)nruns), dim3(kBlock), 0, s, a.tile_count,
-                     ntiles, a.run_sum);
-  hipLaunchKernelGGL(k_uw_scan_top, dim3(1), dim3(kBlock), 0, s, a.run_sum, nruns, a.n_acc);
-  hipLaunchKernelGGL(k_uw_scan_tiles, dim3((unsigned)nruns), dim3(kBlock), 0, s, a.tile_count,
-                     ntiles, a.run_sum, a.tile_off);
+  launch_uw_scans(a, s);
   if (a.cols_out || a.idx_out || a.w_out) {
     if (a.order == 1)
       hipLaunchKernelGGL(k_uw_kept_index, dim3((unsigned)ntiles), dim3(kBlock), 0, s, a);
     const uint64_t grid = (ntiles + kXcds - 1) / kXcds * kXcds;
-    hipLaunchKernelGGL(k_uw_scatter_cols, dim3((unsigned)grid), dim3(kBlock), 0, s, a,
-                       a.cols_out ? ncols : 0);
+    if (a.scan_here)
+      hipLaunchKernelGGL(k_uw_scatter_cols<true>, dim3((unsigned)grid), dim3(kBlock), 0, s, a,
+                         a.cols_out ? ncols : 0);
+    else
+      hipLaunchKernelGGL(k_uw_scatter_cols<false>, dim3((unsigned)grid), dim3(kBlock), 0, s, a,
+                         a.cols_out ? ncols : 0);
   }
   return (int)hipGetLastError();
 }

@@ -9,6 +9,53 @@ namespace hpsp {
 
 constexpr int kItems = kUwTile / kBlock;  // 4 groups of 64 events per wave
 
+// Accepted events before a tile and in all: from the scan's arrays, or summed
+// from the counts here (a.scan_here: at most four tiles per thread; a template
+// argument, because the summing code cost the large regenerating scatter 2% even
+// unused).  Every
+// thread of a block calls it, for one tile; block 0 then writes the total.
+struct TilePlace {
+  uint64_t off, nacc;
+};
+struct TileSums {  // __shared__
+  uint32_t before[kBlock / kWave], all[kBlock / kWave];
+};
+template <bool HERE>
+__device__ __forceinline__ TilePlace tile_place(const UnweightArgs& a, uint64_t tile,
+                                                TileSums& sh) {
+  if constexpr (!HERE) return {a.tile_off[tile], *a.n_acc};
+  const uint32_t t = threadIdx.x;
+  const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
+  uint32_t all = 0, before = 0;
+  for (uint32_t i = t; i < ntiles; i += kBlock) {
+    uint32_t n;
+    if (a.scan_here == kScanBlocks) {
+      const uint64_t c = a.tile_off[i];  // four 16-bit counts, 256 at most each
+      const uint32_t pairs = (uint32_t)c + (uint32_t)(c >> 32);
+      n = (pairs & 0xFFFFu) + (pairs >> 16);
+    } else {
+      n = a.tile_count[i];
+    }
+    all += n;
+    before += i < tile ? n : 0u;
+  }
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    all += __shfl_xor(all, off, kWave);
+    before += __shfl_xor(before, off, kWave);
+  }
+  if (__lane_id() == 0) {
+    sh.before[t / kWave] = before;
+    sh.all[t / kWave] = all;
+  }
+  __syncthreads();
+  static_assert(kBlock / kWave == 4, "four waves");
+  const uint64_t off = sh.before[0] + sh.before[1] + sh.before[2] + sh.before[3];
+  const uint64_t nacc = sh.all[0] + sh.all[1] + sh.all[2] + sh.all[3];
+  if (blockIdx.x == 0 && t == 0) *a.n_acc = nacc;
+  return {off, nacc};
+}
+
 // Destinations of one group of 64 samples in the stable partition: kept lanes
 // to goff + (kept lanes below), the others to nacc + (k0 - goff) + (rejected
 // lanes below).
@@ -54,7 +101,7 @@ struct BlockPart {
 };
 
 __device__ __forceinline__ BlockPart block_part(const UnweightArgs& a, uint64_t g0, int wave,
-                                                uint64_t ngroups) {
+                                                uint64_t ngroups, uint64_t tile_off) {
   constexpr int kGroupsPerTile = kUwTile / kWave;
   constexpr int kWavesPerBlock = kBlock / kWave;
   static_assert(kGroupsPerTile <= kWave && kGroupsPerTile % kWavesPerBlock == 0,
@@ -73,7 +120,7 @@ __device__ __forceinline__ BlockPart block_part(const UnweightArgs& a, uint64_t 
   const int lw = gb + wave;
   const uint32_t before = gb ? (uint32_t)__builtin_amdgcn_readlane((int)incl, gb - 1) : 0u;
   BlockPart b;
-  b.goff = a.tile_off[tile] + before;
+  b.goff = tile_off + before;
   b.acc_wave = (lw ? (uint32_t)__builtin_amdgcn_readlane((int)incl, lw - 1) : 0u) - before;
   b.a_blk = (uint32_t)__builtin_amdgcn_readlane((int)incl, gb + kWavesPerBlock - 1) - before;
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)fl, lw);
@@ -100,6 +147,17 @@ __device__ __forceinline__ bool ratio_above(double w, double maxv, double rmax, 
   bool r = gap > 0.0;
   if (!settled) r = (w / maxv) > u;
   return r;
+}
+
+// The count of a 256-event block of a flags kernel with one group of 64 events
+// per wave (kScanBlocks); every block of the tiles calls it.
+__device__ __forceinline__ void put_block_count(const UnweightArgs& a, uint32_t count,
+                                                uint32_t (&sh)[kBlock / kWave]) {
+  if (__lane_id() == 0) sh[threadIdx.x / kWave] = count;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    reinterpret_cast<uint16_t*>(a.tile_off)[blockIdx.x] =
+        (uint16_t)(sh[0] + sh[1] + sh[2] + sh[3]);
 }
 
 // Tile of a block: each XCD takes a contiguous range of tiles, so that
