@@ -279,7 +279,9 @@ __global__ __launch_bounds__(kBlock) void k_event_weight(const WeightArgs a) {
   }
 }
 
-// Block maxima of w*f (Decays.inl:488-490), then one block folds them.
+// Block maxima of w*f (Decays.inl:488-490), then one block folds them; the
+// values themselves into a.w_out where given, for the flags to read (8 bytes an
+// event instead of its momenta again).
 template <int N>
 __global__ __launch_bounds__(kBlock) void k_max_weight(const WeightArgs a, double* block_max) {
   __shared__ double sh[kBlock];
@@ -290,6 +292,7 @@ __global__ __launch_bounds__(kBlock) void k_max_weight(const WeightArgs a, doubl
     load_event<N>(a.cols, a.ld, k, p);
     double w = event_weight_f64<N>(p, a.d.m, a.d.maxw);
     if (a.use_f) w = w * functor_eval<double>(a.f, p);
+    if (a.w_out) a.w_out[k] = w;
     mx = (mx < w) ? w : mx;
   }
   sh[threadIdx.x] = mx;

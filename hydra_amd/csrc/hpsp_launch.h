@@ -159,7 +159,7 @@ struct WeightArgs {
   int use_f;
   const double* cols;
   uint64_t ld, n;
-  double* w_out;
+  double* w_out;       // values (event_weight; max_weight: null to skip)
 };
 
 struct UnweightArgs {
@@ -310,6 +310,10 @@ inline void launch_avg(uint64_t n, int waves_wide, Narrow&& narrow, Wide&& wide)
   else
     narrow((unsigned)(nchunks < 8192 ? nchunks : 8192));
 }
+
+// Blocks of the kernels that leave one maximum each to a last block: 8 waves
+// per SIMD (65536 took that block 42 us).
+constexpr unsigned kMaxBlocks = 2048;
 
 inline unsigned grid_for(uint64_t items, unsigned cap = 65536u) {
   const uint64_t b = (items + kBlock - 1) / kBlock;

@@ -8,8 +8,8 @@ import ctypes
 import numpy as np
 import pytest
 import torch
-from gpu_util import (DEV, generate, make_decay, ptr, rng_words, stream_handle, unweight,
-                      unweight_sample)
+from gpu_util import (DEV, generate, make_decay, make_functor, ptr, rng_words, stream_handle,
+                      unweight, unweight_sample)
 from hydra_amd import capi
 
 pytestmark = pytest.mark.gpu
@@ -91,3 +91,24 @@ def test_sample_counts(n):
         assert k == keep.sum()
         assert np.array_equal(out[:, :k], x[:, keep])
         assert np.array_equal(np.sort(out, axis=1), np.sort(x, axis=1))
+
+
+@pytest.mark.parametrize("N", [2, 3, 5, 9])
+def test_functor_maximum_from_values(N):
+    # Unweight(F) that finds the maximum (its values kept in the output until
+    # the scatter) against the one that is given it (values formed for the flags)
+    dec = decay(N)
+    f = make_functor(capi.F_BW_SUM, [(0.9, 0.1, 0.5, -0.1, 0, 1), (1.2, 0.2, 0.6, 1.5, 0, N - 1)])
+    lib = capi.lib()
+    for n in (1, 255, 1025, 300000, (1 << 20) + 5):
+        cols, _, _ = generate(dec, SEED, n)
+        ws = torch.empty(lib.hpsp_unweight_workspace_size(n), dtype=torch.uint8, device=DEV)
+        top = torch.empty(1, dtype=torch.float64, device=DEV)
+        capi.check(lib.hpsp_max_weight(ctypes.byref(dec), ctypes.byref(f), ptr(cols), n, n, ptr(ws),
+                                       ws.numel(), ptr(top), stream_handle()), "hpsp_max_weight")
+        want = unweight(dec, cols, UW, f=f, max_value=float(top.item()))
+        for out, idx in ((True, True), (False, True), (True, False), (False, False)):
+            got = unweight(dec, cols, UW, f=f, want_out=out, want_idx=idx)
+            assert got[0] == want[0]
+            for a, b in zip(got[1:3], want[1:3]):
+                assert a is None or torch.equal(a, b)
