@@ -4,7 +4,7 @@
 //
 //   Evaluate(mother, result, functors...)   EvalMother.h:283-306
 //     the event's engine is the PhaseSpace seed discarded by evt + 3N, as in
-//     Generate: the wave shares its squares words (EventWords).
+//     Generate: the block shares its engine words (BlockEventWords).
 //   Evaluate(mothers, result, functors...)  EvalMothers.h:145-273
 //     each event seeds its own engine with pair_hash(evt, seed) and does not
 //     discard, so every lane evaluates its own words (LaneWords); fECM and the
@@ -20,17 +20,13 @@ constexpr int kNumN = HPSP_MAX_N - 1;
 constexpr int kNumE = 6;
 
 template <int N, int E>
-static void eval_one(bool mothers, const EvalArgs& in, hipStream_t s) {
-  EvalArgs a = in;
-  // runs over one mother (as Generate); over mothers each lane seeds its own
-  // engine, one group per wave
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  a.run = mothers ? 1u : run_groups(ngroups);
-  const unsigned g = grid_for_runs((ngroups + a.run - 1) / a.run);
-  if (mothers)
-    hipLaunchKernelGGL((k_evaluate_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_evaluate_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+static void eval_one(bool mothers, const EvalArgs& a, hipStream_t s) {
+  over_grids(a, [&](const EvalArgs& c, unsigned g) {
+    if (mothers)
+      hipLaunchKernelGGL((k_evaluate_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, c);
+    else
+      hipLaunchKernelGGL((k_evaluate_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, c);
+  });
 }
 
 template <int I>

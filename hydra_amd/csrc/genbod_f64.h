@@ -158,17 +158,6 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
   return wt;
 }
 
-// Column stores of the generation kernels: plain global stores.  Where the
-// columns start on cache lines these write whole lines and stream as fast as
-// non-temporal ones; where a caller's column stride leaves a group's lines
-// partial, plain stores let L2 merge the neighbouring groups' halves, where
-// non-temporal ones sent each partial line to HBM on its own (3-body Generate
-// of 2^27 events at a stride of n + 1: 3.0-4.1 ms against 4.7 ms).
-template <typename T>
-__device__ __forceinline__ void st(T* ptr, T v) {
-  *glob(ptr) = v;
-}
-
 // AverageOn's value of a described functor: divisions through reciprocals
 // (the result is compared within a tolerance, not bit for bit).  A user's
 // callable brings its own overload (found by argument-dependent lookup).
@@ -296,87 +285,79 @@ struct LaneWords {
   }
 };
 
-// Evaluate (EvalMother.h:283-306, EvalMothers.h:145-273): runs of a.run
-// consecutive groups of 64 events per wave, as in k_generate_f64: over one mother the squares words of a group's second half
-// are the next group's first.
+// Evaluate (EvalMother.h:283-306, EvalMothers.h:145-273): one group of 64
+// events per wave, as k_generate_f64; over one mother the block's events share
+// their engine words.
 template <int N, int ENGINE, bool MOTHERS, typename FS = DescSet>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : point_waves_for(N), 8)))
 void k_evaluate_f64(const EvalArgsT<FS> a) {
-  __shared__ typename EventWords<N, ENGINE>::Window win[MOTHERS ? 1 : kBlock / kWave];
+  struct Nothing {};
+  __shared__ std::conditional_t<MOTHERS, Nothing, typename BlockEventWords<N, ENGINE>::Store> sw;
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t run_len = a.run ? a.run : 1;  // the launcher sets it; 0 reads as 1
-  const uint64_t nruns = (ngroups + run_len - 1) / run_len;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave; run < nruns;
-       run += nwaves) {
-    const uint64_t g_first = run * run_len;
-    const uint64_t g_end = (g_first + run_len < ngroups) ? g_first + run_len : ngroups;
-    EventWords<N, ENGINE> ewords;
-    for (uint64_t g = g_first; g < g_end; ++g) {
-      const uint64_t k0 = g * kWave;
-      const uint64_t k = k0 + (uint64_t)lane;
-      const bool live = k < a.n;
-      constexpr int P = N + (MOTHERS ? 1 : 0);
-      double p[P][4];
-      double wt;
-      if constexpr (MOTHERS) {
-        const uint64_t km = live ? k : 0;
-        double m4[4];
+  const uint64_t kb = (uint64_t)blockIdx.x * kBlock;
+  [[maybe_unused]] BlockEventWords<N, ENGINE> bwords;
+  if constexpr (!MOTHERS) bwords.fill(sw, a.d, a.first + kb);
+  const uint64_t k0 = kb + (uint64_t)(wave * kWave);
+  if (k0 >= a.n) return;  // wave-uniform
+  const uint64_t k = k0 + (uint64_t)lane;
+  const bool live = k < a.n;
+  constexpr int P = N + (MOTHERS ? 1 : 0);
+  double p[P][4];
+  double wt;
+  if constexpr (MOTHERS) {
+    const uint64_t km = live ? k : 0;
+    double m4[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) m4[c] = a.mothers[(uint64_t)c * a.mld + km];
-        // fECM = mother.mass() - sum(m); maximum weight of this mother
-        // (EvalMothers.h:151-176)
-        DecayK d = a.d;
-        {
+    for (int c = 0; c < 4; ++c) m4[c] = a.mothers[(uint64_t)c * a.mld + km];
+    // fECM = mother.mass() - sum(m); maximum weight of this mother
+    // (EvalMothers.h:151-176)
+    DecayK d = a.d;
+    {
 #pragma clang fp contract(off)
-          double te = mass_of(m4[0], m4[1], m4[2], m4[3]);
+      double te = mass_of(m4[0], m4[1], m4[2], m4[3]);
 #pragma unroll
-          for (int i = 0; i < N; ++i) te -= d.m[i];
-          d.mas0 = 0.0 * te + d.msum[0];
-          d.masN = 1.0 * te + d.msum[N - 1];
-          d.rmasN = rcp_fast(d.masN);
-          d.plain = d.plain_m && te >= 0.0 && te <= 0x1p+299;
-          double emmax = te + d.m[0], emmin = 0.0, wtmax = 1.0;
+      for (int i = 0; i < N; ++i) te -= d.m[i];
+      d.mas0 = 0.0 * te + d.msum[0];
+      d.masN = 1.0 * te + d.msum[N - 1];
+      d.rmasN = rcp_fast(d.masN);
+      d.plain = d.plain_m && te >= 0.0 && te <= 0x1p+299;
+      double emmax = te + d.m[0], emmin = 0.0, wtmax = 1.0;
 #pragma unroll
-          for (int i = 1; i < N; ++i) {
-            emmin += d.m[i - 1];
-            emmax += d.m[i];
-            wtmax *= pdk(emmax, emmin, d.m[i]);
-          }
-          d.ecm = te;
-          d.maxw = 1.0 / wtmax;
-        }
-        LaneWords<N, ENGINE> words;
-        words.init(pair_hash(a.first + k, a.seed));
-        double q[N][4];
-        wt = genbod_f64<N, ENGINE>(d, words, q);
-        const double bx = m4[1] / m4[0], by = m4[2] / m4[0], bz = m4[3] / m4[0];
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          boost_general(q[i], bx, by, bz);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) p[i + 1][c] = q[i][c];
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) p[0][c] = m4[c];
-      } else {
-        ewords.next(win[wave], a.d, a.first + k0, lane, g == g_first);
-        wt = genbod_f64<N, ENGINE>(a.d, ewords, p);
-        if (a.d.do_boost) {
-#pragma unroll
-          for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);
-        }
+      for (int i = 1; i < N; ++i) {
+        emmin += d.m[i - 1];
+        emmax += d.m[i];
+        wtmax *= pdk(emmax, emmin, d.m[i]);
       }
-      if (live) {
-        double* out = a.out + k0;
-        st(uniform_ptr(out) + lane, wt);
-        eval_set(a.fs, p, [&](int j, double v) {
-          st(uniform_ptr(out + (uint64_t)(1 + j) * a.ld) + lane, v);
-        });
-      }
+      d.ecm = te;
+      d.maxw = 1.0 / wtmax;
     }
+    LaneWords<N, ENGINE> words;
+    words.init(pair_hash(a.first + k, a.seed));
+    double q[N][4];
+    wt = genbod_f64<N, ENGINE>(d, words, q);
+    const double bx = m4[1] / m4[0], by = m4[2] / m4[0], bz = m4[3] / m4[0];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      boost_general(q[i], bx, by, bz);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) p[i + 1][c] = q[i][c];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) p[0][c] = m4[c];
+  } else {
+    wt = genbod_f64<N, ENGINE>(a.d, bwords, p);
+    if (a.d.do_boost) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);
+    }
+  }
+  if (live) {
+    double* out = a.out + k0;
+    st(uniform_ptr(out) + lane, wt);
+    eval_set(a.fs, p, [&](int j, double v) {
+      st(uniform_ptr(out + (uint64_t)(1 + j) * a.ld) + lane, v);
+    });
   }
 }
 

@@ -11,77 +11,60 @@
 
 namespace hpsp {
 
-// Each wave takes runs of a.run consecutive groups of 64 events (grid-stride
-// over runs): a group's second 64 words (or Random123 blocks) are the next
-// group's first, so within a run each lane evaluates one per group instead of
-// two.  COLS = false is the weights pass of a deferred Generate
-// (no momentum columns): without the column stores' addresses and store
-// paths in its loop, the scalar registers it spills are reloaded outside the
-// loop only.
+// One group of 64 consecutive events per wave; the block's 256 events share
+// their engine words through LDS (BlockEventWords: about one word or Random123
+// block evaluated per event).  Without a loop over groups nothing is kept in
+// scalar registers from one to the next and spilled, and blocks are dispatched
+// in order, so the chip's stores stay in a narrow moving window of the columns.
+// COLS = false is the weights pass of a deferred Generate (no momentum columns).
+// Against runs of up to 16 groups per wave (91 registers and 5 waves per SIMD
+// for 3 bodies, 142 and 3 for 10; now 56 and 8, 120 and 4): 1e6 3-body events
+// 23.3 -> 20.1 us, 3e6 4-body Threefry ones 101 -> 86 us, 2^24 10-body ones 1.50
+// -> 1.47 ms, mixed near threshold 653 -> 608 us, Evaluate of 1e7 164 -> 148 us.
 template <int N, int ENGINE, bool MOTHERS, bool COLS = true>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : point_waves_for(N), 8)))
 void k_generate_f64(const GenArgs a) {
-  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
+  __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
   const int lane = __lane_id();
   // wave index as a scalar so that column bases stay in SGPRs and every
   // store is (scalar base) + lane * 8
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t run_len = a.run ? a.run : 1;  // the launcher sets it; 0 reads as 1
-  const uint64_t nruns = (ngroups + run_len - 1) / run_len;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave; run < nruns;
-       run += nwaves) {
-    const uint64_t g_first = run * run_len;
-    const uint64_t g_end = (g_first + run_len < ngroups) ? g_first + run_len : ngroups;
-    EventWords<N, ENGINE> words;
-    for (uint64_t g = g_first; g < g_end; ++g) {
-      const uint64_t k0 = g * kWave;
-      const uint64_t k = k0 + (uint64_t)lane;
-      const bool live = k < a.n;
+  const uint64_t kb = (uint64_t)blockIdx.x * kBlock;
+  BlockEventWords<N, ENGINE> words;
+  words.fill(sw, a.d, a.first + kb);
+  const uint64_t k0 = kb + (uint64_t)(wave * kWave);
+  if (k0 >= a.n) return;  // wave-uniform
+  const uint64_t k = k0 + (uint64_t)lane;
+  const bool live = k < a.n;
+  double p[N][4];
+  const double wt = genbod_f64<N, ENGINE>(a.d, words, p);
 
-      words.next(win[wave], a.d, a.first + k0, lane, g == g_first);
-      double p[N][4];
-      const double wt = genbod_f64<N, ENGINE>(a.d, words, p);
-
-      if constexpr (MOTHERS) {
-        // applyBoostTo(mother) with beta = p/E (DecayMothers.h:228-233).
-        const uint64_t km = live ? k : 0;
-        const double e = a.mothers[km];
-        const double bx = a.mothers[a.mld + km] / e;
-        const double by = a.mothers[2 * a.mld + km] / e;
-        const double bz = a.mothers[3 * a.mld + km] / e;
+  if constexpr (MOTHERS) {
+    // applyBoostTo(mother) with beta = p/E (DecayMothers.h:228-233).
+    const uint64_t km = live ? k : 0;
+    const double e = a.mothers[km];
+    const double bx = a.mothers[a.mld + km] / e;
+    const double by = a.mothers[2 * a.mld + km] / e;
+    const double bz = a.mothers[3 * a.mld + km] / e;
 #pragma unroll
-        for (int i = 0; i < N; ++i) boost_general(p[i], bx, by, bz);
-      } else {
-        if (a.d.do_boost) {
+    for (int i = 0; i < N; ++i) boost_general(p[i], bx, by, bz);
+  } else {
+    if (a.d.do_boost) {
 #pragma unroll
-          for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);
-        }
-      }
-
-      if (live) {
-        if (!COLS || !a.cols) {
-          // weights only: the momenta are formed for them and not stored
-        } else if (a.out_f32) {
-          float* c = static_cast<float*>(a.cols) + k0;
-#pragma unroll
-          for (int i = 0; i < N; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, (float)p[i][q]);
-        } else {
-          double* c = static_cast<double*>(a.cols) + k0;
-#pragma unroll
-          for (int i = 0; i < N; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, p[i][q]);
-        }
-        if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
-        if (a.evw) st(uniform_ptr(a.evw + k0) + lane, event_weight_f64<N>(p, a.d.m, a.d.maxw));
-      }
+      for (int i = 0; i < N; ++i) boost_folded(p[i], a.d);
     }
+  }
+
+  if (live) {
+    if (!COLS || !a.cols) {
+      // weights only: the momenta are formed for them and not stored
+    } else if (a.out_f32) {
+      store_columns<N>(static_cast<float*>(a.cols) + k0, a.ld, lane, p);
+    } else {
+      store_columns<N>(static_cast<double*>(a.cols) + k0, a.ld, lane, p);
+    }
+    if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
+    if (a.evw) st(uniform_ptr(a.evw + k0) + lane, event_weight_f64<N>(p, a.d.m, a.d.maxw));
   }
 }
 
@@ -96,7 +79,7 @@ void k_generate_f64(const GenArgs a) {
 //
 // One group of 64 events per wave (the block's engine words are evaluated once
 // each and shared through LDS, so an event costs one word or Random123 block,
-// as in k_generate_f64's runs).  The block's 256
+// as in k_generate_f64).  The block's 256
 // events fall into two contiguous runs of the output, its accepted events and
 // its rejected ones; for N <= 6 they are staged in LDS in partition order and
 // every column is written by all 256 threads as those two runs, so that only
@@ -325,22 +308,15 @@ constexpr int kNumN = HPSP_MAX_N - 1;
 constexpr int kNumE = 6;
 
 template <int N, int E>
-static void gen_one(const GenArgs& in, hipStream_t s) {
-  GenArgs a = in;
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  // momentum columns of at most 3 daughters (with or without the weight
-  // column): bound by the stores (more daughters bring arithmetic enough to
-  // gain from 16)
-  uint64_t cap = (a.cols && N <= 3) ? kRunMaxStores : kRunMax;
-  if (a.run_cap && a.run_cap < cap) cap = a.run_cap;
-  a.run = run_groups(ngroups, cap);
-  const unsigned g = grid_for_runs((ngroups + a.run - 1) / a.run);
-  if (a.mothers)
-    hipLaunchKernelGGL((k_generate_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
-  else if (!a.cols)
-    hipLaunchKernelGGL((k_generate_f64<N, E, false, false>), dim3(g), dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_generate_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+static void gen_one(const GenArgs& a, hipStream_t s) {
+  over_grids(a, [&](const GenArgs& c, unsigned g) {
+    if (c.mothers)
+      hipLaunchKernelGGL((k_generate_f64<N, E, true>), dim3(g), dim3(kBlock), 0, s, c);
+    else if (!c.cols)
+      hipLaunchKernelGGL((k_generate_f64<N, E, false, false>), dim3(g), dim3(kBlock), 0, s, c);
+    else
+      hipLaunchKernelGGL((k_generate_f64<N, E, false>), dim3(g), dim3(kBlock), 0, s, c);
+  });
 }
 
 template <int N, int E>

@@ -135,66 +135,47 @@ __device__ __forceinline__ void final_boost_f32(float (&p)[N][4], const DecayK& 
   }
 }
 
-// Runs of a.run consecutive groups of 64 events per wave, as in
-// k_generate_f64 (one engine word or block per lane and group within a run).
+// One group of 64 events per wave, the block's engine words shared, as in
+// k_generate_f64.
 template <int N, int ENGINE, bool MOTHERS>
 __global__ __launch_bounds__(kBlock) void k_generate_mixed(const GenArgs a) {
-  __shared__ typename EventWords<N, ENGINE>::Window win[kBlock / kWave];
+  __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t run_len = a.run ? a.run : 1;  // the launcher sets it; 0 reads as 1
-  const uint64_t nruns = (ngroups + run_len - 1) / run_len;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-  for (uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave; run < nruns;
-       run += nwaves) {
-    const uint64_t g_first = run * run_len;
-    const uint64_t g_end = (g_first + run_len < ngroups) ? g_first + run_len : ngroups;
-    EventWords<N, ENGINE> words;
-    for (uint64_t g = g_first; g < g_end; ++g) {
-      const uint64_t k0 = g * kWave;
-      const uint64_t k = k0 + (uint64_t)lane;
-      const bool live = k < a.n;
-      words.next(win[wave], a.d, a.first + k0, lane, g == g_first);
-      float p[N][4];
-      const double wt = genbod_mixed<N, ENGINE>(a.d, words, p);
-      if constexpr (MOTHERS) {
-        const uint64_t km = live ? k : 0;
-        const float ie = __builtin_amdgcn_rcpf((float)a.mothers[km]);
-        const float bx = (float)a.mothers[a.mld + km] * ie;
-        const float by = (float)a.mothers[2 * a.mld + km] * ie;
-        const float bz = (float)a.mothers[3 * a.mld + km] * ie;
+  const uint64_t kb = (uint64_t)blockIdx.x * kBlock;
+  BlockEventWords<N, ENGINE> words;
+  words.fill(sw, a.d, a.first + kb);
+  const uint64_t k0 = kb + (uint64_t)(wave * kWave);
+  if (k0 >= a.n) return;  // wave-uniform
+  const uint64_t k = k0 + (uint64_t)lane;
+  const bool live = k < a.n;
+  float p[N][4];
+  const double wt = genbod_mixed<N, ENGINE>(a.d, words, p);
+  if constexpr (MOTHERS) {
+    const uint64_t km = live ? k : 0;
+    const float ie = __builtin_amdgcn_rcpf((float)a.mothers[km]);
+    const float bx = (float)a.mothers[a.mld + km] * ie;
+    const float by = (float)a.mothers[2 * a.mld + km] * ie;
+    const float bz = (float)a.mothers[3 * a.mld + km] * ie;
 #pragma unroll
-        for (int i = 0; i < N; ++i) boost_general_f32(p[i], bx, by, bz);
-      } else {
-        final_boost_f32<N>(p, a.d);
-      }
-      if (live) {
-        if (!a.cols) {
-          // weights only
-        } else if (a.out_f32) {
-          float* c = static_cast<float*>(a.cols) + k0;
-#pragma unroll
-          for (int i = 0; i < N; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              *(glob_u(c + (uint64_t)(4 * i + q) * a.ld) + lane) = p[i][q];
-        } else {
-          double* c = static_cast<double*>(a.cols) + k0;
-#pragma unroll
-          for (int i = 0; i < N; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              *(glob_u(c + (uint64_t)(4 * i + q) * a.ld) + lane) = (double)p[i][q];
-        }
-        if (a.wt) *(glob_u(a.wt + k0) + lane) = wt;
-        // PhaseSpaceWeight of the mixed form: the FP64 generation weight,
-        // which it equals in exact arithmetic.  Recomputed from the FP32
-        // momenta (masses of running sums, then pdk) it would lose up to all
-        // of its digits where a - b - c cancels near threshold.
-        if (a.evw) *(glob_u(a.evw + k0) + lane) = wt;
-      }
+    for (int i = 0; i < N; ++i) boost_general_f32(p[i], bx, by, bz);
+  } else {
+    final_boost_f32<N>(p, a.d);
+  }
+  if (live) {
+    if (!a.cols) {
+      // weights only
+    } else if (a.out_f32) {
+      store_columns<N>(static_cast<float*>(a.cols) + k0, a.ld, lane, p);
+    } else {
+      store_columns<N>(static_cast<double*>(a.cols) + k0, a.ld, lane, p);
     }
+    if (a.wt) *(glob_u(a.wt + k0) + lane) = wt;
+    // PhaseSpaceWeight of the mixed form: the FP64 generation weight,
+    // which it equals in exact arithmetic.  Recomputed from the FP32
+    // momenta (masses of running sums, then pdk) it would lose up to all
+    // of its digits where a - b - c cancels near threshold.
+    if (a.evw) *(glob_u(a.evw + k0) + lane) = wt;
   }
 }
 
@@ -428,20 +409,13 @@ static void regen_mixed_one(const UnweightArgs& a, hipStream_t s) {
 }
 
 template <int N, int E>
-static void gen_one(const GenArgs& in, hipStream_t s) {
-  GenArgs a = in;
-  const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  // momentum columns of at most 3 daughters (with or without the weight
-  // column): bound by the stores (more daughters bring arithmetic enough to
-  // gain from 16)
-  uint64_t cap = (a.cols && N <= 3) ? kRunMaxStores : kRunMax;
-  if (a.run_cap && a.run_cap < cap) cap = a.run_cap;
-  a.run = run_groups(ngroups, cap);
-  const unsigned g = grid_for_runs((ngroups + a.run - 1) / a.run);
-  if (a.mothers)
-    hipLaunchKernelGGL((k_generate_mixed<N, E, true>), dim3(g), dim3(kBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_generate_mixed<N, E, false>), dim3(g), dim3(kBlock), 0, s, a);
+static void gen_one(const GenArgs& a, hipStream_t s) {
+  over_grids(a, [&](const GenArgs& c, unsigned g) {
+    if (c.mothers)
+      hipLaunchKernelGGL((k_generate_mixed<N, E, true>), dim3(g), dim3(kBlock), 0, s, c);
+    else
+      hipLaunchKernelGGL((k_generate_mixed<N, E, false>), dim3(g), dim3(kBlock), 0, s, c);
+  });
 }
 
 template <int N, int E>

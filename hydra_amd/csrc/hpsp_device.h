@@ -20,6 +20,11 @@ constexpr int kWave = 64;
 // one-event-per-lane kernels: the FP64 chains are long and dependent, so
 // occupancy hides their latency; larger N needs more live momenta.
 constexpr int waves_for(int N) { return N <= 4 ? 4 : (N <= 6 ? 3 : (N <= 10 ? 2 : 1)); }
+// The same for Generate and Evaluate, one group per wave without a loop over
+// groups: what their registers allow without spills.
+constexpr int point_waves_for(int N) {
+  return N <= 3 ? 8 : (N == 4 ? 6 : (N <= 6 ? 5 : (N <= 10 ? 4 : 3)));
+}
 
 // Kernel-side decay description; everything that depends only on the decay
 // is folded on the host (engine keys, final boost constants).
@@ -69,6 +74,37 @@ __device__ __forceinline__ gptr<T> glob(T* p) {
 template <typename T>
 __device__ __forceinline__ gptr<T> glob_u(T* p) {
   return (gptr<T>)uniform_ptr(p);
+}
+
+// Column stores of the generation kernels: plain global stores.  Where the
+// columns start on cache lines these write whole lines and stream as fast as
+// non-temporal ones; where a caller's column stride leaves a group's lines
+// partial, plain stores let L2 merge the neighbouring groups' halves, where
+// non-temporal ones sent each partial line to HBM on its own (3-body Generate
+// of 2^27 events at a stride of n + 1: 3.0-4.1 ms against 4.7 ms).
+template <typename T>
+__device__ __forceinline__ void st(T* ptr, T v) {
+  *glob(ptr) = v;
+}
+
+// The 4N columns of a group of 64 events, the first of which is at base: the
+// column's address is stepped from one to the next in scalar registers (the
+// compiler would form them all ahead, by 64-bit products, and spill).
+template <int N, typename T, typename R>
+__device__ __forceinline__ void store_columns(T* base, uint64_t ld, int lane,
+                                              const R (&p)[N][4]) {
+  T* c = uniform_ptr(base);
+  const uint64_t step = ld * sizeof(T);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      st(c + lane, (T)p[i][q]);
+      uint64_t v = reinterpret_cast<uint64_t>(c) + step;
+      asm("" : "+s"(v));
+      c = reinterpret_cast<T*>(v);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

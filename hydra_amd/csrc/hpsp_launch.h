@@ -26,8 +26,18 @@ struct GenArgs {
   double* evw;
   const double* mothers;  // FP64 mother columns (E,px,py,pz) or null
   uint64_t mld;
-  uint32_t run;      // consecutive groups of 64 events per wave (>= 1; set by the launcher)
-  uint32_t run_cap;  // 0: the launcher's policy; else the longest run allowed
+
+  // the same call's events from off on, n of them
+  GenArgs part(uint64_t off, uint64_t count) const {
+    GenArgs c = *this;
+    c.first += off;
+    c.n = count;
+    if (c.cols) c.cols = static_cast<char*>(c.cols) + off * (out_f32 ? 4 : 8);
+    if (c.wt) c.wt += off;
+    if (c.evw) c.evw += off;
+    if (c.mothers) c.mothers += off;
+    return c;
+  }
 };
 
 // AverageOn arguments; FK is the functor: a FunctorK description here, a
@@ -61,7 +71,15 @@ struct EvalArgsT {
   uint64_t mld;
   double* out;              // 1 + nf columns of ld doubles
   uint64_t ld;
-  uint32_t run;             // consecutive groups of 64 events per wave (set by the launcher)
+
+  EvalArgsT part(uint64_t off, uint64_t count) const {
+    EvalArgsT c = *this;
+    c.first += off;
+    c.n = count;
+    if (c.mothers) c.mothers += off;
+    c.out += off;
+    return c;
+  }
 };
 using EvalArgs = EvalArgsT<DescSet>;
 
@@ -272,17 +290,23 @@ int launch_unweight_sample(int ncols, const UnweightArgs& a, double* block_max,
 int launch_rng_words(int engine, const uint64_t* key, uint64_t discard, uint64_t n,
                      uint64_t* out, hipStream_t s);
 
-// Blocks for a grid-stride launch over `items` work items of kBlock each.
-// Groups of 64 events per wave in a generation run (k_generate_*,
-// k_evaluate_f64 over one mother): a longer run shares more engine words
-// between consecutive groups, but the runs must still give every SIMD several
-// waves; the longest power of two up to max_run that leaves kRunMinRuns runs.
-// A launch bound by its column stores (momenta of at most 3 daughters, with or
-// without the weight column) takes max_run = kRunMaxStores: longer runs spread
-// the chip's concurrent writes over a wider window of the columns (3-body
-// momenta alone at 2^27 events: 2.25 ms with runs of 4, 2.42 ms with 16;
-// momenta and weights 2.55 ms against 2.63-2.69), where launches with more
-// arithmetic per byte gain from 16 (4 to 8 daughters: 2-4%).
+// One launch(args, blocks) of kBlock events per block for every 2^31 events (a
+// dispatch holds fewer than 2^32 work-items).
+constexpr uint64_t kGridEvents = 1ULL << 31;
+template <typename Args, typename Launch>
+inline void over_grids(const Args& a, Launch&& launch) {
+  for (uint64_t off = 0; off < a.n; off += kGridEvents) {
+    const uint64_t n = a.n - off < kGridEvents ? a.n - off : kGridEvents;
+    launch(a.part(off, n), (unsigned)((n + kBlock - 1) / kBlock));
+  }
+}
+
+// Groups of 64 elements per wave in a run of k_range_generate: a longer run
+// shares more engine words between consecutive groups, but the runs must still
+// give every SIMD several waves; the longest power of two up to max_run that
+// leaves kRunMinRuns runs.  A launch bound by its column stores (momenta of at
+// most 3 daughters) takes max_run = kRunMaxStores: longer runs spread the chip's
+// concurrent writes over a wider window of the columns.
 inline uint32_t run_groups(uint64_t ngroups, uint64_t max_run = kRunMax) {
   uint64_t r = 1;
   while (r < max_run && ngroups >= 2 * r * kRunMinRuns) r *= 2;
@@ -315,6 +339,7 @@ inline void launch_avg(uint64_t n, int waves_wide, Narrow&& narrow, Wide&& wide)
 // per SIMD (65536 took that block 42 us).
 constexpr unsigned kMaxBlocks = 2048;
 
+// Blocks for a grid-stride launch over `items` work items of kBlock each.
 inline unsigned grid_for(uint64_t items, unsigned cap = 65536u) {
   const uint64_t b = (items + kBlock - 1) / kBlock;
   return (unsigned)(b == 0 ? 1 : (b < cap ? b : cap));

@@ -338,10 +338,6 @@ struct hpsp_server {
         a.ld = q->ld;
         a.out_f32 = q->r.out_f32;
         a.evw = q->weights ? q->weights + it.off : nullptr;
-        // chunks of several streams share the chip: one group per wave (runs
-        // lengthen the waves, and with them the tails of concurrent chunks;
-        // 9% less throughput at saturation)
-        a.run_cap = 1;
         e = (q->r.prec == HPSP_FP64) ? launch_generate_f64(N, E, a, s)
                                      : launch_generate_mixed(N, E, a, s);
       } else {

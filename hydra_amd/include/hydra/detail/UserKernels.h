@@ -371,13 +371,12 @@ void user_evaluate_t(hydra::tuple<T...>*, hpsp_decay const& d, uint64_t seed,
   static_assert(pack_width<hydra::tuple<T...>, FnPack<F...>>::value == (int)sizeof...(F),
                 "Evaluate: each functor returns one value");
   if (n == 0) return;
-  const uint64_t ngroups = (n + hpsp::kWave - 1) / hpsp::kWave;
-  const uint32_t run = MOTHERS ? 1u : hpsp::run_groups(ngroups);
-  hpsp::EvalArgsT<FS> a{hpsp::make_decayk(&d, seed), FS{make_pack(f...)}, seed, first, n,
-                        mothers, mld, out, ld, run};
-  const unsigned g = hpsp::grid_for_runs((ngroups + run - 1) / run);
-  hipLaunchKernelGGL((hpsp::k_evaluate_f64<(int)N, ENGINE, MOTHERS, FS>), dim3(g),
-                     dim3(hpsp::kBlock), 0, 0, a);
+  const hpsp::EvalArgsT<FS> a{hpsp::make_decayk(&d, seed), FS{make_pack(f...)}, seed, first, n,
+                              mothers, mld, out, ld};
+  hpsp::over_grids(a, [](const hpsp::EvalArgsT<FS>& c, unsigned g) {
+    hipLaunchKernelGGL((hpsp::k_evaluate_f64<(int)N, ENGINE, MOTHERS, FS>), dim3(g),
+                       dim3(hpsp::kBlock), 0, 0, c);
+  });
   hip_check(hipGetLastError(), "PhaseSpace::Evaluate");
   hpsp_sync("PhaseSpace::Evaluate");
 }
