@@ -218,6 +218,8 @@ int evaluate_common(const hpsp_decay* d, const hpsp_functor* fs, int nf, uint64_
     if (rc) return rc;
   }
   a.fs.nf = nf;
+  for (int j = 0; j < nf; ++j)
+    a.fs.pairs |= a.fs.f[j].kind != HPSP_F_ONE && a.fs.f[j].kind != HPSP_F_COS_HELICITY;
   a.seed = seed;
   a.first = first;
   a.n = n;

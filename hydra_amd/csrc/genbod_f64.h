@@ -11,17 +11,20 @@
 // formed with the same operations except: exactly-zero terms are dropped,
 // products and sums are fused (one rounding instead of two), sin/cos and
 // square roots outside the weight chain are evaluated to about one ulp, and
-// the boost factors use gamma = E*/M, gamma*beta = p/M.
+// the boost factors use gamma*beta = p/M, gamma = sqrt(1 + (p/M)^2).
 //
 // GENBOD is bound by its vector instructions.  The fused forms, the weight
 // chain and PhaseSpaceWeight without a branch and a library path per square
 // root, one reciprocal per invariant mass for the chain's division and the
 // boost, and the decay's constants formed on the host took the 10-body
-// Generate of 2^24 events from 1.89 to 1.57 ms (193 -> 144 registers, 3 waves
-// per SIMD instead of 2), AverageOn of the 3-body Dalitz model over 2^24
-// events from 239 to 221 us, Evaluate of 10^7 events from 174 to 164 us.  The
-// momenta's errors against extended precision did not grow (3 bodies: 2.28 ->
-// 2.26e-16 E RMS; 10: 1.51 -> 1.47e-15).
+// Generate of 2^24 events from 1.89 to 1.57 ms, AverageOn of the 3-body Dalitz
+// model over 2^24 events from 239 to 221 us, Evaluate of 10^7 events from 174 to
+// 164 us.  gamma from gamma beta (one square root, no selects), the first
+// boost's back-to-back pair formed once and no guard on the energies' square
+// roots: 1e6 3-body events 20.1 -> 18.8 us, the 10-body Generate 1.47 -> 1.44 ms,
+// AverageOn 208 -> 199 us, Evaluate 145 -> 137 us.  The momenta's errors against
+// extended precision did not grow (3 bodies: 2.28 -> 2.24e-16 E RMS; 10: 1.51 ->
+// 1.47e-15).
 #pragma once
 
 #include <type_traits>
@@ -63,17 +66,19 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
   // RN(s / a) / 2, with the reciprocal of invMas[n] shared with the boost.
   double wt = d.maxw;
   double pd[N - 1];
-  double rmas[N];  // 1 / invMas[1 .. N-1]
+  double gb[N - 1];  // gamma beta of the boost of step i = 1 .. N-2, pd[i] / invMas[i]
+  double ra = 0.0;   // 1 / invMas[n]
   bool ok = d.plain != 0;
-  rmas[N - 1] = d.rmasN;
 #pragma unroll
   for (int n = 0; n < N - 1; ++n) {
     const double a = invMas[n + 1];
     const double x = pdk_radicand(a, invMas[n], d.m[n + 1]);
     ok = ok & sqrt_range(x);
-    if (n < N - 2) rmas[n + 1] = rcp_fast(a);
-    pd[n] = 0.5 * div_core(sqrt_core(x), a, rmas[n + 1]);
+    const double rn = n < N - 2 ? rcp_fast(a) : d.rmasN;
+    pd[n] = 0.5 * div_core(sqrt_core(x), a, rn);
     wt *= pd[n];
+    if (n > 0) gb[n] = pd[n] * ra;
+    ra = rn;
   }
   if (__builtin_expect(!ok, 0)) {
     wt = d.maxw;
@@ -82,21 +87,24 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
       pd[n] = __builtin_sqrt(pdk_radicand(invMas[n + 1], invMas[n], d.m[n + 1])) /
               (2 * invMas[n + 1]);
       wt *= pd[n];
+      // for pd = 0 (beta = 0; NaN) the reference's boost does nothing
+      if (n > 0) gb[n] = pd[n] > 0.0 ? pd[n] * rcp_fast(invMas[n]) : 0.0;
     }
   }
 
   // Daughter 0 along +y; it is rotated for the first time at i = 1.
-  p[0][0] = sqrt_fast(__builtin_fma(pd[0], pd[0], d.msq[0]));
+  p[0][0] = sqrt_pos(__builtin_fma(pd[0], pd[0], d.msq[0]));
   p[0][1] = 0.0;
   p[0][2] = pd[0];
   p[0][3] = 0.0;
 
+  [[maybe_unused]] double y0 = 0.0, gy0 = 0.0;  // step 1: py of daughter 0, gamma py
 #pragma unroll
   for (int i = 1; i < N; ++i) {
     // keep the scheduler from hoisting later steps' angles and boosts
     // above this one: their results would all be live at once
     if constexpr (N > 4) __builtin_amdgcn_sched_barrier(0);
-    p[i][0] = sqrt_fast(__builtin_fma(pd[i - 1], pd[i - 1], d.msq[i]));
+    p[i][0] = sqrt_pos(__builtin_fma(pd[i - 1], pd[i - 1], d.msq[i]));
     p[i][1] = 0.0;
     p[i][2] = -pd[i - 1];
     p[i][3] = 0.0;
@@ -113,7 +121,11 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
 #pragma unroll
     for (int j = 0; j <= i; ++j) {
       const bool fresh = (j == i) || (i == 1);  // px = pz = 0 before this rotation
-      if (fresh) {
+      if (i == 1 && j == 1) {  // back to back with daughter 0
+        p[1][1] = -p[0][1];
+        p[1][2] = -p[0][2];
+        p[1][3] = -p[0][3];
+      } else if (fresh) {
         const double y = p[j][2];
         const double t = -(sZ * y);  // cZ*0 - sZ*y
         p[j][2] = cZ * y;            // sZ*0 + cZ*y
@@ -133,25 +145,28 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
     if (i == N - 1) break;
 
     // Boost along +y by beta = pd/sqrt(pd^2 + M^2) (Vector3R(0, beta, 0)):
-    // only E and py change.  With E* = sqrt(pd^2 + M^2) the reference's
-    // gamma = 1/sqrt(1 - beta^2), gamma*beta and (gamma-1)/beta^2 * beta^2 are
-    // E*/M, pd/M and gamma - 1; the momenta are formed as
-    // E' = gamma E + gamma beta py and py' = gamma beta E + gamma py.
-    // For pd = 0 (beta = 0) the reference's boost does nothing; here gamma = 1
-    // and gamma beta = 0 are selected instead, which leave E and py as they
-    // are (up to the sign of a zero py): a branch costs register moves on
-    // every event, selects of the boosted components 4(i+1) instructions.
+    // only E and py change.  The reference's gamma = 1/sqrt(1 - beta^2) and
+    // gamma*beta are sqrt(1 + (pd/M)^2) and pd/M; (gamma-1)/beta^2 * beta^2 is
+    // gamma - 1.  The momenta are formed as E' = gamma E + gamma beta py and
+    // py' = gamma beta E + gamma py: for gamma beta = 0 as they were (up to the
+    // sign of a zero py).
     {
-      const bool boost = pd[i] > 0.0;
-      const double inv_m = rmas[i];
-      const double estar = sqrt_fast(__builtin_fma(pd[i], pd[i], invMas[i] * invMas[i]));
-      const double gamma = boost ? estar * inv_m : 1.0;
-      const double gby = boost ? pd[i] * inv_m : 0.0;
+      const double gby = gb[i];
+      const double gamma = sqrt_pos(__builtin_fma(gby, gby, 1.0));
 #pragma unroll
       for (int j = 0; j <= i; ++j) {
         const double e2 = p[j][0], py2 = p[j][2];
-        p[j][0] = __builtin_fma(gby, py2, gamma * e2);
-        p[j][2] = __builtin_fma(gby, e2, gamma * py2);
+        if (i == 1 && j == 1) {  // py2 = -p[0][2] before this boost: its product with gamma
+          p[1][0] = __builtin_fma(-gby, y0, gamma * e2);
+          p[1][2] = __builtin_fma(gby, e2, -gy0);
+        } else {
+          if (i == 1) {
+            y0 = py2;
+            gy0 = gamma * py2;
+          }
+          p[j][0] = __builtin_fma(gby, py2, gamma * e2);
+          p[j][2] = __builtin_fma(gby, e2, i == 1 ? gy0 : gamma * py2);
+        }
       }
     }
   }
@@ -181,7 +196,8 @@ __device__ __forceinline__ double avg_value(const FunctorK& f, const double (&p)
 constexpr int avg_wide_waves(int N) { return N <= 6 ? 16 : 8; }  // 128 or 256 registers
 
 template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorK, int WAVES = kBlock / kWave>
-__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+__global__ __launch_bounds__(WAVES * kWave)
+    __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? waves_for(N) : WAVES / 4, 8)))
 void k_average_f64(const AvgArgsT<FK> a) {
   constexpr int kFold = kBlock / kWave;  // waves that fold
   constexpr bool kWide = WAVES > kFold;
@@ -263,7 +279,8 @@ void k_average_f64(const AvgArgsT<FK> a) {
 // j's.  A user's set of callables brings its own overload.
 template <int P, typename Out>
 __device__ __forceinline__ void eval_set(const DescSet& s, const double (&p)[P][4], Out&& out) {
-  for (int j = 0; j < s.nf; ++j) out(j, functor_eval<double>(s.f[j], p));
+  const RegAcc<double, P> acc(p, s.pairs != 0);
+  for (int j = 0; j < s.nf; ++j) out(j, functor_eval_acc<double, true>(s.f[j], acc));
 }
 
 // Words of an engine seeded per event and not discarded.
@@ -289,7 +306,8 @@ struct LaneWords {
 // events per wave, as k_generate_f64; over one mother the block's events share
 // their engine words.
 template <int N, int ENGINE, bool MOTHERS, typename FS = DescSet>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : point_waves_for(N), 8)))
+__global__ __launch_bounds__(kBlock)
+    __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : eval_waves_for(N), 8)))
 void k_evaluate_f64(const EvalArgsT<FS> a) {
   struct Nothing {};
   __shared__ std::conditional_t<MOTHERS, Nothing, typename BlockEventWords<N, ENGINE>::Store> sw;

@@ -22,7 +22,8 @@ namespace hpsp {
 // 23.3 -> 20.1 us, 3e6 4-body Threefry ones 101 -> 86 us, 2^24 10-body ones 1.50
 // -> 1.47 ms, mixed near threshold 653 -> 608 us, Evaluate of 1e7 164 -> 148 us.
 template <int N, int ENGINE, bool MOTHERS, bool COLS = true>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : point_waves_for(N), 8)))
+__global__ __launch_bounds__(kBlock)
+    __attribute__((amdgpu_waves_per_eu(MOTHERS ? waves_for(N) : point_waves_for(N), 8)))
 void k_generate_f64(const GenArgs a) {
   __shared__ typename BlockEventWords<N, ENGINE>::Store sw;
   const int lane = __lane_id();

@@ -19,19 +19,22 @@ constexpr int kWave = 64;
 // Minimum waves per SIMD requested from the register allocator for the
 // one-event-per-lane kernels: the FP64 chains are long and dependent, so
 // occupancy hides their latency; larger N needs more live momenta.
-constexpr int waves_for(int N) { return N <= 4 ? 4 : (N <= 6 ? 3 : (N <= 10 ? 2 : 1)); }
+constexpr int waves_for(int N) {
+  return N <= 3 ? 5 : (N == 4 ? 4 : (N <= 6 ? 3 : (N <= 10 ? 2 : 1)));
+}
 // The same for Generate and Evaluate, one group per wave without a loop over
 // groups: what their registers allow without spills.
 constexpr int point_waves_for(int N) {
   return N <= 3 ? 8 : (N == 4 ? 6 : (N <= 6 ? 5 : (N <= 10 ? 4 : 3)));
 }
+constexpr int eval_waves_for(int N) { return N <= 3 ? 6 : (N <= 6 ? 5 : (N <= 10 ? 4 : 3)); }
 
 // Kernel-side decay description; everything that depends only on the decay
 // is folded on the host (engine keys, final boost constants).
 struct DecayK {
   double m[HPSP_MAX_N];
   double msum[HPSP_MAX_N];  // ((0 + m0) + m1) + ... + m[n], the chain's running sum
-  double msq[HPSP_MAX_N];   // m[n]^2
+  double msq[HPSP_MAX_N];   // m[n]^2, at least 2^-1000 (a sum with it is never 0)
   double ecm;
   double maxw;
   double mas0, masN;  // invMas[0] = 0 ecm + msum[0] and invMas[N-1] = 1 ecm + msum[N-1]
@@ -46,10 +49,16 @@ struct DecayK {
   int do_boost;
 };
 
+// A described functor; a Breit-Wigner term's constants are formed on the host:
+// with D = M^2 - s and g = M G its amplitude is c (D + i g) / (D^2 + g^2).
 struct FunctorK {
   int kind;
   int nterms;
-  double m[HPSP_MAX_TERMS], g[HPSP_MAX_TERMS], cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
+  double m2[HPSP_MAX_TERMS], mg[HPSP_MAX_TERMS], mg2[HPSP_MAX_TERMS];  // M^2, g, g^2
+  double cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
+  double cig[HPSP_MAX_TERMS], crg[HPSP_MAX_TERMS];  // ci g, cr g
+  float m2f[HPSP_MAX_TERMS], mg2f[HPSP_MAX_TERMS], crf[HPSP_MAX_TERMS], cif[HPSP_MAX_TERMS];
+  float cigf[HPSP_MAX_TERMS], crgf[HPSP_MAX_TERMS];
   int a[HPSP_MAX_TERMS], b[HPSP_MAX_TERMS];
 };
 
@@ -548,6 +557,18 @@ __device__ __forceinline__ double sqrt_fast(double x) {
   return __builtin_fma(d, h, g);
 }
 
+// The same for x > 0 (normal), without the guard.
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y;
+  double h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  const double d = __builtin_fma(-g, g, x);
+  return __builtin_fma(d, h, g);
+}
+
 // Reciprocal within about one ulp: estimate and two Newton steps.
 __device__ __forceinline__ double rcp_fast(double x) {
   double r = __builtin_amdgcn_rcp(x);
@@ -725,32 +746,65 @@ __device__ __forceinline__ Real pair_mass2(const Real (&u)[4], const Real (&w)[4
   return v[0] * v[0] - v[1] * v[1] - v[2] * v[2] - v[3] * v[3];
 }
 
-// Four-vectors of one event in registers (the generation kernels).
+// Four-vectors of one event in registers (the generation kernels); indices are
+// wave-uniform.  With at most four four-vectors the pair masses lie in a table of
+// all P(P-1)/2 pairs, formed once per event where a functor wants pairs: a pair
+// is then one of 3 or 6 scalars instead of two four-vector selections.  (Scalar
+// branches to each pair's own code cost more than the selects: AverageOn of the
+// 3-body Dalitz model over 2^24 events 217 us against 208, Evaluate of 10^7 153
+// against 145.)
 template <typename Real, int P>
 struct RegAcc {
   const Real (&p)[P][4];
-  // With at most four four-vectors, the functors of particle pairs take the
-  // pair masses from a table of all P(P-1)/2 pairs formed once per event
-  // (the pair named by wave-uniform indices is then one of 3 or 6 scalars)
-  // instead of selecting two four-vectors per term.
-  static constexpr bool kPairTable = P >= 2 && P <= 4;
+  static constexpr bool kTable = P >= 2 && P <= 4;
   static constexpr int kPairs = P * (P - 1) / 2;
-  __device__ __forceinline__ void pair_table(Real (&m2)[kPairs > 0 ? kPairs : 1]) const {
-    int k = 0;
+  Real m2[kTable ? kPairs : 1];
+  __device__ __forceinline__ RegAcc(const Real (&p_)[P][4], bool pairs) : p(p_) {
+    if constexpr (kTable) {
+      if (pairs) {  // wave-uniform
+        int k = 0;
 #pragma unroll
-    for (int a = 0; a < P; ++a)
+        for (int a = 0; a < P; ++a)
 #pragma unroll
-      for (int b = a + 1; b < P; ++b) m2[k++] = pair_mass2(p[a], p[b]);
-  }
-  // index in pair_table of the pair (a, b), a != b
-  __device__ __forceinline__ static int pair_index(int a, int b) {
-    const int lo = a < b ? a : b, hi = a < b ? b : a;
-    return lo * (2 * P - lo - 1) / 2 + (hi - lo - 1);
+          for (int b = a + 1; b < P; ++b) m2[k++] = pair_mass2(p[a], p[b]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < kPairs; ++k) m2[k] = 0;
+      }
+    }
   }
   __device__ __forceinline__ void get(int i, Real (&v)[4]) const { pick4(p, i, v); }
-  // p[first] + ... + p[last - 1], left to right, through the unrolled array
+  // (p[a] + p[b])^2
+  __device__ __forceinline__ Real pair(int a, int b) const {
+    if constexpr (kTable) {
+      if (a != b) {
+        const int lo = a < b ? a : b, hi = a < b ? b : a;
+        return pick1(m2, lo * (2 * P - lo - 1) / 2 + (hi - lo - 1));
+      }
+    }
+    Real u[4], v[4];
+    get(a, u);
+    get(b, v);
+    return pair_mass2(u, v);
+  }
+  // p[first] + ... + p[last - 1], left to right, through the unrolled array;
+  // all of them, or all but the first (the daughters beside their mother),
+  // without the selects
   __device__ __forceinline__ void sum(int first, int last, Real (&Pv)[4]) const {
 #pragma clang fp contract(off)
+    if (last == P && first <= 1) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) Pv[c] = p[1][c];
+      if (first == 0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) Pv[c] = p[0][c] + Pv[c];
+      }
+#pragma unroll
+      for (int i = 2; i < P; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) Pv[c] = Pv[c] + p[i][c];
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c) Pv[c] = 0;
 #pragma unroll
@@ -763,6 +817,11 @@ struct RegAcc {
     }
   }
 };
+
+// Whether a functor takes pair masses.
+__device__ __forceinline__ bool wants_pairs(const FunctorK& f) {
+  return f.kind != HPSP_F_ONE && f.kind != HPSP_F_COS_HELICITY;
+}
 
 // Three-momentum products of Vector4R (Vector4R.inl:372-386, 426-454).
 template <typename Real>
@@ -789,29 +848,9 @@ __device__ __forceinline__ void unit3(Real (&v)[4]) {
   for (int c = 0; c < 4; ++c) v[c] *= inv;
 }
 
-// Whether an accessor offers the table of pair masses (RegAcc with P <= 4).
-template <typename Acc, typename = void>
-struct has_pair_table : std::false_type {};
-template <typename Acc>
-struct has_pair_table<Acc, std::void_t<decltype(Acc::kPairTable)>>
-    : std::integral_constant<bool, Acc::kPairTable> {};
-template <typename Acc, bool = has_pair_table<Acc>::value>
-struct pair_table_size : std::integral_constant<int, 1> {};
-template <typename Acc>
-struct pair_table_size<Acc, true> : std::integral_constant<int, Acc::kPairs> {};
-template <typename Real, typename Acc>
-__device__ __forceinline__ Real pair_from_table(const Acc& acc, int a, int b) {
-  if constexpr (has_pair_table<Acc>::value) {
-    Real tab[Acc::kPairs];
-    acc.pair_table(tab);
-    return pick1(tab, Acc::pair_index(a, b));
-  } else {
-    return Real(0);
-  }
-}
-
-// Functor value of one event; acc.get(i, v) yields four-vector i and
-// acc.sum(first, last, P) the left-to-right sum of four-vectors [first, last).
+// Functor value of one event; acc.get(i, v) yields four-vector i, acc.pair(a, b)
+// the pair's mass squared and acc.sum(first, last, P) the left-to-right sum of
+// four-vectors [first, last).
 // The decay-plane angle (atan2 and two normalisations) is compiled only where
 // Plane is set, the kernels over stored particles: in the generation kernels
 // its registers would be reserved for every functor.
@@ -822,15 +861,7 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
   if (f.kind == HPSP_F_MASS2_01 || f.kind == HPSP_F_MASS2 || f.kind == HPSP_F_MASS) {
     const int ia = f.kind == HPSP_F_MASS2_01 ? 0 : f.a[0];
     const int ib = f.kind == HPSP_F_MASS2_01 ? 1 : f.b[0];
-    Real m2;
-    if (has_pair_table<Acc>::value && ia != ib) {
-      m2 = pair_from_table<Real>(acc, ia, ib);
-    } else {
-      Real u[4], v[4];
-      acc.get(ia, u);
-      acc.get(ib, v);
-      m2 = pair_mass2(u, v);
-    }
+    const Real m2 = acc.pair(ia, ib);
     if (f.kind != HPSP_F_MASS) return (double)m2;
     // Vector4R::mass: 0 unless the square is positive
     if constexpr (sizeof(Real) == 4)
@@ -898,52 +929,35 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
     return chi;
   }
   Real Ar = 0, Ai = 0;
-  Real tab[pair_table_size<Acc>::value];
-  if constexpr (has_pair_table<Acc>::value) acc.pair_table(tab);
   for (int k = 0; k < f.nterms; ++k) {
-    Real s = 0;
-    bool tabled = false;
-    if constexpr (has_pair_table<Acc>::value) {
-      if (f.a[k] != f.b[k]) {
-        s = pick1(tab, Acc::pair_index(f.a[k], f.b[k]));
-        tabled = true;
-      }
-    }
-    if (!tabled) {
-      Real u[4], w[4];
-      acc.get(f.a[k], u);
-      acc.get(f.b[k], w);
-      s = pair_mass2(u, w);
-    }
-    const Real M = (Real)f.m[k], G = (Real)f.g[k];
-    const Real dr = M * M - s;
-    const Real di = -(M * G);
-    const Real den = dr * dr + di * di;
-    Real br, bi;
+    const Real s = acc.pair(f.a[k], f.b[k]);
     if constexpr (Exact) {
-      br = dr / den;
-      bi = -di / den;
+      const Real dr = f.m2[k] - s;
+      const Real den = dr * dr + f.mg2[k];
+      const Real br = dr / den;
+      const Real bi = f.mg[k] / den;
+      const Real tr = f.cr[k] * br - f.ci[k] * bi;
+      const Real ti = f.cr[k] * bi + f.ci[k] * br;
+      Ar += tr;
+      Ai += ti;
+    } else if constexpr (sizeof(Real) == 4) {
+      const float dr = f.m2f[k] - s;
+      const float inv = __builtin_amdgcn_rcpf(__builtin_fmaf(dr, dr, f.mg2f[k]));
+      Ar = __builtin_fmaf(__builtin_fmaf(f.crf[k], dr, -f.cigf[k]), inv, Ar);
+      Ai = __builtin_fmaf(__builtin_fmaf(f.cif[k], dr, f.crgf[k]), inv, Ai);
     } else {
-      Real inv;
-      if constexpr (sizeof(Real) == 4)
-        inv = __builtin_amdgcn_rcpf(den);
-      else
-        inv = rcp_fast(den);
-      br = dr * inv;
-      bi = -di * inv;
+      const double dr = f.m2[k] - s;
+      const double inv = rcp_fast(__builtin_fma(dr, dr, f.mg2[k]));
+      Ar = __builtin_fma(__builtin_fma(f.cr[k], dr, -f.cig[k]), inv, Ar);
+      Ai = __builtin_fma(__builtin_fma(f.ci[k], dr, f.crg[k]), inv, Ai);
     }
-    const Real cr = (Real)f.cr[k], ci = (Real)f.ci[k];
-    const Real tr = cr * br - ci * bi;
-    const Real ti = cr * bi + ci * br;
-    Ar += tr;
-    Ai += ti;
   }
   return (double)(Ar * Ar + Ai * Ai);
 }
 
 template <typename Real, bool Exact = true, int P>
 __device__ __forceinline__ double functor_eval(const FunctorK& f, const Real (&p)[P][4]) {
-  return functor_eval_acc<Real, Exact>(f, RegAcc<Real, P>{p});
+  return functor_eval_acc<Real, Exact>(f, RegAcc<Real, P>(p, wants_pairs(f)));
 }
 
 // ---------------------------------------------------------------------------
@@ -987,8 +1001,8 @@ __device__ __forceinline__ void stats_push(Stats& s, double f, double wt) {
   const double w = s.w + wt;
   const double delta = f - s.mean;
   const double r = wt * rcp_fast(w);
-  const double mean = s.mean + delta * r;
-  s.m2 = s.m2 + wt * delta * (f - mean);
+  const double mean = __builtin_fma(delta, r, s.mean);
+  s.m2 = __builtin_fma(wt * delta, f - mean, s.m2);
   s.mean = mean;
   s.w = w;
 }

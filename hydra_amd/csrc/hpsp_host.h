@@ -60,7 +60,8 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
   for (int i = 0; i < d->n; ++i) {
     sum += d->masses[i];
     k.msum[i] = sum;
-    k.msq[i] = d->masses[i] * d->masses[i];
+    const double sq = d->masses[i] * d->masses[i];
+    k.msq[i] = sq < 0x1p-1000 ? 0x1p-1000 : sq;
     plain = plain && d->masses[i] > 0.0;
   }
   k.mas0 = 0.0 * d->ecm + k.msum[0];
@@ -135,10 +136,20 @@ inline int make_functork(const hpsp_functor* f, int nvec, FunctorK* out,
     for (int k = 0; k < f->nterms; ++k) {
       if (f->a[k] < 0 || f->a[k] >= nvec || f->b[k] < 0 || f->b[k] >= nvec)
         return HPSP_ERR_INVALID_ARGUMENT;
-      out->m[k] = f->m[k];
-      out->g[k] = f->g[k];
+      const double g = f->m[k] * f->g[k];
+      out->m2[k] = f->m[k] * f->m[k];
+      out->mg[k] = g;
+      out->mg2[k] = g * g;
       out->cr[k] = f->cr[k];
       out->ci[k] = f->ci[k];
+      out->cig[k] = f->ci[k] * g;
+      out->crg[k] = f->cr[k] * g;
+      out->m2f[k] = (float)out->m2[k];
+      out->mg2f[k] = (float)out->mg2[k];
+      out->crf[k] = (float)f->cr[k];
+      out->cif[k] = (float)f->ci[k];
+      out->cigf[k] = (float)out->cig[k];
+      out->crgf[k] = (float)out->crg[k];
       out->a[k] = f->a[k];
       out->b[k] = f->b[k];
     }

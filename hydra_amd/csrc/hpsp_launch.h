@@ -58,6 +58,7 @@ using AvgArgs = AvgArgsT<FunctorK>;
 struct DescSet {
   FunctorK f[HPSP_MAX_EVAL_FUNCTORS];
   int nf;
+  int pairs;  // some functor takes pair masses
 };
 
 // Evaluate arguments; FS is the set of functors whose values are written.
@@ -101,6 +102,12 @@ struct MemAcc {
     const uint64_t ld = p.ld[i];
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = c[(uint64_t)q * ld];
+  }
+  __device__ __forceinline__ double pair(int a, int b) const {
+    double u[4], v[4];
+    get(a, u);
+    get(b, v);
+    return pair_mass2(u, v);
   }
   __device__ __forceinline__ void sum(int first, int last, double (&Pv)[4]) const {
 #pragma clang fp contract(off)
