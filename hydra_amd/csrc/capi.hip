@@ -700,16 +700,28 @@ static ChainK make_chaink(const hpsp_decay* d, double scale2) {
   ck.ks_fixed = (2.0 * K + 4.0) * ck.ks_unit;
   ck.ic2_0 = 1.0 / (d->masses[0] * d->masses[0]);
   ck.C = d->max_weight * d->max_weight * (ck.rmax * ck.rmax) * ldexp(1.0, -2 * (d->n - 1));
-  // the squared test needs q >= 0: max and maxw positive
-  ck.fast_ok = ck.rmax_ok && d->max_weight > 0.0 && ck.C >= 0x1p-900 && ck.C <= 0x1p+900;
-  ck.A3 = 0.0;
-  ck.C3 = 0.0;
+  // the squared test needs q >= 0: max and maxw positive.  The 3-body chain,
+  // whose kernel does not look at q^2's range, takes masses whose products of
+  // eight (and d's no closer to zero than B < 2^-10 leaves them) are normal
+  double sum = 0.0;
+  bool ok = true;
+  for (int i = 0; i < d->n; ++i) {
+    sum += d->masses[i];
+    ok = ok && d->masses[i] >= 0x1p-100;
+  }
+  ok = d->n != 3 || (ok && d->ecm >= 0.0 && d->ecm + sum <= 0x1p+100);
+  ck.fast_ok = ok && ck.rmax_ok && d->max_weight > 0.0 && ck.C >= 0x1p-900 && ck.C <= 0x1p+900;
+  ck.C *= 0x1p64;
+  ck.C3 = ck.A2 = ck.sp2 = ck.sm2 = 0.0;
+  ck.ecm32 = d->ecm * 0x1p-32;
   if (d->n == 3) {
     // invMas[2] as the chain forms it: 1 * ecm + ((0 + m0) + m1 + m2)
-    double sum = 0.0;
-    for (int i = 0; i < 3; ++i) sum += d->masses[i];
-    ck.A3 = 1.0 * d->ecm + sum;
-    ck.C3 = ck.C / (ck.A3 * ck.A3);
+    const double A = 1.0 * d->ecm + sum;
+    const double sp = d->masses[1] + d->masses[0], sm = d->masses[1] - d->masses[0];
+    ck.A2 = A * A;
+    ck.sp2 = sp * sp;
+    ck.sm2 = sm * sm;
+    ck.C3 = ck.C / ck.A2;
   }
   return ck;
 }

@@ -12,21 +12,15 @@
 
 namespace hpsp {
 
-// pdk in FP64 with the reference's subtraction order (so the a - b - c
-// cancellation near threshold is the FP64 one) and a one-ulp square root and
-// reciprocal instead of correctly rounded ones.
-__device__ __forceinline__ double pdk_fast(double a, double b, double c) {
-#pragma clang fp contract(off)
-  const double x = (a - b - c) * (a + b + c) * (a - b + c) * (a + b - c);
-  return sqrt_fast(x) * rcp_fast(2 * a);
-}
-
 // FP64 weight chain of DecayMother::process (DecayMother.h:170-212):
 // sorted uniforms, invMas, pdk and the weight product in the reference's
-// order; the momenta pd are handed on in FP32.
+// order (so the a - b - c cancellation near threshold is the FP64 one), pdk
+// with a one-ulp square root and reciprocal instead of correctly rounded ones.
+// The momenta pd and invMas[1 .. N-2], which the boosts take, are handed on in
+// FP32.
 template <int N, int ENGINE, typename WordFn>
 __device__ __forceinline__ double weight_chain(const DecayK& d, const WordFn& word,
-                                               double (&invMas)[N], float (&pd)[N - 1]) {
+                                               float (&pd)[N - 1], float (&mas)[N - 1]) {
 #pragma clang fp contract(off)
   double rno[N];
   rno[0] = 0.0;
@@ -40,18 +34,17 @@ __device__ __forceinline__ double weight_chain(const DecayK& d, const WordFn& wo
 #pragma unroll
     for (int k = 0; k < N - 2; ++k) rno[k + 1] = to_unit<ENGINE>(v[k]);
   }
-  double sum = 0.0;
-#pragma unroll
-  for (int n = 0; n < N; ++n) {
-    sum += d.m[n];
-    invMas[n] = rno[n] * d.ecm + sum;
-  }
   double wt = d.maxw;
+  double c = d.mas0;
 #pragma unroll
   for (int n = 0; n < N - 1; ++n) {
-    const double q = pdk_fast(invMas[n + 1], invMas[n], d.m[n + 1]);
+    const double a = n < N - 2 ? rno[n + 1] * d.ecm + d.msum[n + 1] : d.masN;
+    const double r = n < N - 2 ? rcp_fast(a) : d.rmasN;
+    const double q = sqrt_fast(pdk_radicand(a, c, d.m[n + 1])) * (0.5 * r);
     wt *= q;
     pd[n] = (float)q;
+    if (n + 1 < N - 1) mas[n + 1] = (float)a;
+    c = a;
   }
   return wt;
 }

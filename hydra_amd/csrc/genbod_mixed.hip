@@ -45,20 +45,18 @@ template <int N, int ENGINE, typename WordFn>
 __device__ __forceinline__ double genbod_mixed(const DecayK& d, const WordFn& word,
                                                float (&p)[N][4]) {
 #pragma clang fp contract(off)
-  float pd[N - 1];
-  double invMas[N];
-  const double wt = weight_chain<N, ENGINE>(d, word, invMas, pd);
+  float pd[N - 1], mas[N - 1];
+  const double wt = weight_chain<N, ENGINE>(d, word, pd, mas);
 
-  const float m0 = (float)d.m[0];
-  p[0][0] = __builtin_amdgcn_sqrtf(__builtin_fmaf(pd[0], pd[0], m0 * m0));
+  p[0][0] = __builtin_amdgcn_sqrtf(__builtin_fmaf(pd[0], pd[0], d.msqf[0]));
   p[0][1] = 0.0f;
   p[0][2] = pd[0];
   p[0][3] = 0.0f;
 
+  [[maybe_unused]] float y0 = 0.0f, gy0 = 0.0f;  // step 1: daughter 0's terms of py
 #pragma unroll
   for (int i = 1; i < N; ++i) {
-    const float mi = (float)d.m[i];
-    p[i][0] = __builtin_amdgcn_sqrtf(__builtin_fmaf(pd[i - 1], pd[i - 1], mi * mi));
+    p[i][0] = __builtin_amdgcn_sqrtf(__builtin_fmaf(pd[i - 1], pd[i - 1], d.msqf[i]));
     p[i][1] = 0.0f;
     p[i][2] = -pd[i - 1];
     p[i][3] = 0.0f;
@@ -73,7 +71,11 @@ __device__ __forceinline__ double genbod_mixed(const DecayK& d, const WordFn& wo
 #pragma unroll
     for (int j = 0; j <= i; ++j) {
       const bool fresh = (j == i) || (i == 1);
-      if (fresh) {
+      if (i == 1 && j == 1) {  // back to back with daughter 0
+        p[1][1] = -p[0][1];
+        p[1][2] = -p[0][2];
+        p[1][3] = -p[0][3];
+      } else if (fresh) {
         const float y = p[j][2];
         const float t = -(sZ * y);
         p[j][2] = cZ * y;
@@ -94,7 +96,7 @@ __device__ __forceinline__ double genbod_mixed(const DecayK& d, const WordFn& wo
 
     // beta = pd/sqrt(pd^2 + M^2); gamma = 1/sqrt(1-beta^2);
     // (gamma-1)/beta^2 written as gamma^2/(gamma+1) (no cancellation).
-    const float M = (float)invMas[i];
+    const float M = mas[i];
     const float pi2 = pd[i] * pd[i];
     const float beta = pd[i] * __builtin_amdgcn_rsqf(__builtin_fmaf(M, M, pi2));
     const float b2 = beta * beta;
@@ -104,8 +106,18 @@ __device__ __forceinline__ double genbod_mixed(const DecayK& d, const WordFn& wo
 #pragma unroll
     for (int j = 0; j <= i; ++j) {
       const float e2 = p[j][0], py2 = p[j][2];
-      p[j][0] = __builtin_fmaf(gamma, e2, gby * py2);
-      p[j][2] = __builtin_fmaf(gby, e2, __builtin_fmaf(gb2yy, py2, py2));
+      if (i == 1 && j == 1) {  // py2 is minus daughter 0's
+        p[1][0] = __builtin_fmaf(gamma, e2, -gy0);
+        p[1][2] = __builtin_fmaf(gby, e2, -y0);
+      } else {
+        const float gy = gby * py2, y = __builtin_fmaf(gb2yy, py2, py2);
+        if (i == 1) {
+          gy0 = gy;
+          y0 = y;
+        }
+        p[j][0] = __builtin_fmaf(gamma, e2, gy);
+        p[j][2] = __builtin_fmaf(gby, e2, y);
+      }
     }
   }
   return wt;
@@ -311,9 +323,8 @@ __global__ __launch_bounds__(kBlock) void k_uw_flags_direct(const UnweightArgs a
     const bool rmax_ok = __builtin_fabs(rmax) >= 0x1p-1000 && __builtin_fabs(rmax) <= 0x1p+1000;
     Words words;
     words.next(win[wave], a.d, a.gen_first + g * kWave, lane, true);
-    double invMas[N];
-    float pd[N - 1];
-    const double w = weight_chain<N, ENGINE>(a.d, words, invMas, pd);
+    float pd[N - 1], mas[N - 1];
+    const double w = weight_chain<N, ENGINE>(a.d, words, pd, mas);
     const double u = (double)squares3(a.uw_key, a.jump + k) * 0x1p-32;
     ball = __ballot(k < a.n && ratio_above(w, a.maxv, rmax, rmax_ok, u));
     if (lane == 0) *(glob(a.flags) + g) = ball;

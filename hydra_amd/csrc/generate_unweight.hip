@@ -98,15 +98,18 @@ struct OneWord {
 };
 
 // The weight chain of one event (DecayMother.h:170-212: sorted uniforms,
-// invMas, the pdk terms), squared: returns q^2 = C prod_i d1 d2 / a^2 with
-// C = (maxw / max)^2 / 4^(N-1), and the bound B of the file comment; sure is
+// invMas, the pdk terms), squared: returns 2^64 q^2 = C prod_i d1 d2 / a^2 with
+// C = 2^64 (maxw / max)^2 / 4^(N-1) (2^64: the accept word is squared as the
+// integer it is), and the bound B of the file comment; sure is
 // false where a term of B is not defined (d1 or d2 not positive) or B is not
 // below 2^-10 (there the terms the first-order bound leaves out are below
 // 2^-10 of it, far inside the margin K leaves).  With c the previous step's
 // a (1/m0^2 at the first step), ka + kc is
 // (d1 (a^2 + c|b-c|) + d2 (a^2 + c(b+c))) / (d1 d2) + 1, and B needs
 // only estimates of 1/(d1 d2) and 1/a^2: it is a bound with a wide margin,
-// formed with fused multiply-adds.
+// formed with fused multiply-adds.  d1 = a^2 - (b + c)^2 from the rounded
+// square of a and a fused multiply-add is off by at most 2^-53 (a^2 + 2 (b + c)^2
+// + d1), so d1 d2 by less than 3 * 2^-53 ka of itself: inside the rounding terms.
 template <int N, int ENGINE, bool MOM = true, typename WordFn>
 __device__ __forceinline__ double chain_q2(const DecayK& d, const WordFn& word, double C,
                                            double ks_fixed, double ks_unit, double ic2_0,
@@ -140,12 +143,10 @@ __device__ __forceinline__ double chain_q2(const DecayK& d, const WordFn& word, 
     for (int k = 0; k < N - 2; ++k) rno[k + 1] = to_unit<ENGINE>(v[k]);
   }
   double invMas[N];
-  double sum = 0.0;
+  invMas[0] = d.mas0;
+  invMas[N - 1] = d.masN;
 #pragma unroll
-  for (int n = 0; n < N; ++n) {
-    sum += d.m[n];
-    invMas[n] = rno[n] * d.ecm + sum;
-  }
+  for (int n = 1; n < N - 1; ++n) invMas[n] = rno[n] * d.ecm + d.msum[n];
   double P = 1.0, A = 1.0;
   double Bs = 40.0 * N * eps;  // the roundings of the two chains
   double ic2 = ic2_0;
@@ -154,10 +155,10 @@ __device__ __forceinline__ double chain_q2(const DecayK& d, const WordFn& word, 
   for (int n = 0; n < N - 1; ++n) {
     const double a = invMas[n + 1], b = d.m[n + 1], c = invMas[n];
     const double spc = b + c, smc = b - c;
-    const double d1 = (a - spc) * (a + spc);
-    const double d2 = (a - smc) * (a + smc);
-    const double x = d1 * d2;
     const double a2 = a * a;
+    const double d1 = __builtin_fma(-spc, spc, a2);
+    const double d2 = __builtin_fma(-smc, smc, a2);
+    const double x = d1 * d2;
     P *= x;
     A *= a2;
     ok = ok && __builtin_fmin(d1, d2) > 0.0;
@@ -191,16 +192,12 @@ __device__ __forceinline__ double chain_q2(const DecayK& d, const WordFn& word, 
 // + 120 eps (stored as (X, Y) pairs); a bin where a denominator is not
 // positive gets infinity.
 __device__ __forceinline__ int bin3(uint32_t v) {
-  const uint32_t side = v >> 31;
-  const uint32_t t = side ? ~v : v;  // < 2^31
-  int idx;
-  if (t < 8) {
-    idx = (int)t;
-  } else {
-    const int e = 31 - __builtin_clz(t);  // 3 .. 30
-    idx = (e - 2) * 8 + (int)((t >> (e - 3)) & 7u);
-  }
-  return (int)side * kBin3Side + idx;
+  const uint32_t side = (uint32_t)((int32_t)v >> 31);  // all ones in the upper half
+  const uint32_t t = v ^ side;                         // < 2^31
+  // exponent and 3 leading bits of t, from its (exact) double
+  const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, (double)t) >> 32);
+  const uint32_t idx = t < 8 ? t : (hi >> 17) - (1023 + 2) * 8;
+  return (int)(idx + (side & (uint32_t)kBin3Side));
 }
 
 // count, where given, is cleared (the chain's list, filled by the next kernel).
@@ -260,8 +257,8 @@ __global__ __launch_bounds__(kBlock) void k_chain_table3(const DecayK d, double2
   XY[i] = make_double2(x * (1.0 + 0x1p-40), y * (1.0 + 0x1p-40));
 }
 
-// The 3-body chain: q^2 as chain_q2 forms it, with the step of the common A
-// folded into C3 = C / A^2, and B from the table.
+// The 3-body chain: 2^64 q^2 as chain_q2 forms it, with the step of the common
+// A folded into C3 = C / A^2, and B from the table.
 template <int ENGINE, bool MOM = true, typename WordFn>
 __device__ __forceinline__ double chain3_q2(const DecayK& d, const WordFn& word, const ChainK& ck,
                                             const double2* XY, double& B) {
@@ -269,14 +266,13 @@ __device__ __forceinline__ double chain3_q2(const DecayK& d, const WordFn& word,
   constexpr double eps = 0x1p-53;
   const uint64_t w0 = word(0);
   const uint32_t v = is_squares<ENGINE>() ? (uint32_t)w0 : (uint32_t)(w0 >> 32);
-  const double s01 = (0.0 + d.m[0]) + d.m[1];
-  const double A = ck.A3;
-  const double a0 = to_unit<ENGINE>(w0) * d.ecm + s01;
-  const double m0 = d.m[0], m1 = d.m[1], m2 = d.m[2];
-  const double spc0 = m1 + m0, smc0 = m1 - m0;
-  const double x0 = ((a0 - spc0) * (a0 + spc0)) * ((a0 - smc0) * (a0 + smc0));
-  const double spc1 = m2 + a0, smc1 = m2 - a0;
-  const double x1 = ((A - spc1) * (A + spc1)) * ((A - smc1) * (A + smc1));
+  // r ecm + (m0 + m1), the word's 2^-32 folded into ecm for 32-bit ones
+  const double a0 = is_squares<ENGINE>() ? (double)v * ck.ecm32 + d.msum[1]
+                                         : to_unit<ENGINE>(w0) * d.ecm + d.msum[1];
+  const double a2 = a0 * a0;
+  const double x0 = __builtin_fma(a0, a0, -ck.sp2) * __builtin_fma(a0, a0, -ck.sm2);
+  const double spc1 = d.m[2] + a0, smc1 = d.m[2] - a0;
+  const double x1 = __builtin_fma(-spc1, spc1, ck.A2) * __builtin_fma(-smc1, smc1, ck.A2);
   double ks = MOM ? ck.ks_fixed : 0.0;
   if constexpr (MOM && !is_squares<ENGINE>()) {
     double s2 = 1.0;
@@ -290,7 +286,7 @@ __device__ __forceinline__ double chain3_q2(const DecayK& d, const WordFn& word,
   }
   const double2 xy = XY[bin3(v)];
   B = __builtin_fma(ks, xy.x, xy.y);
-  return ck.C3 * (x0 * x1) * rcp_fast(a0 * a0);
+  return ck.C3 * (x0 * x1) * rcp_fast(a2);
 }
 
 }  // namespace
@@ -353,11 +349,11 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
       q2 = chain_q2<N, ENGINE>(a.d, words, ck.C, ck.ks_fixed, ck.ks_unit, ck.ic2_0, B, sure);
     }
     const bool live = k < a.n;
-    const double u = (double)squares3_y(a.uw_key, ykey) * 0x1p-32;  // ctr = jump + k
+    const double u = (double)squares3_y(a.uw_key, ykey);  // 2^32 u; ctr = jump + k
     const double u2 = u * u;
     const double e = B + 0x1p-47;
-    sure = sure && ck.fast_ok && q2 >= 0x1p-1000 && q2 <= 0x1p+1000 &&
-           __builtin_fabs(q2 - u2) > q2 * (e * (2.0 + e));
+    if constexpr (N != 3) sure = sure && q2 >= 0x1p-936;
+    sure = sure && ck.fast_ok && __builtin_fabs(q2 - u2) > q2 * (e * (2.0 + e));
     const uint64_t ball = __ballot(live && q2 > u2);
     const uint64_t doubt = __ballot(live && !sure);
     if (lane == 0) {
@@ -497,18 +493,17 @@ void k_uw_flags_mixed(const UnweightArgs a, const ChainK ck, const double* tab3)
       sure = sure && B < 0x1p-10;
     }
     const bool live = k < a.n;
-    const double u = (double)squares3_y(a.uw_key, ykey) * 0x1p-32;  // ctr = jump + k
+    const double u = (double)squares3_y(a.uw_key, ykey);  // 2^32 u; ctr = jump + k
     const double u2 = u * u;
     const double e = B + 0x1p-47;
-    sure = sure && ck.fast_ok && q2 >= 0x1p-1000 && q2 <= 0x1p+1000 &&
-           __builtin_fabs(q2 - u2) > q2 * (e * (2.0 + e));
+    if constexpr (N != 3) sure = sure && q2 >= 0x1p-936;
+    sure = sure && ck.fast_ok && __builtin_fabs(q2 - u2) > q2 * (e * (2.0 + e));
     bool acc = q2 > u2;
     if (live && !sure) {
       // the container's weight, as the mixed Generate forms it
-      double invMas[N];
-      float pd[N - 1];
-      const double w = weight_chain<N, ENGINE>(a.d, mw, invMas, pd);
-      acc = ratio_above(w, a.maxv, ck.rmax, ck.rmax_ok, u);
+      float pd[N - 1], mas[N - 1];
+      const double w = weight_chain<N, ENGINE>(a.d, mw, pd, mas);
+      acc = ratio_above(w, a.maxv, ck.rmax, ck.rmax_ok, u * 0x1p-32);
     }
     const uint64_t ball = __ballot(live && acc);
     if (lane == 0) *(glob(a.flags) + g) = ball;

@@ -35,6 +35,7 @@ struct DecayK {
   double m[HPSP_MAX_N];
   double msum[HPSP_MAX_N];  // ((0 + m0) + m1) + ... + m[n], the chain's running sum
   double msq[HPSP_MAX_N];   // m[n]^2, at least 2^-1000 (a sum with it is never 0)
+  float msqf[HPSP_MAX_N];   // m[n] rounded to FP32, squared in FP32 (mixed precision)
   double ecm;
   double maxw;
   double mas0, masN;  // invMas[0] = 0 ecm + msum[0] and invMas[N-1] = 1 ecm + msum[N-1]
@@ -57,8 +58,9 @@ struct FunctorK {
   double m2[HPSP_MAX_TERMS], mg[HPSP_MAX_TERMS], mg2[HPSP_MAX_TERMS];  // M^2, g, g^2
   double cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
   double cig[HPSP_MAX_TERMS], crg[HPSP_MAX_TERMS];  // ci g, cr g
-  float m2f[HPSP_MAX_TERMS], mg2f[HPSP_MAX_TERMS], crf[HPSP_MAX_TERMS], cif[HPSP_MAX_TERMS];
-  float cigf[HPSP_MAX_TERMS], crgf[HPSP_MAX_TERMS];
+  // the mixed form's, from M and G rounded to FP32
+  float m2f[HPSP_MAX_TERMS], mgf[HPSP_MAX_TERMS], mg2f[HPSP_MAX_TERMS];
+  float crf[HPSP_MAX_TERMS], cif[HPSP_MAX_TERMS];
   int a[HPSP_MAX_TERMS], b[HPSP_MAX_TERMS];
 };
 
@@ -942,9 +944,13 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
       Ai += ti;
     } else if constexpr (sizeof(Real) == 4) {
       const float dr = f.m2f[k] - s;
-      const float inv = __builtin_amdgcn_rcpf(__builtin_fmaf(dr, dr, f.mg2f[k]));
-      Ar = __builtin_fmaf(__builtin_fmaf(f.crf[k], dr, -f.cigf[k]), inv, Ar);
-      Ai = __builtin_fmaf(__builtin_fmaf(f.cif[k], dr, f.crgf[k]), inv, Ai);
+      const float inv = __builtin_amdgcn_rcpf(dr * dr + f.mg2f[k]);
+      const float br = dr * inv;
+      const float bi = f.mgf[k] * inv;
+      const float tr = f.crf[k] * br - f.cif[k] * bi;
+      const float ti = f.crf[k] * bi + f.cif[k] * br;
+      Ar += tr;
+      Ai += ti;
     } else {
       const double dr = f.m2[k] - s;
       const double inv = rcp_fast(__builtin_fma(dr, dr, f.mg2[k]));

@@ -62,6 +62,8 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
     k.msum[i] = sum;
     const double sq = d->masses[i] * d->masses[i];
     k.msq[i] = sq < 0x1p-1000 ? 0x1p-1000 : sq;
+    const float mf = (float)d->masses[i];
+    k.msqf[i] = mf * mf;
     plain = plain && d->masses[i] > 0.0;
   }
   k.mas0 = 0.0 * d->ecm + k.msum[0];
@@ -144,12 +146,12 @@ inline int make_functork(const hpsp_functor* f, int nvec, FunctorK* out,
       out->ci[k] = f->ci[k];
       out->cig[k] = f->ci[k] * g;
       out->crg[k] = f->cr[k] * g;
-      out->m2f[k] = (float)out->m2[k];
-      out->mg2f[k] = (float)out->mg2[k];
+      const float mf = (float)f->m[k], gf = mf * (float)f->g[k];
+      out->m2f[k] = mf * mf;
+      out->mgf[k] = gf;
+      out->mg2f[k] = gf * gf;
       out->crf[k] = (float)f->cr[k];
       out->cif[k] = (float)f->ci[k];
-      out->cigf[k] = (float)out->cig[k];
-      out->crgf[k] = (float)out->crg[k];
       out->a[k] = f->a[k];
       out->b[k] = f->b[k];
     }

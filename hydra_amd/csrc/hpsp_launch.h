@@ -255,13 +255,16 @@ int launch_uw_scans(const UnweightArgs& a, hipStream_t s);
 constexpr int kBin3Side = 8 + 28 * 8;  // bins per end of [0, 1]
 constexpr int kBin3 = 2 * kBin3Side;
 struct ChainK {
-  double C;         // (maxw / max)^2 / 4^(N-1)
-  double C3;        // C / A^2, A = invMas[2] (N = 3)
-  double A3;        // that A
+  double C;         // 2^64 (maxw / max)^2 / 4^(N-1)
+  // N = 3, with A = invMas[2]:
+  double C3;        // C / A^2
+  double A2;        // A^2
+  double sp2, sm2;  // (m1 + m0)^2, (m1 - m0)^2
+  double ecm32;     // ecm / 2^32
   double ks_unit;   // eps S^2, S^2 bounding E^2 + p^2 of any subsystem
   double ks_fixed;  // (2K + 4) eps S^2 with the squares engines' K = 2^17 N
   double ic2_0;     // 1 / m0^2
-  int fast_ok;      // max and maxw positive, 1/max and C in range
+  int fast_ok;      // max and maxw positive, 1/max and C (N = 3: the masses) in range
   double rmax;      // RN(1 / max) and whether it is normal (ratio_above)
   int rmax_ok;
 };
