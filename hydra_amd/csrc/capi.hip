@@ -178,6 +178,8 @@ static int generate_common(const hpsp_decay* d, uint64_t seed, uint64_t first, u
   a.evw = evw;
   a.mothers = mothers;
   a.mld = mld;
+  const uint64_t stored = (cols ? (out_f32 ? 16ull : 32ull) * d->n : 0) + (wt ? 8 : 0) + (evw ? 8 : 0);
+  a.xcd_ranges = prec == HPSP_FP64 && d->n <= 3 && n >= kXcdRangeBytes / stored;
   const int e = (prec == HPSP_FP64) ? launch_generate_f64(d->n, d->engine, a, as_stream(stream))
                                     : launch_generate_mixed(d->n, d->engine, a, as_stream(stream));
   return hip_status(e);

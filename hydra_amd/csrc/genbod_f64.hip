@@ -15,7 +15,8 @@ namespace hpsp {
 // their engine words through LDS (BlockEventWords: about one word or Random123
 // block evaluated per event).  Without a loop over groups nothing is kept in
 // scalar registers from one to the next and spilled, and blocks are dispatched
-// in order, so the chip's stores stay in a narrow moving window of the columns.
+// in order, so each XCD's stores stay in a narrow moving window of the columns
+// (xcd_block).
 // COLS = false is the weights pass of a deferred Generate (no momentum columns).
 // Against runs of up to 16 groups per wave (91 registers and 5 waves per SIMD
 // for 3 bodies, 142 and 3 for 10; now 56 and 8, 120 and 4): 1e6 3-body events
@@ -30,7 +31,7 @@ void k_generate_f64(const GenArgs a) {
   // wave index as a scalar so that column bases stay in SGPRs and every
   // store is (scalar base) + lane * 8
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint64_t kb = (uint64_t)blockIdx.x * kBlock;
+  const uint64_t kb = xcd_block(a.n, a.xcd_ranges) * kBlock;
   BlockEventWords<N, ENGINE> words;
   words.fill(sw, a.d, a.first + kb);
   const uint64_t k0 = kb + (uint64_t)(wave * kWave);

@@ -72,3 +72,20 @@ def test_runs_equal_single_groups(engine, N):
                 c, w, _ = generate(dec, 7, k, first=(first + b) % 2 ** 64, prec=prec)
                 assert torch.equal(cols[:, b:b + k], c)
                 assert torch.equal(wt[b:b + k], w)
+
+
+@pytest.mark.parametrize("N,momenta", [(2, True), (3, True), (3, False)])
+def test_blocks_in_xcd_ranges(N, momenta):
+    # at and above 4 GiB of output each XCD takes a contiguous range of blocks:
+    # every range's edge and the ragged end, against short calls at the same events
+    per = 32 * N + (0 if momenta else 8)
+    n = ((4 << 30) // per // 2048 + 1) * 2048 + 256 * 3 + 17  # blocks no multiple of 8
+    dec = make_decay(*decay(N))
+    cols, wt, _ = generate(dec, 3, n, want_wt=not momenta, want_evw=False)
+    per_xcd = (((n + 255) // 256 + 7) // 8) * 256
+    for e in [0] + [x * per_xcd for x in range(1, 8)] + [n - 300]:
+        lo, hi = max(0, e - 300), min(n, e + 300)
+        ref, wref, _ = generate(dec, 3, hi - lo, first=lo)
+        assert torch.equal(cols[:, lo:hi].cpu(), ref.cpu())
+        if wt is not None:
+            assert torch.equal(wt[lo:hi].cpu(), wref.cpu())
