@@ -121,22 +121,29 @@ void k_range_generate(const RangeArgs a) {
   }
 }
 
+// Threads of a fill's block: every block adds its bins to the contents in the
+// end, and those atomics, blocks times bins on few cache lines, not the
+// elements set the time of smaller fills (1e6 elements into 100 bins: 2048
+// blocks of 256 threads 53 us, 512 of them 31).
+constexpr int kRangeHistBlock = 512;
+
 template <int N>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
+__global__ __launch_bounds__(kRangeHistBlock)
+    __attribute__((amdgpu_waves_per_eu(N <= 6 ? waves_for(N) : 2, 8)))
 void k_range_hist(const RangeArgs a) {
   extern __shared__ double bins[];
-  __shared__ typename RangeWords<N>::Window win[kBlock / kWave];
+  __shared__ typename RangeWords<N>::Window win[kRangeHistBlock / kWave];
   const uint64_t nslots = a.h.nbins + 2;
   if (a.use_lds) {
-    for (uint64_t b = threadIdx.x; b < nslots; b += kBlock) bins[b] = 0.0;
+    for (uint64_t b = threadIdx.x; b < nslots; b += kRangeHistBlock) bins[b] = 0.0;
     __syncthreads();
   }
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
   const uint64_t nruns = (ngroups + a.run - 1) / a.run;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-  uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  const uint64_t nwaves = (uint64_t)gridDim.x * (kRangeHistBlock / kWave);
+  uint64_t run = (uint64_t)blockIdx.x * (kRangeHistBlock / kWave) + (uint64_t)wave;
   RangeWords<N> words;
   words.first(a.x_start, run * a.run * kWave, lane);
   for (; run < nruns; run += nwaves) {
@@ -167,7 +174,7 @@ void k_range_hist(const RangeArgs a) {
   }
   if (a.use_lds) {
     __syncthreads();
-    for (uint64_t b = threadIdx.x; b < nslots; b += kBlock) {
+    for (uint64_t b = threadIdx.x; b < nslots; b += kRangeHistBlock) {
       const double v = bins[b];
       if (v != 0.0) unsafeAtomicAdd(&a.contents[b], v);
     }
@@ -193,17 +200,20 @@ static void hist_one(RangeArgs a, hipStream_t s) {
   const uint64_t nslots = a.h.nbins + 2;
   a.use_lds = nslots <= a.lds_slots ? 1 : 0;
   const size_t lds = a.use_lds ? nslots * sizeof(double) : 0;
-  // several blocks per CU while the private bins are small; the per-block
-  // merge costs nslots atomics
-  const unsigned cap = (a.use_lds && lds > 32768) ? 512u : 2048u;
-  const unsigned g = grid_for(a.n, cap);
-  // one run per wave: nothing is stored on the way
+  // 8 waves per SIMD while the private bins are small, at least four groups per
+  // wave beyond one block per CU
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t nwaves = (uint64_t)g * (kBlock / kWave);
+  constexpr uint64_t kWaves = kRangeHistBlock / kWave;
+  const uint64_t cap = (a.use_lds && lds > 32768) ? 256 : 1024;
+  const uint64_t few = std::min<uint64_t>(256, (ngroups + kWaves - 1) / kWaves);
+  const unsigned g = (unsigned)std::max(
+      few, std::min<uint64_t>(cap, (ngroups + 4 * kWaves - 1) / (4 * kWaves)));
+  // one run per wave: nothing is stored on the way
+  const uint64_t nwaves = g * kWaves;
   const uint64_t per = (ngroups + nwaves - 1) / nwaves;
   a.run = (uint32_t)(per < 1 ? 1 : (per < (1u << 20) ? per : (1u << 20)));
   a.a_stride = minstd_pow(nwaves * a.run * kWave);
-  hipLaunchKernelGGL(k_range_hist<N>, dim3(g), dim3(kBlock), lds, s, a);
+  hipLaunchKernelGGL(k_range_hist<N>, dim3(g), dim3(kRangeHistBlock), lds, s, a);
 }
 
 template <int... I>
