@@ -16,7 +16,8 @@
 //   events   the events of a Decays container in SoA columns, each axis a
 //            functor of the event (the lazy `events | dalitz_calculator` of
 //            phsp_basic.inl:196-214, fused into the fill), weights from a
-//            column, the PhaseSpaceWeight of the event, or 1;
+//            column, the PhaseSpaceWeight of the event, or 1; the daughters
+//            are filled from as particles where the axes read few of them;
 //   particles  stored four-vectors given particle by particle (a melded
 //            decay chain, phsp_chain.inl:244), read only where a functor
 //            uses them; weights from a column or 1.
@@ -28,17 +29,52 @@
 
 namespace hpsp {
 
-template <int N>
+// s_waitcnt vmcnt(0) alone: export and LDS counters at their maxima.
+constexpr int kWaitLoads = 0xF70;
+
+// From here on an event with a PhaseSpaceWeight has its axes from memory, not from
+// the daughters in registers, where they read fewer four-vectors than there are
+// daughters (FEW): 4N momenta beside a functor's selections spilled, and what an
+// axis reads is read again for the weight from L2 (1e7 events, two pair masses: 10
+// bodies 795 -> 607 us; 9 bodies 541 -> 584, 8 bodies 480 -> 532).  Axes that read
+// more stay with the registers (10 bodies, three Breit-Wigner terms and a helicity
+// cosine: 794 us against 1057).
+constexpr int kMemAxes = 10;
+
+// Bound by the columns it reads: 3-body events with a weight column at 6.2 TB/s.
+// Without a PhaseSpaceWeight to form, a wave waits for each daughter's four
+// columns before it asks for the next: with all 13 columns asked for at once the
+// same bytes came slower (6e7 3-body events 1076 -> 1002 us, 4e7 4-body ones 884
+// -> 868), and more bytes in flight from a look ahead at the next event gained
+// nothing (1118 us).  From 9 bodies on the selections bound it, and the waits cost
+// (1e6 9-body events 65 -> 71 us).
+template <int N, bool FEW>
 __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
                                            double (&x)[HPSP_HIST_MAX_DIM], double& w) {
+  if constexpr (FEW) {
+    const MemAcc acc{a.parts, k};
+#pragma unroll
+    for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
+      x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true>(a.axes[d], acc) : 0.0;
+  }
   double p[N][4];
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) p[i][c] = a.cols[(uint64_t)(4 * i + c) * a.ld + k];
+    for (int c = 0; c < 4; ++c) {
+      if (N >= 3 && N <= 8 && c == 0 && i > 0 && a.weight_mode != HPSP_HIST_WEIGHT_PHSP) {
+        __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      p[i][c] = a.cols[(uint64_t)(4 * i + c) * a.ld + k];
+    }
+  if constexpr (!FEW) {
 #pragma unroll
-  for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
-    x[d] = (d < a.h.ndim) ? functor_eval<double>(a.axes[d], p) : 0.0;
+    for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d) {
+      const RegAcc<double, N, (N <= 8)> acc(p, wants_pairs(a.axes[d]));
+      x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true>(a.axes[d], acc) : 0.0;
+    }
+  }
   if (a.weight_mode == HPSP_HIST_WEIGHT_COLUMN)
     w = a.w[k];
   else if (a.weight_mode == HPSP_HIST_WEIGHT_PHSP)
@@ -48,7 +84,7 @@ __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
 }
 
 // N = 0: axis values from columns; N >= 2: from the events' momenta.
-template <int N>
+template <int N, bool FEW = false>
 __global__ __launch_bounds__(kHistBlock) void k_hist_fill(const HistArgs a) {
   extern __shared__ double bins[];
   const uint64_t nslots = a.h.nbins + 2;
@@ -72,7 +108,7 @@ __global__ __launch_bounds__(kHistBlock) void k_hist_fill(const HistArgs a) {
         x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true, true>(a.axes[d], acc) : 0.0;
       w = a.w ? a.w[k] : 1.0;
     } else {
-      event_axes<N>(a, k, x, w);
+      event_axes<N, FEW>(a, k, x, w);
     }
     const uint64_t key = hist_key(a.h, x);
     if (key == kDrop) continue;
@@ -101,14 +137,30 @@ void launch_zero(double* p, uint64_t n, hipStream_t s) {
                      dim3(256), 0, s, p, n);
 }
 
+// Four-vectors that an axis reads of an event.
+static int axis_reads(const FunctorK& f) {
+  switch (f.kind) {
+    case HPSP_F_ONE: return 0;
+    case HPSP_F_BW_SUM: return 2 * f.nterms;
+    case HPSP_F_COS_HELICITY: return f.b[1] + 2;
+    default: return 2;
+  }
+}
+
 template <int N>
-static void hist_one(const HistArgs& a, unsigned grid, size_t lds, hipStream_t s) {
+static void hist_one(const HistArgs& a, unsigned grid, size_t lds, bool few, hipStream_t s) {
+  if constexpr (N >= kMemAxes) {
+    if (few) {
+      hipLaunchKernelGGL((k_hist_fill<N, true>), dim3(grid), dim3(kHistBlock), lds, s, a);
+      return;
+    }
+  }
   hipLaunchKernelGGL(k_hist_fill<N>, dim3(grid), dim3(kHistBlock), lds, s, a);
 }
 
 template <int... I>
 static constexpr auto hist_table(std::integer_sequence<int, I...>) {
-  return std::array<void (*)(const HistArgs&, unsigned, size_t, hipStream_t), sizeof...(I)>{
+  return std::array<void (*)(const HistArgs&, unsigned, size_t, bool, hipStream_t), sizeof...(I)>{
       &hist_one<(I == 0 ? 0 : I + 1)>...};
 }
 // index 0: columns; index N - 1 (N = 2..HPSP_MAX_N): events of N daughters
@@ -119,17 +171,38 @@ int launch_histogram_fill(int N, const HistArgs& in, hipStream_t s) {
   const uint64_t nslots = a.h.nbins + 2;
   launch_zero(a.contents, nslots, s);
   if (a.n == 0) return (int)hipGetLastError();
+  bool few = false;
+  if (N > 0) {  // the events' daughters as particles
+    a.parts.n = N;
+    for (int i = 0; i < N; ++i) {
+      a.parts.cols[i] = a.cols + (uint64_t)(4 * i) * a.ld;
+      a.parts.ld[i] = a.ld;
+    }
+    // Fewer four-vectors than daughters, and no weight that needs them all: the
+    // particles' kernel reads those alone (1e7 events into two pair masses: 5
+    // bodies 295 -> 233 us, 10 bodies 728 -> 230).  4 bodies read their four in
+    // registers (4e7 events 869 us against 908), and so do axes that together
+    // read a daughter twice.
+    int reads = 0;
+    for (int d = 0; d < a.h.ndim; ++d) reads += axis_reads(a.axes[d]);
+    few = reads < N;
+    if (N >= 5 && few && a.weight_mode != HPSP_HIST_WEIGHT_PHSP) {
+      if (a.weight_mode != HPSP_HIST_WEIGHT_COLUMN) a.w = nullptr;
+      N = -1;
+    }
+  }
   a.use_lds = nslots <= a.lds_slots ? 1 : 0;
   const size_t lds = a.use_lds ? nslots * sizeof(double) : 0;
   // one block per CU: each block's bins are added to the contents in the end, on
   // few cache lines where bins are few (400 bins, 2e6 3-body events: 1024 blocks
   // 54 us, 512 49, 256 43, 128 61; 10^4 bins: 512 66, 256 51, 128 65)
   const uint64_t want = (a.n + kHistBlock - 1) / kHistBlock;
-  const unsigned grid = (unsigned)std::min<uint64_t>(want, 256);
+  const uint64_t cap = a.use_lds ? 256 : 1024;
+  const unsigned grid = (unsigned)std::min<uint64_t>(want, cap);
   if (N < 0)
-    hist_one<-1>(a, grid, lds, s);
+    hist_one<-1>(a, grid, lds, few, s);
   else
-    kHist[N == 0 ? 0 : N - 1](a, grid, lds, s);
+    kHist[N == 0 ? 0 : N - 1](a, grid, lds, few, s);
   return (int)hipGetLastError();
 }
 

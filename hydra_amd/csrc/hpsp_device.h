@@ -755,7 +755,7 @@ __device__ __forceinline__ Real pair_mass2(const Real (&u)[4], const Real (&w)[4
 // branches to each pair's own code cost more than the selects: AverageOn of the
 // 3-body Dalitz model over 2^24 events 217 us against 208, Evaluate of 10^7 153
 // against 145.)
-template <typename Real, int P>
+template <typename Real, int P, bool AllSum = true>
 struct RegAcc {
   const Real (&p)[P][4];
   static constexpr bool kTable = P >= 2 && P <= 4;
@@ -791,10 +791,11 @@ struct RegAcc {
   }
   // p[first] + ... + p[last - 1], left to right, through the unrolled array;
   // all of them, or all but the first (the daughters beside their mother),
-  // without the selects
+  // without the selects (AllSum; its registers spill beside 9 and more
+  // daughters in a kernel of 128)
   __device__ __forceinline__ void sum(int first, int last, Real (&Pv)[4]) const {
 #pragma clang fp contract(off)
-    if (last == P && first <= 1) {
+    if (AllSum && last == P && first <= 1) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) Pv[c] = p[1][c];
       if (first == 0) {

@@ -124,6 +124,42 @@ def test_fill_events_vs_oracle(oracle, N):
         check_weighted(got, exp, exp)
 
 
+@pytest.mark.parametrize("N", [4, 5, 6, 8, 9, 10, 12])
+def test_event_axes_equal_their_columns(N):
+    # axes that read fewer daughters than there are, as many and more, from
+    # registers or from memory: the counts of the axis values as columns
+    m = [0.2 + 0.1 * ((5 * i) % 7) for i in range(N)]
+    M = 1.8 * sum(m)
+    dec = make_decay(M, m)
+    n, ld = 30011, 30020
+    cols, _, evw = generate(dec, 17, n, ld=ld, want_wt=False)
+    bw = [(1.1, 0.2, 0.7, 0.3, 0, N - 1), (1.5, 0.3, 0.4, -0.2, 1, 2), (0.9, 0.1, 1.0, 0.0, 3, 1)]
+    pair = make_functor(capi.F_MASS2, (N - 1, 1))
+    sets = [([pair, make_functor(capi.F_MASS, (2, 3))], [[0, M * M], [0, M]]),
+            ([make_functor(capi.F_BW_SUM, bw)], [[0, 10]]),
+            ([make_functor(capi.F_COS_HELICITY, (0, 1)), pair], [[-1, 1], [0, M * M]])]
+    p = capi.Particles()
+    p.n = N
+    for i in range(N):
+        p.cols[i], p.ld[i] = cols.data_ptr() + 32 * ld * i, ld
+    for axes, lim in sets:
+        x = torch.empty((len(axes), n), dtype=torch.float64, device=DEV)
+        check(lib().hpsp_particles_evaluate(ctypes.byref(p), capi.functor_array(axes), len(axes), n,
+                                            ptr(x), n, stream_handle()), "evaluate")
+        grid, lo, hi = [60] * len(axes), [v[0] for v in lim], [v[1] for v in lim]
+        h = capi.make_histogram(grid, lo, hi)
+        ref = []
+        for w in (None, evw):
+            out = torch.empty(60 ** len(axes) + 2, dtype=torch.float64, device=DEV)
+            check(lib().hpsp_histogram_fill(ctypes.byref(h), ptr(x), n, n, ptr(w), ptr(out),
+                                            stream_handle()), "fill")
+            ref.append(out.cpu().numpy())
+        got = fill_events(grid, lo, hi, dec, axes, cols, capi.HIST_WEIGHT_ONE, n=n)
+        assert np.array_equal(got, ref[0]) and got.sum() == n
+        for mode, wc in ((capi.HIST_WEIGHT_COLUMN, evw), (capi.HIST_WEIGHT_PHSP, None)):
+            check_weighted(fill_events(grid, lo, hi, dec, axes, cols, mode, wc, n=n), ref[1], ref[1])
+
+
 def test_fill_repeats_and_empty():
     """A fill overwrites the contents; n = 0 leaves them zero."""
     x = np.linspace(0, 1, 1001)[None, :]
