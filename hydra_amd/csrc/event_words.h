@@ -5,8 +5,8 @@
 // e + 3N .. e + 3N + W - 1, with the Random123 ones the words of the blocks
 // (2 or 4 words) of counters e + 3N + 1 .. e + 3N + NB, NB = ceil(W / A).  So
 // neighbouring events read all but one of the same words or blocks.  A wave
-// (EventWords, in the kernels that take runs of groups of 64 events) or a
-// block (BlockEventWords, in the regenerating scatters) evaluates each word or
+// (EventWords, in AverageOn and the flags kernels) or a block
+// (BlockEventWords, in Generate and the regenerating scatters) evaluates each word or
 // block once and puts it into LDS; the event in lane l reads word j at slot
 // l + j / A, an immediate offset from one address.  The kernels that read them
 // are bound by their vector instructions: evaluating every block in every lane

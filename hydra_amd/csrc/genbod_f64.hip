@@ -180,7 +180,7 @@ void k_uw_regen(const UnweightArgs a) {
 // PhaseSpaceWeight formed and the reference's test applied (FlagDaugthers,
 // Decays.inl:75-89), one group of 64 per wave.  In place of the weight chain's
 // four launches (its list's counter, table, flags, doubtful events): the 3-body
-// call of 1e5 events 25 us -> 12, the 10-body one of 4e4 42 -> 25.
+// call of 1e5 events 25 us -> 12, the 10-body one of 4e4 42 -> 17.5.
 template <int N, int ENGINE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves_for(N), 8)))
 void k_uw_flags_exact(const UnweightArgs a) {
@@ -251,14 +251,18 @@ __device__ __forceinline__ void load_event(const double* cols, uint64_t ld, uint
     for (int q = 0; q < 4; ++q) p[i][q] = __builtin_nontemporal_load(cols + (uint64_t)(4 * i + q) * ld + k);
 }
 
-// PhaseSpaceWeight (and PhaseSpaceReweight) of stored events.
+// PhaseSpaceWeight (and PhaseSpaceReweight) of stored events.  Bound by the
+// columns: event_weight_any, whose branches keep the loads and square roots of a
+// few daughters in flight, holds fewer registers than the branch-free form (12
+// bodies 160 against 190, 3 waves per SIMD against 2: 5e6 events 365 us against
+// 447, with a Breit-Wigner sum 386 against 530; 3 bodies the same).
 template <int N>
 __global__ __launch_bounds__(kBlock) void k_event_weight(const WeightArgs a) {
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < a.n; k += stride) {
     double p[N][4];
     load_event<N>(a.cols, a.ld, k, p);
-    double w = event_weight_f64<N>(p, a.d.m, a.d.maxw);
+    double w = event_weight_any<N>(p, a.d.m, a.d.maxw);
     if (a.use_f) w = w * functor_eval<double>(a.f, p);
     a.w_out[k] = w;
   }
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void k_max_weight(const WeightArgs a, doubl
   for (uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < a.n; k += stride) {
     double p[N][4];
     load_event<N>(a.cols, a.ld, k, p);
-    double w = event_weight_f64<N>(p, a.d.m, a.d.maxw);
+    double w = event_weight_any<N>(p, a.d.m, a.d.maxw);
     if (a.use_f) w = w * functor_eval<double>(a.f, p);
     if (a.w_out) a.w_out[k] = w;
     mx = (mx < w) ? w : mx;

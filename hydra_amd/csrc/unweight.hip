@@ -98,8 +98,8 @@ __global__ __launch_bounds__(kBlock) void k_uw_flags(const UnweightArgs a) {
 // kScanThreads tiles, sums the counts before them itself (four per load) and
 // scans its own.  At 2^27 events (128 runs) its longest block reads 0.5 MB, a
 // few us, where three kernels (below) take three launches, 14 us at 10^7 events;
-// beyond kScanOneRuns runs the reads would grow with the
-// square and the three kernels take over.
+// beyond kScanOneRuns runs the reads would grow with the square and the three
+// kernels take over.
 constexpr int kScanThreads = 1024;
 constexpr uint64_t kScanOneRuns = 256;
 __global__ __launch_bounds__(kScanThreads) void k_uw_scan(const uint32_t* tile_count,
