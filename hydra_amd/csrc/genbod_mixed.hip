@@ -355,7 +355,8 @@ void k_uw_regen_mixed(const UnweightArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t g0 = blk * kWavesPerBlock;
   __shared__ TileSums sums;
-  const TilePlace at = tile_place<HERE>(a, g0 / (kUwTile / kWave), sums);
+  const TilePlace at = tile_place<HERE>(a.n, a.scan_here, a.tile_count, a.tile_off, a.n_acc,
+                                        g0 / (kUwTile / kWave), sums);
   const BlockPart bp = block_part(a, g0, wave, ngroups, at.off);
   const uint64_t goff = bp.goff;
   const uint32_t acc_wave = bp.acc_wave, a_blk = bp.a_blk;

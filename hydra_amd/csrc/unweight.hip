@@ -244,7 +244,8 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter_staged(const UnweightArgs
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t g0 = blk * kWavesPerBlock;
   __shared__ TileSums sums;
-  const TilePlace at = tile_place<HERE>(a, g0 / (kUwTile / kWave), sums);
+  const TilePlace at = tile_place<HERE>(a.n, a.scan_here, a.tile_count, a.tile_off, a.n_acc,
+                                        g0 / (kUwTile / kWave), sums);
   const BlockPart bp = block_part(a, g0, wave, ngroups, at.off);
   const uint64_t goff = bp.goff;
   const uint32_t acc_wave = bp.acc_wave, a_blk = bp.a_blk;
@@ -302,7 +303,8 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter(const UnweightArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = kUwTile / kWave;
   __shared__ TileSums sums;
-  const TilePlace at = tile_place<HERE>(a, tile, sums);
+  const TilePlace at = tile_place<HERE>(a.n, a.scan_here, a.tile_count, a.tile_off, a.n_acc,
+                                        tile, sums);
   const uint64_t tile_base = at.off;
   const uint64_t nacc = at.nacc;
   // group offsets inside the tile: lanes 0..15 of wave 0 each load one flag
@@ -422,7 +424,8 @@ __global__ __launch_bounds__(kBlock) void k_uw_scatter_cols(const UnweightArgs a
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = kUwTile / kWave;
   __shared__ TileSums sums;
-  const TilePlace at = tile_place<HERE>(a, tile, sums);
+  const TilePlace at = tile_place<HERE>(a.n, a.scan_here, a.tile_count, a.tile_off, a.n_acc,
+                                        tile, sums);
   const uint64_t tile_base = at.off;
   const uint64_t nacc = at.nacc;
   if (wave == 0) {

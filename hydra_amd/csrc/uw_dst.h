@@ -10,10 +10,14 @@ namespace hpsp {
 constexpr int kItems = kUwTile / kBlock;  // 4 groups of 64 events per wave
 
 // Accepted events before a tile and in all: from the scan's arrays, or summed
-// from the counts here (a.scan_here: at most four tiles per thread; a template
+// from the counts here (scan_here: at most four tiles per thread; a template
 // argument, because the summing code cost the large regenerating scatter 2% even
-// unused).  Every
-// thread of a block calls it, for one tile; block 0 then writes the total.
+// unused).  Every thread of a block calls it, for one tile; block 0 then writes
+// the total.  The arguments come by value: taking the kernel's arguments by
+// reference moved the lane's index into another block of the program, and
+// k_uw_scatter then formed every load's address in vector registers and waited
+// for a batch's loads before its first stores (4e6 12-body events with a weight
+// column 718 -> 752 us).
 struct TilePlace {
   uint64_t off, nacc;
 };
@@ -21,23 +25,25 @@ struct TileSums {  // __shared__
   uint32_t before[kBlock / kWave], all[kBlock / kWave];
 };
 template <bool HERE>
-__device__ __forceinline__ TilePlace tile_place(const UnweightArgs& a, uint64_t tile,
-                                                TileSums& sh) {
-  if constexpr (!HERE) return {a.tile_off[tile], *a.n_acc};
+__device__ __forceinline__ TilePlace tile_place(uint64_t n, int scan_here,
+                                                const uint32_t* tile_count,
+                                                const uint64_t* tile_off, uint64_t* n_acc,
+                                                uint64_t tile, TileSums& sh) {
+  if constexpr (!HERE) return {tile_off[tile], *n_acc};
   const uint32_t t = threadIdx.x;
-  const uint64_t ntiles = (a.n + kUwTile - 1) / kUwTile;
+  const uint64_t ntiles = (n + kUwTile - 1) / kUwTile;
   uint32_t all = 0, before = 0;
   for (uint32_t i = t; i < ntiles; i += kBlock) {
-    uint32_t n;
-    if (a.scan_here == kScanBlocks) {
-      const uint64_t c = a.tile_off[i];  // four 16-bit counts, 256 at most each
+    uint32_t count;
+    if (scan_here == kScanBlocks) {
+      const uint64_t c = tile_off[i];  // four 16-bit counts, 256 at most each
       const uint32_t pairs = (uint32_t)c + (uint32_t)(c >> 32);
-      n = (pairs & 0xFFFFu) + (pairs >> 16);
+      count = (pairs & 0xFFFFu) + (pairs >> 16);
     } else {
-      n = a.tile_count[i];
+      count = tile_count[i];
     }
-    all += n;
-    before += i < tile ? n : 0u;
+    all += count;
+    before += i < tile ? count : 0u;
   }
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) {
@@ -52,7 +58,7 @@ __device__ __forceinline__ TilePlace tile_place(const UnweightArgs& a, uint64_t 
   static_assert(kBlock / kWave == 4, "four waves");
   const uint64_t off = sh.before[0] + sh.before[1] + sh.before[2] + sh.before[3];
   const uint64_t nacc = sh.all[0] + sh.all[1] + sh.all[2] + sh.all[3];
-  if (blockIdx.x == 0 && t == 0) *a.n_acc = nacc;
+  if (blockIdx.x == 0 && t == 0) *n_acc = nacc;
   return {off, nacc};
 }
 

@@ -1,0 +1,21 @@
+"""What the compiler made of kernels whose speed hangs on it: properties that a
+change elsewhere can take away without any wrong result."""
+import re
+
+import pytest
+
+import code_objects as co
+
+
+@pytest.mark.skipif(not co.have_objdump(), reason="llvm-objdump of ROCm")
+@pytest.mark.parametrize("N", [7, 9, 12])
+@pytest.mark.parametrize("here", [0, 1])
+def test_scatter_loads_from_scalar_bases(N, here):
+    """k_uw_scatter's columns: the base in scalar registers, one lane offset for
+    all of them (with addresses in vector registers the kernel's stores waited
+    for whole batches of loads)."""
+    (name,) = co.find(f"k_uw_scatterILi{N}ELb{here}E")
+    loads = [i for i in co.instructions(name) if i.startswith("global_load_dwordx2")]
+    scalar = [i for i in loads if re.search(r", s\[\d+:\d+\]", i)]
+    assert len(loads) >= 4 * N * 4  # every column of the four groups
+    assert len(scalar) >= 4 * N * 4
