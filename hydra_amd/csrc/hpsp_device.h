@@ -776,6 +776,7 @@ struct RegAcc {
     }
   }
   __device__ __forceinline__ void get(int i, Real (&v)[4]) const { pick4(p, i, v); }
+  __device__ __forceinline__ const RegAcc& pairs() const { return *this; }
   // (p[a] + p[b])^2
   __device__ __forceinline__ Real pair(int a, int b) const {
     if constexpr (kTable) {
@@ -851,8 +852,8 @@ __device__ __forceinline__ void unit3(Real (&v)[4]) {
   for (int c = 0; c < 4; ++c) v[c] *= inv;
 }
 
-// Functor value of one event; acc.get(i, v) yields four-vector i, acc.pair(a, b)
-// the pair's mass squared and acc.sum(first, last, P) the left-to-right sum of
+// Functor value of one event; acc.get(i, v) yields four-vector i,
+// acc.pairs().pair(a, b) the pair's mass squared and acc.sum(first, last, P) the left-to-right sum of
 // four-vectors [first, last).
 // The decay-plane angle (atan2 and two normalisations) is compiled only where
 // Plane is set, the kernels over stored particles: in the generation kernels
@@ -864,7 +865,7 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
   if (f.kind == HPSP_F_MASS2_01 || f.kind == HPSP_F_MASS2 || f.kind == HPSP_F_MASS) {
     const int ia = f.kind == HPSP_F_MASS2_01 ? 0 : f.a[0];
     const int ib = f.kind == HPSP_F_MASS2_01 ? 1 : f.b[0];
-    const Real m2 = acc.pair(ia, ib);
+    const Real m2 = acc.pairs().pair(ia, ib);
     if (f.kind != HPSP_F_MASS) return (double)m2;
     // Vector4R::mass: 0 unless the square is positive
     if constexpr (sizeof(Real) == 4)
@@ -932,8 +933,9 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
     return chi;
   }
   Real Ar = 0, Ai = 0;
+  const auto& pairs = acc.pairs();
   for (int k = 0; k < f.nterms; ++k) {
-    const Real s = acc.pair(f.a[k], f.b[k]);
+    const Real s = pairs.pair(f.a[k], f.b[k]);
     if constexpr (Exact) {
       const Real dr = f.m2[k] - s;
       const Real den = dr * dr + f.mg2[k];
@@ -965,6 +967,22 @@ __device__ __forceinline__ double functor_eval_acc(const FunctorK& f, const Acc&
 template <typename Real, bool Exact = true, int P>
 __device__ __forceinline__ double functor_eval(const FunctorK& f, const Real (&p)[P][4]) {
   return functor_eval_acc<Real, Exact>(f, RegAcc<Real, P>(p, wants_pairs(f)));
+}
+
+// The same of a stored event, in the kernels that its columns bound, where
+// registers are waves: the pair masses are formed where a functor takes them
+// (LateAcc; before the branch on its kind they were held beside the momenta: 4
+// bodies 85 registers against 75), and all daughters summed by the general loop (8
+// bodies 118 against 110).
+template <int P>
+struct LateAcc : RegAcc<double, P, false> {
+  using Reg = RegAcc<double, P, false>;
+  __device__ __forceinline__ LateAcc(const double (&p)[P][4]) : Reg(p, false) {}
+  __device__ __forceinline__ Reg pairs() const { return Reg(this->p, true); }
+};
+template <int P>
+__device__ __forceinline__ double functor_stored(const FunctorK& f, const double (&p)[P][4]) {
+  return functor_eval_acc<double, true>(f, LateAcc<P>(p));
 }
 
 // ---------------------------------------------------------------------------

@@ -104,6 +104,7 @@ struct MemAcc {
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = c[(uint64_t)q * ld];
   }
+  __device__ __forceinline__ const MemAcc& pairs() const { return *this; }
   __device__ __forceinline__ double pair(int a, int b) const {
     double u[4], v[4];
     get(a, u);

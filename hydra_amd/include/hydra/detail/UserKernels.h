@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kBlock) void k_user_values(const UserValuesArgs<FS>
     for (int i = 0; i < N; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) p[i][q] = a.cols[(uint64_t)(4 * i + q) * a.ld + k];
-    const double w = a.with_weight ? event_weight_f64<N>(p, a.d.m, a.d.maxw) : 1.0;
+    const double w = a.with_weight ? event_weight_any<N>(p, a.d.m, a.d.maxw) : 1.0;
     eval_set_scaled(a.fs, p, w, [&](int j, double v) { a.out[(uint64_t)j * a.ldo + k] = v; });
   }
 }

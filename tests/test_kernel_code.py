@@ -19,3 +19,18 @@ def test_scatter_loads_from_scalar_bases(N, here):
     scalar = [i for i in loads if re.search(r", s\[\d+:\d+\]", i)]
     assert len(loads) >= 4 * N * 4  # every column of the four groups
     assert len(scalar) >= 4 * N * 4
+
+
+# Waves per SIMD of the kernels over stored events, which the columns bound, for
+# 2 .. 12 bodies.
+STORED = {
+    "k_event_weight": [8, 7, 6, 5, 5, 4, 4, 4, 3, 3, 3],
+    "k_max_weight": [8, 7, 6, 5, 5, 4, 4, 4, 3, 3, 3],
+}
+
+
+@pytest.mark.parametrize("kernel", STORED)
+def test_stored_events_waves(kernel):
+    for N, want in zip(range(2, 13), STORED[kernel]):
+        (k,) = co.find(f"{kernel}ILi{N}E").values()
+        assert co.waves(k) >= want, (kernel, N, k[".vgpr_count"])
