@@ -177,7 +177,7 @@ __device__ __forceinline__ double genbod_f64(const DecayK& d, const WordFn& word
 // (the result is compared within a tolerance, not bit for bit).  A user's
 // callable brings its own overload (found by argument-dependent lookup).
 template <int P>
-__device__ __forceinline__ double avg_value(const FunctorK& f, const double (&p)[P][4]) {
+__device__ __forceinline__ double avg_value(const FunctorFastK& f, const double (&p)[P][4]) {
   return functor_eval<double, false>(f, p);
 }
 
@@ -195,7 +195,7 @@ __device__ __forceinline__ double avg_value(const FunctorK& f, const double (&p)
 // staged values in the same order: the same partial, bit for bit.
 constexpr int avg_wide_waves(int N) { return N <= 6 ? 16 : 8; }  // 128 or 256 registers
 
-template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorK, int WAVES = kBlock / kWave>
+template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorFastK, int WAVES = kBlock / kWave>
 __global__ __launch_bounds__(WAVES * kWave)
     __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? waves_for(N) : WAVES / 4, 8)))
 void k_average_f64(const AvgArgsT<FK> a) {

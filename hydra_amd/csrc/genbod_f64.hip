@@ -329,7 +329,8 @@ static void gen_one(const GenArgs& a, hipStream_t s) {
 }
 
 template <int N, int E>
-static void avg_one(const AvgArgs& a, hipStream_t s) {
+static void avg_one(const AvgArgs& in, hipStream_t s) {
+  const AvgArgsT<FunctorFastK> a = with_functor(in, in.f.fast);
   constexpr int kWaves = avg_wide_waves(N);
   launch_avg(
       a.n, kWaves,
@@ -341,10 +342,10 @@ static void avg_one(const AvgArgs& a, hipStream_t s) {
       },
       [&](unsigned g, unsigned threads) {
         if (a.mothers)
-          hipLaunchKernelGGL((k_average_f64<N, E, true, FunctorK, kWaves>), dim3(g), dim3(threads),
-                             0, s, a);
+          hipLaunchKernelGGL((k_average_f64<N, E, true, FunctorFastK, kWaves>), dim3(g),
+                             dim3(threads), 0, s, a);
         else
-          hipLaunchKernelGGL((k_average_f64<N, E, false, FunctorK, kWaves>), dim3(g),
+          hipLaunchKernelGGL((k_average_f64<N, E, false, FunctorFastK, kWaves>), dim3(g),
                              dim3(threads), 0, s, a);
       });
 }

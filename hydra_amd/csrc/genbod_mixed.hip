@@ -221,7 +221,8 @@ struct ShiftedSums {
 constexpr int kAvgWideWaves = 16;
 
 template <int N, int ENGINE, bool MOTHERS, int WAVES = kBlock / kWave>
-__global__ __launch_bounds__(WAVES * kWave) void k_average_mixed(const AvgArgs a) {
+__global__ __launch_bounds__(WAVES * kWave)
+void k_average_mixed(const AvgArgsT<FunctorMixedK> a) {
   constexpr int kFold = kBlock / kWave;  // waves that fold
   constexpr bool kWide = WAVES > kFold;
   constexpr int kGroups = kAvgChunk / kWave;
@@ -431,7 +432,8 @@ static void gen_one(const GenArgs& a, hipStream_t s) {
 }
 
 template <int N, int E>
-static void avg_one(const AvgArgs& a, hipStream_t s) {
+static void avg_one(const AvgArgs& in, hipStream_t s) {
+  const AvgArgsT<FunctorMixedK> a = with_functor(in, in.f.mixed);
   launch_avg(
       a.n, kAvgWideWaves,
       [&](unsigned g) {

@@ -96,12 +96,40 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
   return k;
 }
 
+// The constants of Breit-Wigner term k.
+inline void set_term(FunctorK* out, int k, const hpsp_functor& f) {
+  const double g = f.m[k] * f.g[k];
+  out->m2[k] = f.m[k] * f.m[k];
+  out->mg[k] = g;
+  out->mg2[k] = g * g;
+  out->cr[k] = f.cr[k];
+  out->ci[k] = f.ci[k];
+}
+inline void set_term(FunctorFastK* out, int k, const hpsp_functor& f) {
+  const double g = f.m[k] * f.g[k];
+  out->m2[k] = f.m[k] * f.m[k];
+  out->mg2[k] = g * g;
+  out->cr[k] = f.cr[k];
+  out->ci[k] = f.ci[k];
+  out->cig[k] = f.ci[k] * g;
+  out->crg[k] = f.cr[k] * g;
+}
+inline void set_term(FunctorMixedK* out, int k, const hpsp_functor& f) {
+  const float m = (float)f.m[k], g = m * (float)f.g[k];
+  out->m2[k] = m * m;
+  out->mg[k] = g;
+  out->mg2[k] = g * g;
+  out->cr[k] = (float)f.cr[k];
+  out->ci[k] = (float)f.ci[k];
+}
+
 // nvec: four-vectors the functor sees; first_daughter: index of the first
 // decay product among them (0, or 1 when the mother comes first).
 // The decay-plane angle only where the kernels compile it (allow_plane: the
 // entry points over stored particles).
-inline int make_functork(const hpsp_functor* f, int nvec, FunctorK* out,
-                         int first_daughter = 0, bool allow_plane = false) {
+template <typename FK>
+inline int make_functork(const hpsp_functor* f, int nvec, FK* out, int first_daughter = 0,
+                         bool allow_plane = false) {
   memset(out, 0, sizeof(*out));
   if (!f) {
     out->kind = HPSP_F_ONE;
@@ -138,26 +166,19 @@ inline int make_functork(const hpsp_functor* f, int nvec, FunctorK* out,
     for (int k = 0; k < f->nterms; ++k) {
       if (f->a[k] < 0 || f->a[k] >= nvec || f->b[k] < 0 || f->b[k] >= nvec)
         return HPSP_ERR_INVALID_ARGUMENT;
-      const double g = f->m[k] * f->g[k];
-      out->m2[k] = f->m[k] * f->m[k];
-      out->mg[k] = g;
-      out->mg2[k] = g * g;
-      out->cr[k] = f->cr[k];
-      out->ci[k] = f->ci[k];
-      out->cig[k] = f->ci[k] * g;
-      out->crg[k] = f->cr[k] * g;
-      const float mf = (float)f->m[k], gf = mf * (float)f->g[k];
-      out->m2f[k] = mf * mf;
-      out->mgf[k] = gf;
-      out->mg2f[k] = gf * gf;
-      out->crf[k] = (float)f->cr[k];
-      out->cif[k] = (float)f->ci[k];
+      set_term(out, k, *f);
       out->a[k] = f->a[k];
       out->b[k] = f->b[k];
     }
   }
   if (f->kind == HPSP_F_MASS2_01 && nvec < 2) return HPSP_ERR_INVALID_ARGUMENT;
   return HPSP_OK;
+}
+
+inline int make_functork(const hpsp_functor* f, int nvec, AvgFunctor* out,
+                         int first_daughter = 0) {
+  const int rc = make_functork(f, nvec, &out->fast, first_daughter);
+  return rc ? rc : make_functork(f, nvec, &out->mixed, first_daughter);
 }
 
 inline int hip_status(int e) { return e == (int)hipSuccess ? HPSP_OK : HPSP_ERR_HIP; }

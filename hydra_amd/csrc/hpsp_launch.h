@@ -41,9 +41,9 @@ struct GenArgs {
   }
 };
 
-// AverageOn arguments; FK is the functor: a FunctorK description here, a
-// user's callable in a translation unit that compiles its own kernels
-// (hydra_amd/include/hydra/detail/UserKernels.h).
+// AverageOn arguments; FK is the functor: in the kernels a description
+// (FunctorFastK, FunctorMixedK) or a user's callable in a translation unit that
+// compiles its own kernels (hydra_amd/include/hydra/detail/UserKernels.h).
 template <typename FK>
 struct AvgArgsT {
   DecayK d;
@@ -53,7 +53,16 @@ struct AvgArgsT {
   uint64_t mld;
   Stats* partials;  // one per kAvgChunk events
 };
-using AvgArgs = AvgArgsT<FunctorK>;
+// A described functor in both forms, of which each launcher passes its own on.
+struct AvgFunctor {
+  FunctorFastK fast;
+  FunctorMixedK mixed;
+};
+using AvgArgs = AvgArgsT<AvgFunctor>;
+template <typename FK>
+inline AvgArgsT<FK> with_functor(const AvgArgs& a, const FK& f) {
+  return {a.d, f, a.first, a.n, a.mothers, a.mld, a.partials};
+}
 
 // Up to HPSP_MAX_EVAL_FUNCTORS described functors, evaluated one by one.
 struct DescSet {

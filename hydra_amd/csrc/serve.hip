@@ -126,7 +126,7 @@ struct Request {
   uint64_t ticket = 0;
   hpsp_request r{};
   DecayK dk{};
-  FunctorK fk{};
+  AvgFunctor fk{};
   size_t bytes = 0, off = 0;
   uint64_t next = 0;        // next event offset to launch
   bool launched_all = false;

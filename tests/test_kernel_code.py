@@ -34,3 +34,20 @@ def test_stored_events_waves(kernel):
     for N, want in zip(range(2, 13), STORED[kernel]):
         (k,) = co.find(f"{kernel}ILi{N}E").values()
         assert co.waves(k) >= want, (kernel, N, k[".vgpr_count"])
+
+
+# Bytes of a kernel's arguments: of calls on few events, the launch is the time.
+ARGUMENTS = {
+    "k_evaluate_f64ILi3ELi0ELb0E": 2208,
+    "k_hist_fillILi3ELb0E": 2080,
+    "k_average_f64ILi3ELi0ELb0ENS_13FunctorFastKELi4E": 1088,
+    "k_average_mixedILi3ELi0ELb0ELi4E": 960,
+    "k_uw_flagsILi3E": 928,
+    "k_range_histILi3E": 1824,
+}
+
+
+@pytest.mark.parametrize("kernel", ARGUMENTS)
+def test_argument_bytes(kernel):
+    (k,) = co.find(kernel).values()
+    assert k[".kernarg_segment_size"] <= ARGUMENTS[kernel]
