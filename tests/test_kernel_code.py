@@ -40,7 +40,7 @@ def test_stored_events_waves(kernel):
 ARGUMENTS = {
     "k_evaluate_f64ILi3ELi0ELb0E": 2208,
     "k_hist_fillILi3ELb0E": 2080,
-    "k_average_f64ILi3ELi0ELb0ENS_13FunctorFastKELi4E": 1088,
+    "k_average_f64ILi3ELi0ELb0ENS_12FunctorFastKELi4E": 1088,
     "k_average_mixedILi3ELi0ELb0ELi4E": 960,
     "k_uw_flagsILi3E": 928,
     "k_range_histILi3E": 1824,
