@@ -42,12 +42,20 @@ constexpr int kWaitLoads = 0xF70;
 constexpr int kMemAxes = 10;
 
 // Bound by the columns it reads: 3-body events with a weight column at 6.2 TB/s.
-// Without a PhaseSpaceWeight to form, a wave waits for each daughter's four
-// columns before it asks for the next: with all 13 columns asked for at once the
-// same bytes came slower (6e7 3-body events 1076 -> 1002 us, 4e7 4-body ones 884
-// -> 868), and more bytes in flight from a look ahead at the next event gained
-// nothing (1118 us).  From 9 bodies on the selections bound it, and the waits cost
-// (1e6 9-body events 65 -> 71 us).
+// Without a PhaseSpaceWeight to form, a wave of a large fill waits for each
+// daughter's four columns before it asks for the next (kByDaughter beside the
+// weight's mode): with all 12 or 13 columns asked for at once the same bytes came
+// slower (2e7 3-body events 327 -> 306 us, 4-body ones 428 -> 412), and more bytes
+// in flight from a look ahead at the next event gained nothing.  From kWaitEvents
+// on: with 1e6 events both take the same time, and below, where a wave has one
+// group of events or two, the waits are its time (1e5 3-body events 10.7 us
+// against 10.3, 4-body ones 12.3 against 11.6); 5 and more bodies come here where
+// the axes read as many, and wait at every size.  From 9 bodies on the selections
+// bound it, and the waits cost; with a PhaseSpaceWeight they do at every size (2e7
+// 3-body events 331 -> 337 us, 4-body ones 449 -> 457).
+constexpr uint64_t kWaitEvents = 1 << 21;
+constexpr int kByDaughter = 8;  // added to the mode
+
 template <int N, bool FEW>
 __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
                                            double (&x)[HPSP_HIST_MAX_DIM], double& w) {
@@ -62,7 +70,8 @@ __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
   for (int i = 0; i < N; ++i)
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      if (N >= 3 && N <= 8 && c == 0 && i > 0 && a.weight_mode != HPSP_HIST_WEIGHT_PHSP) {
+      if (N >= 3 && N <= 8 && c == 0 && i > 0 &&
+          (N <= 4 ? a.weight_mode >= kByDaughter : a.weight_mode != HPSP_HIST_WEIGHT_PHSP)) {
         __builtin_amdgcn_s_waitcnt(kWaitLoads);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -71,11 +80,18 @@ __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
   if constexpr (!FEW) {
 #pragma unroll
     for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d) {
-      const RegAcc<double, N, (N <= 8)> acc(p, wants_pairs(a.axes[d]));
-      x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true>(a.axes[d], acc) : 0.0;
+      // 4 bodies: the six pairs before the branch on the axis' kind cost registers
+      // (122 against 111; 2e4 events 11.0 -> 10.8 us, 1e5 11.4 -> 11.1); 3 and 7
+      // bodies with the weight lose by it (1e6 events 26 -> 27, 50 -> 52)
+      if constexpr (N == 4) {
+        x[d] = (d < a.h.ndim) ? functor_stored<true>(a.axes[d], p) : 0.0;
+      } else {
+        const RegAcc<double, N, (N <= 8)> acc(p, wants_pairs(a.axes[d]));
+        x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true>(a.axes[d], acc) : 0.0;
+      }
     }
   }
-  if (a.weight_mode == HPSP_HIST_WEIGHT_COLUMN)
+  if ((N <= 4 ? a.weight_mode % kByDaughter : a.weight_mode) == HPSP_HIST_WEIGHT_COLUMN)
     w = a.w[k];
   else if (a.weight_mode == HPSP_HIST_WEIGHT_PHSP)
     w = event_weight_f64<N>(p, a.d.m, a.d.maxw);
@@ -186,9 +202,13 @@ int launch_histogram_fill(int N, const HistArgs& in, hipStream_t s) {
     int reads = 0;
     for (int d = 0; d < a.h.ndim; ++d) reads += axis_reads(a.axes[d]);
     few = reads < N;
-    if (N >= 5 && few && a.weight_mode != HPSP_HIST_WEIGHT_PHSP) {
-      if (a.weight_mode != HPSP_HIST_WEIGHT_COLUMN) a.w = nullptr;
-      N = -1;
+    if (a.weight_mode != HPSP_HIST_WEIGHT_PHSP) {
+      if (N >= 5 && few) {
+        if (a.weight_mode != HPSP_HIST_WEIGHT_COLUMN) a.w = nullptr;
+        N = -1;
+      } else if (N <= 4 && a.n >= kWaitEvents) {
+        a.weight_mode += kByDaughter;
+      }
     }
   }
   a.use_lds = nslots <= a.lds_slots ? 1 : 0;

@@ -991,15 +991,15 @@ __device__ __forceinline__ double functor_eval(const FK& f, const Real (&p)[P][4
 // (LateAcc; before the branch on its kind they were held beside the momenta: 4
 // bodies 85 registers against 75), and all daughters summed by the general loop (8
 // bodies 118 against 110).
-template <int P>
-struct LateAcc : RegAcc<double, P, false> {
-  using Reg = RegAcc<double, P, false>;
+template <int P, bool AllSum>
+struct LateAcc : RegAcc<double, P, AllSum> {
+  using Reg = RegAcc<double, P, AllSum>;
   __device__ __forceinline__ LateAcc(const double (&p)[P][4]) : Reg(p, false) {}
   __device__ __forceinline__ Reg pairs() const { return Reg(this->p, true); }
 };
-template <int P>
+template <bool AllSum = false, int P>
 __device__ __forceinline__ double functor_stored(const FunctorK& f, const double (&p)[P][4]) {
-  return functor_eval_acc<double, true>(f, LateAcc<P>(p));
+  return functor_eval_acc<double, true>(f, LateAcc<P, AllSum>(p));
 }
 
 // ---------------------------------------------------------------------------

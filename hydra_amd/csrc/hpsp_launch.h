@@ -161,7 +161,7 @@ struct HistArgs {
   const double* cols;       // events source: 4N momentum columns
   uint64_t ld;
   ParticlesK parts;         // particles source
-  int weight_mode;          // hpsp_hist_weight
+  int weight_mode;          // hpsp_hist_weight (the launcher may add kByDaughter)
   const double* w;
   uint64_t n;
   double* contents;         // nbins + 2

@@ -160,6 +160,39 @@ def test_event_axes_equal_their_columns(N):
             check_weighted(fill_events(grid, lo, hi, dec, axes, cols, mode, wc, n=n), ref[1], ref[1])
 
 
+@pytest.mark.parametrize("N", [3, 4])
+@pytest.mark.parametrize("over", [-1, 7])
+def test_events_beside_the_size_where_loads_wait(N, over):
+    """2^21 events: from there a wave reads one daughter's columns after the other's."""
+    m = [0.2 + 0.1 * ((5 * i) % 7) for i in range(N)]
+    M = 1.8 * sum(m)
+    dec = make_decay(M, m)
+    n = (1 << 21) + over
+    cols, _, evw = generate(dec, 17, n, want_wt=False)
+    axes = [make_functor(capi.F_MASS2, (0, N - 1)), make_functor(capi.F_COS_HELICITY, (0, 1))]
+    p = capi.Particles()
+    p.n = N
+    for i in range(N):
+        p.cols[i], p.ld[i] = cols.data_ptr() + 32 * n * i, n
+    x = torch.empty((2, n), dtype=torch.float64, device=DEV)
+    check(lib().hpsp_particles_evaluate(ctypes.byref(p), capi.functor_array(axes), 2, n, ptr(x), n,
+                                        stream_handle()), "evaluate")
+    grid, lo, hi = [60, 60], [0.0, -1.0], [M * M, 1.0]
+    h = capi.make_histogram(grid, lo, hi)
+    ref = []
+    for w in (None, evw):
+        out = torch.empty(3602, dtype=torch.float64, device=DEV)
+        check(lib().hpsp_histogram_fill(ctypes.byref(h), ptr(x), n, n, ptr(w), ptr(out),
+                                        stream_handle()), "fill")
+        ref.append(out.cpu().numpy())
+    got = fill_events(grid, lo, hi, dec, axes, cols, capi.HIST_WEIGHT_ONE, n=n)
+    assert np.array_equal(got, ref[0]) and got.sum() == n
+    for mode, wc in ((capi.HIST_WEIGHT_COLUMN, evw), (capi.HIST_WEIGHT_PHSP, None)):
+        got = fill_events(grid, lo, hi, dec, axes, cols, mode, wc, n=n)
+        # two sums of a bin's entries in any order, each off by a rounding per entry
+        assert np.all(np.abs(got - ref[1]) <= 2.0 ** -52 * ref[0] * ref[1])
+
+
 def test_fill_repeats_and_empty():
     """A fill overwrites the contents; n = 0 leaves them zero."""
     x = np.linspace(0, 1, 1001)[None, :]
