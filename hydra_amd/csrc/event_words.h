@@ -111,6 +111,16 @@ struct BlockSlots {
   }
 };
 
+// The one block of an event whose e + 3N is d.
+template <int ENGINE, int A>
+__device__ __forceinline__ void event_block(const uint64_t* key, uint64_t d, uint64_t (&out)[A]) {
+  const uint64_t c[4] = {d + 1, d + 1 == 0 ? 1ULL : 0ULL, 0, 0};
+  uint64_t o[4];
+  r123_block<ENGINE>(key, c, o);
+#pragma unroll
+  for (int e = 0; e < A; ++e) out[e] = o[e];
+}
+
 // The first W words of each event of a wave's groups, taken in order.
 template <int N, int ENGINE, int W = 3 * N - 4>
 struct EventWords {
@@ -148,12 +158,7 @@ struct EventWords {
         if constexpr (kShared) v.shift(own);
       }
     } else if constexpr (!kShared) {
-      uint64_t c[4] = {d0 + (uint64_t)lane, 0, 0, 0}, o[4];
-      c[0] += 1;
-      c[1] = c[0] == 0 ? 1 : 0;
-      r123_block<ENGINE>(d.key, c, o);
-#pragma unroll
-      for (int e = 0; e < A; ++e) own[e] = o[e];
+      event_block<ENGINE>(d.key, d0 + (uint64_t)lane, own);
     } else {
       if (restart || again) {
         const BlockSlots<NB> b(d0, kWave);
@@ -182,7 +187,9 @@ struct EventWords {
   }
 };
 
-// The words of the kBlock consecutive events of a block, one per thread.
+// The words of the kBlock consecutive events of a block, one per thread.  Events
+// that need a single Random123 block (2 bodies) have none to share: each thread
+// keeps its own (through LDS, 4e6 2-body events of Philox4x64 57 us against 47).
 template <int N, int ENGINE>
 struct BlockEventWords {
   using T = word_t<ENGINE>;
@@ -190,11 +197,14 @@ struct BlockEventWords {
   static constexpr int A = engine_arity<ENGINE>();
   static constexpr int NB = (W + A - 1) / A;
   static constexpr int kSlots = kBlock + (is_squares<ENGINE>() ? NB - 1 : 2 * NB);
-  struct Store {  // __shared__
+  static constexpr bool kShared = NB > 1;
+  struct Words {
     T w[A][kSlots];
   };
+  struct Nothing {};
+  using Store = std::conditional_t<kShared, Words, Nothing>;  // __shared__
   lptr<T> p;
-  T own;  // word 0
+  T own[kShared ? 1 : A];  // word 0; all of them
 
   // Event first + t in thread t; every thread of the block calls it.
   __device__ __forceinline__ void fill(Store& s, const DecayK& d, uint64_t first) {
@@ -202,12 +212,14 @@ struct BlockEventWords {
     const uint64_t d0 = first + 3 * (uint64_t)N;
     if constexpr (is_squares<ENGINE>()) {
       const uint64_t key = d.key[0];
-      own = squares_word_y<ENGINE>(key, key * (d0 + t));
-      s.w[0][t] = own;
+      own[0] = squares_word_y<ENGINE>(key, key * (d0 + t));
+      s.w[0][t] = own[0];
       if (t < (uint32_t)(NB - 1))
         s.w[0][kBlock + t] = squares_word_y<ENGINE>(key, key * (d0 + kBlock + t));
       __syncthreads();
       p = (lptr<T>)&s.w[0][t];
+    } else if constexpr (!kShared) {
+      event_block<ENGINE>(d.key, d0 + t, own);
     } else {
       const BlockSlots<NB> b(d0, kBlock);
       const uint32_t slots = kBlock + (b.before == ~0ULL ? NB - 1 : 2 * NB);
@@ -219,11 +231,14 @@ struct BlockEventWords {
       }
       __syncthreads();
       p = (lptr<T>)&s.w[0][t + b.shift(t)];
-      own = p[0];
+      own[0] = p[0];
     }
   }
   __device__ __forceinline__ uint64_t operator()(int j) const {
-    return j == 0 ? own : p[(j % A) * kSlots + j / A];
+    if constexpr (kShared)
+      return j == 0 ? own[0] : p[(j % A) * kSlots + j / A];
+    else
+      return own[j];
   }
 };
 

@@ -40,13 +40,14 @@ struct DecayK {
   double maxw;
   double mas0, masN;  // invMas[0] = 0 ecm + msum[0] and invMas[N-1] = 1 ecm + msum[N-1]
   double rmasN;       // RN(1 / invMas[N-1])
-  // Every invMas lies in [2^-300, 2^300], where div_core divides exactly
-  // rounded: plain_m says so of the masses, plain of the masses and ecm.
-  int plain_m, plain;
+  double pd2;         // N = 2: the daughters' momentum
   uint64_t key[4];  // engine key words, already splitmix-ed
   // Final boost of a single mother (Vector4R.inl:312-369) with its derived
   // constants, valid when do_boost != 0 (0 < b2 < 1).
   double bx, by, bz, bxx, byy, bzz, gamma, gb2, gb2xy, gb2xz, gb2yz, gbx, gby, gbz;
+  // Every invMas lies in [2^-300, 2^300], where div_core divides exactly
+  // rounded: plain_m says so of the masses, plain of the masses and ecm.
+  int16_t plain_m, plain;
   int do_boost;
 };
 

@@ -69,6 +69,10 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
   k.mas0 = 0.0 * d->ecm + k.msum[0];
   k.masN = 1.0 * d->ecm + sum;
   k.rmasN = 1.0 / k.masN;
+  if (d->n == 2) {  // pdk, as the device forms it
+    const double a = k.masN, b = k.mas0, c = d->masses[1];
+    k.pd2 = sqrt((a - b - c) * (a + b + c) * (a - b + c) * (a + b - c)) / (2 * a);
+  }
   k.plain_m = plain && k.msum[0] >= 0x1p-300 && sum <= 0x1p+299;
   k.plain = k.plain_m && d->ecm >= 0.0 && d->ecm <= 0x1p+299;
   engine_keys(d->engine, seed, k.key);

@@ -51,3 +51,12 @@ ARGUMENTS = {
 def test_argument_bytes(kernel):
     (k,) = co.find(kernel).values()
     assert k[".kernarg_segment_size"] <= ARGUMENTS[kernel]
+
+
+@pytest.mark.parametrize("engine", range(2, 6))
+@pytest.mark.parametrize("kernel", ["k_generate_f64", "k_evaluate_f64", "k_generate_mixed"])
+def test_single_blocks_stay_in_registers(kernel, engine):
+    """2-body events of the Random123 engines need one block each: nothing of it is
+    shared, so nothing goes through LDS."""
+    for k in co.find(f"{kernel}ILi2ELi{engine}ELb0E").values():
+        assert k[".group_segment_fixed_size"] == 0
