@@ -84,7 +84,7 @@ __device__ __forceinline__ void event_axes(const HistArgs& a, uint64_t k,
       // (122 against 111; 2e4 events 11.0 -> 10.8 us, 1e5 11.4 -> 11.1); 3 and 7
       // bodies with the weight lose by it (1e6 events 26 -> 27, 50 -> 52)
       if constexpr (N == 4) {
-        x[d] = (d < a.h.ndim) ? functor_stored<true>(a.axes[d], p) : 0.0;
+        x[d] = (d < a.h.ndim) ? functor_late<true, true>(a.axes[d], p) : 0.0;
       } else {
         const RegAcc<double, N, (N <= 8)> acc(p, wants_pairs(a.axes[d]));
         x[d] = (d < a.h.ndim) ? functor_eval_acc<double, true>(a.axes[d], acc) : 0.0;
@@ -158,7 +158,7 @@ static int axis_reads(const FunctorK& f) {
   switch (f.kind) {
     case HPSP_F_ONE: return 0;
     case HPSP_F_BW_SUM: return 2 * f.nterms;
-    case HPSP_F_COS_HELICITY: return f.b[1] + 2;
+    case HPSP_F_COS_HELICITY: return f.t[1].b + 2;
     default: return 2;
   }
 }

@@ -56,29 +56,34 @@ struct DecayK {
 // form of the sum has a type with the constants that it reads and no others: a
 // launch of few events pays for its arguments (with one type for all, Evaluate of
 // 1000 2-body events over mothers took 5.6 us against 5.2, of three functors 5.5
-// against 5.0).
-struct FunctorK {  // exactly rounded divisions
+// against 5.0).  A term's constants lie together, its pair first, for few and wide
+// scalar loads (AverageOn of 4e6 8-body events 222 us with an array for each
+// constant, 215 so).
+struct TermK {  // exactly rounded divisions
+  int a, b;
+  double m2, mg, mg2;  // M^2, g, g^2
+  double cr, ci;
+};
+struct TermFastK {  // AverageOn: fused, through reciprocals
+  int a, b;
+  double m2, mg2;
+  double cr, ci;
+  double cig, crg;  // ci g, cr g
+};
+struct TermMixedK {  // AverageOn in mixed precision: from M and G rounded to FP32
+  int a, b;
+  float m2, mg, mg2;
+  float cr, ci;
+};
+template <typename Term>
+struct FunctorT {
   int kind;
   int nterms;
-  double m2[HPSP_MAX_TERMS], mg[HPSP_MAX_TERMS], mg2[HPSP_MAX_TERMS];  // M^2, g, g^2
-  double cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
-  int a[HPSP_MAX_TERMS], b[HPSP_MAX_TERMS];
+  Term t[HPSP_MAX_TERMS];
 };
-struct FunctorFastK {  // AverageOn: fused, through reciprocals
-  int kind;
-  int nterms;
-  double m2[HPSP_MAX_TERMS], mg2[HPSP_MAX_TERMS];
-  double cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
-  double cig[HPSP_MAX_TERMS], crg[HPSP_MAX_TERMS];  // ci g, cr g
-  int a[HPSP_MAX_TERMS], b[HPSP_MAX_TERMS];
-};
-struct FunctorMixedK {  // AverageOn in mixed precision: from M and G rounded to FP32
-  int kind;
-  int nterms;
-  float m2[HPSP_MAX_TERMS], mg[HPSP_MAX_TERMS], mg2[HPSP_MAX_TERMS];
-  float cr[HPSP_MAX_TERMS], ci[HPSP_MAX_TERMS];
-  int a[HPSP_MAX_TERMS], b[HPSP_MAX_TERMS];
-};
+using FunctorK = FunctorT<TermK>;
+using FunctorFastK = FunctorT<TermFastK>;
+using FunctorMixedK = FunctorT<TermMixedK>;
 
 // A wave-uniform pointer pinned to SGPRs, so that per-lane accesses are
 // (scalar base) + lane offset and no 64-bit VGPR address is kept per column.
@@ -881,8 +886,8 @@ __device__ __forceinline__ double functor_eval_acc(const FK& f, const Acc& acc) 
 #pragma clang fp contract(off)
   if (f.kind == HPSP_F_ONE) return 1.0;
   if (f.kind == HPSP_F_MASS2_01 || f.kind == HPSP_F_MASS2 || f.kind == HPSP_F_MASS) {
-    const int ia = f.kind == HPSP_F_MASS2_01 ? 0 : f.a[0];
-    const int ib = f.kind == HPSP_F_MASS2_01 ? 1 : f.b[0];
+    const int ia = f.kind == HPSP_F_MASS2_01 ? 0 : f.t[0].a;
+    const int ib = f.kind == HPSP_F_MASS2_01 ? 1 : f.t[0].b;
     const Real m2 = acc.pairs().pair(ia, ib);
     if (f.kind != HPSP_F_MASS) return (double)m2;
     // Vector4R::mass: 0 unless the square is positive
@@ -895,12 +900,12 @@ __device__ __forceinline__ double functor_eval_acc(const FK& f, const Acc& acc) 
   }
   if (f.kind == HPSP_F_COS_HELICITY) {
     // P = p[first] + ... + p[first + count - 1] left to right (first, count
-    // in a[1], b[1]); q = d + p[b0]; d = p[a0]
+    // in a and b of t[1]); q = d + p[b0]; d = p[a0]
     Real Pv[4];
-    acc.sum(f.a[1], f.a[1] + f.b[1], Pv);
+    acc.sum(f.t[1].a, f.t[1].a + f.t[1].b, Pv);
     Real d[4], e[4], q[4];
-    acc.get(f.a[0], d);
-    acc.get(f.b[0], e);
+    acc.get(f.t[0].a, d);
+    acc.get(f.t[0].b, e);
 #pragma unroll
     for (int c = 0; c < 4; ++c) q[c] = d[c] + e[c];
     const Real pd = dot4(Pv, d);
@@ -925,9 +930,9 @@ __device__ __forceinline__ double functor_eval_acc(const FK& f, const Acc& acc) 
     // in [0, 2 pi) (phsp_chain.inl:191-207): the components of d and h
     // transverse to K's three-momentum, d' = K x d_perp, chi = atan2(y, x)
     Real d[4], e[4], h[4], K[4];
-    acc.get(f.a[0], d);
-    acc.get(f.b[0], e);
-    acc.get(f.a[1], h);
+    acc.get(f.t[0].a, d);
+    acc.get(f.t[0].b, e);
+    acc.get(f.t[1].a, h);
 #pragma unroll
     for (int c = 0; c < 4; ++c) K[c] = d[c] + e[c];
     const Real kk = dot3(K, K);
@@ -953,30 +958,31 @@ __device__ __forceinline__ double functor_eval_acc(const FK& f, const Acc& acc) 
   Real Ar = 0, Ai = 0;
   const auto& pairs = acc.pairs();
   for (int k = 0; k < f.nterms; ++k) {
-    const Real s = pairs.pair(f.a[k], f.b[k]);
+    const auto& t = f.t[k];
+    const Real s = pairs.pair(t.a, t.b);
     if constexpr (Exact) {
-      const Real dr = f.m2[k] - s;
-      const Real den = dr * dr + f.mg2[k];
+      const Real dr = t.m2 - s;
+      const Real den = dr * dr + t.mg2;
       const Real br = dr / den;
-      const Real bi = f.mg[k] / den;
-      const Real tr = f.cr[k] * br - f.ci[k] * bi;
-      const Real ti = f.cr[k] * bi + f.ci[k] * br;
+      const Real bi = t.mg / den;
+      const Real tr = t.cr * br - t.ci * bi;
+      const Real ti = t.cr * bi + t.ci * br;
       Ar += tr;
       Ai += ti;
     } else if constexpr (sizeof(Real) == 4) {
-      const float dr = f.m2[k] - s;
-      const float inv = __builtin_amdgcn_rcpf(dr * dr + f.mg2[k]);
+      const float dr = t.m2 - s;
+      const float inv = __builtin_amdgcn_rcpf(dr * dr + t.mg2);
       const float br = dr * inv;
-      const float bi = f.mg[k] * inv;
-      const float tr = f.cr[k] * br - f.ci[k] * bi;
-      const float ti = f.cr[k] * bi + f.ci[k] * br;
+      const float bi = t.mg * inv;
+      const float tr = t.cr * br - t.ci * bi;
+      const float ti = t.cr * bi + t.ci * br;
       Ar += tr;
       Ai += ti;
     } else {
-      const double dr = f.m2[k] - s;
-      const double inv = rcp_fast(__builtin_fma(dr, dr, f.mg2[k]));
-      Ar = __builtin_fma(__builtin_fma(f.cr[k], dr, -f.cig[k]), inv, Ar);
-      Ai = __builtin_fma(__builtin_fma(f.ci[k], dr, f.crg[k]), inv, Ai);
+      const double dr = t.m2 - s;
+      const double inv = rcp_fast(__builtin_fma(dr, dr, t.mg2));
+      Ar = __builtin_fma(__builtin_fma(t.cr, dr, -t.cig), inv, Ar);
+      Ai = __builtin_fma(__builtin_fma(t.ci, dr, t.crg), inv, Ai);
     }
   }
   return (double)(Ar * Ar + Ai * Ai);
@@ -987,20 +993,25 @@ __device__ __forceinline__ double functor_eval(const FK& f, const Real (&p)[P][4
   return functor_eval_acc<Real, Exact>(f, RegAcc<Real, P>(p, wants_pairs(f)));
 }
 
-// The same of a stored event, in the kernels that its columns bound, where
-// registers are waves: the pair masses are formed where a functor takes them
-// (LateAcc; before the branch on its kind they were held beside the momenta: 4
-// bodies 85 registers against 75), and all daughters summed by the general loop (8
-// bodies 118 against 110).
-template <int P, bool AllSum>
-struct LateAcc : RegAcc<double, P, AllSum> {
-  using Reg = RegAcc<double, P, AllSum>;
-  __device__ __forceinline__ LateAcc(const double (&p)[P][4]) : Reg(p, false) {}
+// The same where registers are waves or spills and one functor is evaluated per
+// event: the pair masses are formed where it takes them (LateAcc), not before the
+// branch on its kind, which held them beside the momenta (weights of stored 4-body
+// events 85 registers against 75; AverageOn of 2 and 3 bodies spilled).
+template <typename Real, int P, bool AllSum>
+struct LateAcc : RegAcc<Real, P, AllSum> {
+  using Reg = RegAcc<Real, P, AllSum>;
+  __device__ __forceinline__ LateAcc(const Real (&p)[P][4]) : Reg(p, false) {}
   __device__ __forceinline__ Reg pairs() const { return Reg(this->p, true); }
 };
-template <bool AllSum = false, int P>
+template <bool Exact, bool AllSum, typename FK, typename Real, int P>
+__device__ __forceinline__ double functor_late(const FK& f, const Real (&p)[P][4]) {
+  return functor_eval_acc<Real, Exact>(f, LateAcc<Real, P, AllSum>(p));
+}
+// Of a stored event: without RegAcc's own sum of all daughters as well (8 bodies 118
+// registers against 110).
+template <int P>
 __device__ __forceinline__ double functor_stored(const FunctorK& f, const double (&p)[P][4]) {
-  return functor_eval_acc<double, true>(f, LateAcc<P, AllSum>(p));
+  return functor_late<true, false>(f, p);
 }
 
 // ---------------------------------------------------------------------------

@@ -101,30 +101,17 @@ inline DecayK make_decayk(const hpsp_decay* d, uint64_t seed) {
 }
 
 // The constants of Breit-Wigner term k.
-inline void set_term(FunctorK* out, int k, const hpsp_functor& f) {
+inline void set_term(TermK* out, int k, const hpsp_functor& f) {
   const double g = f.m[k] * f.g[k];
-  out->m2[k] = f.m[k] * f.m[k];
-  out->mg[k] = g;
-  out->mg2[k] = g * g;
-  out->cr[k] = f.cr[k];
-  out->ci[k] = f.ci[k];
+  *out = {f.a[k], f.b[k], f.m[k] * f.m[k], g, g * g, f.cr[k], f.ci[k]};
 }
-inline void set_term(FunctorFastK* out, int k, const hpsp_functor& f) {
+inline void set_term(TermFastK* out, int k, const hpsp_functor& f) {
   const double g = f.m[k] * f.g[k];
-  out->m2[k] = f.m[k] * f.m[k];
-  out->mg2[k] = g * g;
-  out->cr[k] = f.cr[k];
-  out->ci[k] = f.ci[k];
-  out->cig[k] = f.ci[k] * g;
-  out->crg[k] = f.cr[k] * g;
+  *out = {f.a[k], f.b[k], f.m[k] * f.m[k], g * g, f.cr[k], f.ci[k], f.ci[k] * g, f.cr[k] * g};
 }
-inline void set_term(FunctorMixedK* out, int k, const hpsp_functor& f) {
+inline void set_term(TermMixedK* out, int k, const hpsp_functor& f) {
   const float m = (float)f.m[k], g = m * (float)f.g[k];
-  out->m2[k] = m * m;
-  out->mg[k] = g;
-  out->mg2[k] = g * g;
-  out->cr[k] = (float)f.cr[k];
-  out->ci[k] = (float)f.ci[k];
+  *out = {f.a[k], f.b[k], m * m, g, g * g, (float)f.cr[k], (float)f.ci[k]};
 }
 
 // nvec: four-vectors the functor sees; first_daughter: index of the first
@@ -146,22 +133,22 @@ inline int make_functork(const hpsp_functor* f, int nvec, FK* out, int first_dau
       f->kind == HPSP_F_DECAY_PLANE_ANGLE) {
     if (f->a[0] < 0 || f->a[0] >= nvec || f->b[0] < 0 || f->b[0] >= nvec)
       return HPSP_ERR_INVALID_ARGUMENT;
-    out->a[0] = f->a[0];
-    out->b[0] = f->b[0];
+    out->t[0].a = f->a[0];
+    out->t[0].b = f->b[0];
     if (f->kind == HPSP_F_COS_HELICITY) {
       if (f->b[1] > 0) {  // an explicit parent p[a1] .. p[a1 + b1 - 1]
         if (f->a[1] < 0 || f->a[1] >= nvec || f->b[1] > nvec - f->a[1])
           return HPSP_ERR_INVALID_ARGUMENT;
-        out->a[1] = f->a[1];
-        out->b[1] = f->b[1];
+        out->t[1].a = f->a[1];
+        out->t[1].b = f->b[1];
       } else {  // the sum of the daughters
-        out->a[1] = first_daughter;
-        out->b[1] = nvec - first_daughter;
+        out->t[1].a = first_daughter;
+        out->t[1].b = nvec - first_daughter;
       }
     }
     if (f->kind == HPSP_F_DECAY_PLANE_ANGLE) {
       if (f->a[1] < 0 || f->a[1] >= nvec) return HPSP_ERR_INVALID_ARGUMENT;
-      out->a[1] = f->a[1];
+      out->t[1].a = f->a[1];
     }
   }
   if (f->kind == HPSP_F_BW_SUM) {
@@ -170,9 +157,7 @@ inline int make_functork(const hpsp_functor* f, int nvec, FK* out, int first_dau
     for (int k = 0; k < f->nterms; ++k) {
       if (f->a[k] < 0 || f->a[k] >= nvec || f->b[k] < 0 || f->b[k] >= nvec)
         return HPSP_ERR_INVALID_ARGUMENT;
-      set_term(out, k, *f);
-      out->a[k] = f->a[k];
-      out->b[k] = f->b[k];
+      set_term(&out->t[k], k, *f);
     }
   }
   if (f->kind == HPSP_F_MASS2_01 && nvec < 2) return HPSP_ERR_INVALID_ARGUMENT;

@@ -40,7 +40,7 @@ def test_stored_events_waves(kernel):
 ARGUMENTS = {
     "k_evaluate_f64ILi3ELi0ELb0E": 2208,
     "k_hist_fillILi3ELb0E": 2080,
-    "k_average_f64ILi3ELi0ELb0ENS_12FunctorFastKELi4E": 1088,
+    "k_average_f64ILi3ELi0ELb0E": 1088,
     "k_average_mixedILi3ELi0ELb0ELi4E": 960,
     "k_uw_flagsILi3E": 928,
     "k_range_histILi3E": 1824,
@@ -49,8 +49,8 @@ ARGUMENTS = {
 
 @pytest.mark.parametrize("kernel", ARGUMENTS)
 def test_argument_bytes(kernel):
-    (k,) = co.find(kernel).values()
-    assert k[".kernarg_segment_size"] <= ARGUMENTS[kernel]
+    for k in co.find(kernel).values():
+        assert k[".kernarg_segment_size"] <= ARGUMENTS[kernel]
 
 
 @pytest.mark.parametrize("engine", range(2, 6))
@@ -60,3 +60,13 @@ def test_single_blocks_stay_in_registers(kernel, engine):
     shared, so nothing goes through LDS."""
     for k in co.find(f"{kernel}ILi2ELi{engine}ELb0E").values():
         assert k[".group_segment_fixed_size"] == 0
+
+
+@pytest.mark.parametrize("mothers", [0, 1])
+@pytest.mark.parametrize("N", [2, 3, 4])
+def test_average_spills_nothing(N, mothers):
+    """AverageOn's form of four waves per chunk, every engine."""
+    for engine in range(6):
+        for name, k in co.find(f"k_average_f64ILi{N}ELi{engine}ELb{mothers}E").items():
+            if k[".max_flat_workgroup_size"] == 256:
+                assert k[".vgpr_spill_count"] == 0, name
