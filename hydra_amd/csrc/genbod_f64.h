@@ -207,13 +207,18 @@ __device__ __forceinline__ double avg_value(const FunctorFastK& f, const double 
 // staged values in the same order: the same partial, bit for bit.
 constexpr int avg_wide_waves(int N) { return N <= 6 ? 16 : 8; }  // 128 or 256 registers
 
-// Waves per SIMD asked for of the form with four waves per chunk: over mothers,
-// which hold one more four-vector and a boost, 5 waves would spill up to 3 bodies.
-constexpr int avg_waves_for(int N, bool mothers) { return mothers && N <= 3 ? 4 : waves_for(N); }
+// Waves per SIMD asked for of the form with four waves per chunk: up to 3 bodies 5
+// would spill over mothers, which hold one more four-vector and a boost, and for 2
+// bodies beside Philox' products.
+constexpr int avg_waves_for(int N, int engine, bool mothers) {
+  const bool philox = engine == HPSP_PHILOX || engine == HPSP_PHILOX_LONG;
+  return N <= 3 && (mothers || (N == 2 && philox)) ? 4 : waves_for(N);
+}
 
 template <int N, int ENGINE, bool MOTHERS, typename FK = FunctorFastK, int WAVES = kBlock / kWave>
 __global__ __launch_bounds__(WAVES * kWave)
-    __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? avg_waves_for(N, MOTHERS) : WAVES / 4, 8)))
+    __attribute__((amdgpu_waves_per_eu(WAVES == 4 ? avg_waves_for(N, ENGINE, MOTHERS) : WAVES / 4,
+                                       8)))
 void k_average_f64(const AvgArgsT<FK> a) {
   constexpr int kFold = kBlock / kWave;  // waves that fold
   constexpr bool kWide = WAVES > kFold;
