@@ -12,8 +12,6 @@ namespace hpsp {
 constexpr int kAvgChunk = 4096;  // events per AverageOn reduction chunk
 constexpr int kUwTile = 1024;    // events per Unweight tile (256 threads x 4)
 constexpr int kXcds = 8;         // MI355X: workgroups are dealt to 8 XCDs in turn
-constexpr uint64_t kRunMax = 16;        // longest generation run, in groups of 64 events
-constexpr uint64_t kRunMaxStores = 4;   // longest run of a launch bound by its column stores
 constexpr uint64_t kRunMinRuns = 8192;  // 8 runs per SIMD of 256 CUs x 4 SIMDs
 
 struct GenArgs {
@@ -176,7 +174,6 @@ struct RangeArgs {
   DecayK d;            // key words unused
   uint32_t x_start;
   uint32_t run;        // consecutive groups of 64 elements per wave (set by the launcher)
-  uint32_t a_stride;   // 48271^(elements from a wave's run to its next; set by the launcher)
   uint64_t n;
   double* cols;        // generate: 4N momentum columns of ld doubles
   uint64_t ld;
@@ -343,19 +340,20 @@ inline void over_grids(const Args& a, Launch&& launch) {
 // Groups of 64 elements per wave in a run of k_range_generate: a longer run
 // shares more engine words between consecutive groups, but the runs must still
 // give every SIMD several waves; the longest power of two up to max_run that
-// leaves kRunMinRuns runs.  A launch bound by its column stores (momenta of at
-// most 3 daughters) takes max_run = kRunMaxStores: longer runs spread the chip's
-// concurrent writes over a wider window of the columns.
-inline uint32_t run_groups(uint64_t ngroups, uint64_t max_run = kRunMax) {
+// leaves kRunMinRuns runs.
+inline uint32_t run_groups(uint64_t ngroups, uint64_t max_run) {
   uint64_t r = 1;
   while (r < max_run && ngroups >= 2 * r * kRunMinRuns) r *= 2;
   return (uint32_t)r;
 }
 
-// Blocks of four waves for nruns runs, one run per wave (grid-stride beyond).
-inline unsigned grid_for_runs(uint64_t nruns) {
-  const uint64_t want = (nruns + kBlock / kWave - 1) / (kBlock / kWave);
-  return (unsigned)(want == 0 ? 1 : (want < (1u << 20) ? want : (1u << 20)));
+// Blocks of four waves for the runs of ngroups groups, one run per wave; the runs
+// are lengthened where they would be more than one launch can hold.
+inline unsigned blocks_for_runs(uint64_t ngroups, uint32_t& run) {
+  constexpr uint64_t kWavesPerBlock = kBlock / kWave, kMostRuns = kGridEvents / kWave;
+  while ((ngroups + run - 1) / run > kMostRuns) run *= 2;
+  const uint64_t nruns = (ngroups + run - 1) / run;
+  return (unsigned)((nruns + kWavesPerBlock - 1) / kWavesPerBlock);
 }
 
 // AverageOn over n events: wide(blocks, threads), waves_wide waves per chunk,

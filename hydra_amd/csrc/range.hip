@@ -5,12 +5,11 @@
 // -ffp-contract=off.
 //
 // Engine words.  minstd_rand's word j of element first + k is
-// x_start * a^(k + j) mod m (a = 48271, m = 2^31 - 1).  A wave takes runs of
+// x_start * a^(k + j) mod m (a = 48271, m = 2^31 - 1).  A wave takes one run of
 // consecutive groups of 64 elements, whose words it shares through LDS
 // (WindowView): a lane evaluates the word 64 after its last one, one product
 // with a^64, for each further group.  A run's first words cost one power of
-// a, formed on the scalar unit, and a table lookup; a wave's next run one
-// product with a^(the events between).
+// a, formed on the scalar unit, and a table lookup.
 //
 // Kernels:
 //   k_range_generate<N>  elements into SoA momentum columns and a weight column
@@ -51,28 +50,22 @@ struct RangeWords {
   using View = WindowView<uint32_t, 1, W>;
   using Window = typename View::Win;
   View v;
-  uint32_t x0;  // the lane's word at the run's first group
-  uint32_t x;   // its last word
+  uint32_t x;  // the lane's last word
 
-  // the first run, whose first element is k0
-  __device__ __forceinline__ void first(uint32_t x_start, uint64_t k0, int lane) {
+  // the run's first group, whose first element is k0
+  __device__ __forceinline__ void start(Window& win, uint32_t x_start, uint64_t k0, int lane) {
     const uint32_t xw = minstd_mul(x_start, minstd_pow(k0));
-    x0 = minstd_mul(xw, kPow.v[lane]);
+    const uint32_t lo[1] = {minstd_mul(xw, kPow.v[lane])};
+    x = minstd_mul(lo[0], kMinstdA64);
+    const uint32_t hi[1] = {x};
+    v.start(win, lane, 0, lo, hi);
   }
-  // the run's first group, or the group after the last
-  __device__ __forceinline__ void next(Window& win, int lane, bool restart) {
-    if (restart) {
-      x = minstd_mul(x0, kMinstdA64);
-      const uint32_t lo[1] = {x0}, hi[1] = {x};
-      v.start(win, lane, 0, lo, hi);
-    } else {
-      x = minstd_mul(x, kMinstdA64);
-      const uint32_t hi[1] = {x};
-      v.shift(hi);
-    }
+  // the group after the last
+  __device__ __forceinline__ void next() {
+    x = minstd_mul(x, kMinstdA64);
+    const uint32_t hi[1] = {x};
+    v.shift(hi);
   }
-  // the wave's next run
-  __device__ __forceinline__ void skip(uint32_t a_stride) { x0 = minstd_mul(x0, a_stride); }
   __device__ __forceinline__ uint64_t operator()(int j) const { return v.get(j); }
 };
 
@@ -94,87 +87,90 @@ void k_range_generate(const RangeArgs a) {
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t nruns = (ngroups + a.run - 1) / a.run;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kBlock / kWave);
-  uint64_t run = (uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave;
+  const uint64_t g_first = ((uint64_t)blockIdx.x * (kBlock / kWave) + (uint64_t)wave) * a.run;
+  if (g_first >= ngroups) return;  // wave-uniform
+  const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
   RangeWords<N> words;
-  words.first(a.x_start, run * a.run * kWave, lane);
-  for (; run < nruns; run += nwaves) {
-    const uint64_t g_first = run * a.run;
-    const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
-    for (uint64_t g = g_first; g < g_end; ++g) {
-      const uint64_t k0 = g * kWave;
-      words.next(win[wave], lane, g == g_first);
-      double p[N][4];
-      const double wt = range_event<N>(a.d, words, p);
-      if (k0 + (uint64_t)lane < a.n) {
-        double* c = a.cols + k0;
+  words.start(win[wave], a.x_start, g_first * kWave, lane);
+  for (uint64_t g = g_first;;) {
+    const uint64_t k0 = g * kWave;
+    double p[N][4];
+    const double wt = range_event<N>(a.d, words, p);
+    if (k0 + (uint64_t)lane < a.n) {
+      double* c = a.cols + k0;
 #pragma unroll
-        for (int i = 0; i < N; ++i)
+      for (int i = 0; i < N; ++i)
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, p[i][q]);
-        if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
-      }
+        for (int q = 0; q < 4; ++q)
+          st(uniform_ptr(c + (uint64_t)(4 * i + q) * a.ld) + lane, p[i][q]);
+      if (a.wt) st(uniform_ptr(a.wt + k0) + lane, wt);
     }
-    words.skip(a.a_stride);
+    if (++g == g_end) break;
+    words.next();
   }
 }
 
-// Threads of a fill's block: every block adds its bins to the contents in the
-// end, and those atomics, blocks times bins on few cache lines, not the
+// Most threads of a fill's block: every block adds its bins to the contents in
+// the end, and those atomics, blocks times bins on few cache lines, not the
 // elements set the time of smaller fills (1e6 elements into 100 bins: 2048
-// blocks of 256 threads 53 us, 512 of them 31).
+// blocks of 256 threads 53 us, 512 of them 31).  Fills of up to range_few_groups
+// groups of 64 into few bins take blocks of 256: one wave on each SIMD, whose
+// chains of dependent operations are the time (1001 8-body elements 15.4 us with
+// 512 threads, 13.1 with 256; 2e4 3-body ones 10.6, 10.1).  With 5e4 elements
+// 512 win up to 6 bodies (5: 12.3, 12.7) and lose beyond (8: 16.8, 14.7), and with
+// 10^4 bins the blocks' merges are the time (1001 3-body elements 11.2, 12.5).
 constexpr int kRangeHistBlock = 512;
+constexpr uint64_t range_few_groups(int N) { return N <= 6 ? 512 : 1024; }
+constexpr uint64_t kRangeFewSlots = 4096;
 
 template <int N>
 __global__ __launch_bounds__(kRangeHistBlock)
-    __attribute__((amdgpu_waves_per_eu(N <= 6 ? waves_for(N) : 2, 8)))
+    __attribute__((amdgpu_waves_per_eu(N <= 4 ? 4 : (N <= 6 ? 3 : 2), 8)))
 void k_range_hist(const RangeArgs a) {
   extern __shared__ double bins[];
   __shared__ typename RangeWords<N>::Window win[kRangeHistBlock / kWave];
   const uint64_t nslots = a.h.nbins + 2;
   if (a.use_lds) {
-    for (uint64_t b = threadIdx.x; b < nslots; b += kRangeHistBlock) bins[b] = 0.0;
+    for (uint64_t b = threadIdx.x; b < nslots; b += blockDim.x) bins[b] = 0.0;
     __syncthreads();
   }
   const int lane = __lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  const uint64_t nruns = (ngroups + a.run - 1) / a.run;
-  const uint64_t nwaves = (uint64_t)gridDim.x * (kRangeHistBlock / kWave);
-  uint64_t run = (uint64_t)blockIdx.x * (kRangeHistBlock / kWave) + (uint64_t)wave;
-  RangeWords<N> words;
-  words.first(a.x_start, run * a.run * kWave, lane);
-  for (; run < nruns; run += nwaves) {
-    const uint64_t g_first = run * a.run;
-    const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
-    for (uint64_t g = g_first; g < g_end; ++g) {
+  const uint64_t g_first =
+      ((uint64_t)blockIdx.x * (blockDim.x / kWave) + (uint64_t)wave) * a.run;
+  const uint64_t g_end = (g_first + a.run < ngroups) ? g_first + a.run : ngroups;
+  if (g_first < ngroups) {  // wave-uniform
+    RangeWords<N> words;
+    words.start(win[wave], a.x_start, g_first * kWave, lane);
+    for (uint64_t g = g_first;;) {
       const uint64_t k = g * kWave + (uint64_t)lane;
-      words.next(win[wave], lane, g == g_first);
       double p[N][4];
       const double wt = range_event<N>(a.d, words, p);
-      if (k >= a.n) continue;
-      double x[HPSP_HIST_MAX_DIM];
+      if (k < a.n) {
+        double x[HPSP_HIST_MAX_DIM];
 #pragma unroll
-      for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
-        x[d] = (d < a.h.ndim) ? functor_eval<double>(a.axes[d], p) : 0.0;
-      const double w = a.weight_mode == HPSP_HIST_WEIGHT_GENERATION ? wt
-                       : a.weight_mode == HPSP_HIST_WEIGHT_PHSP
-                           ? event_weight_f64<N>(p, a.d.m, a.d.maxw)
-                           : 1.0;
-      const uint64_t key = hist_key(a.h, x);
-      if (key == kDrop) continue;
-      if (a.use_lds)
-        atomicAdd(&bins[key], w);
-      else
-        unsafeAtomicAdd(&a.contents[key], w);
+        for (int d = 0; d < HPSP_HIST_MAX_DIM; ++d)
+          x[d] = (d < a.h.ndim) ? functor_late<true, true>(a.axes[d], p) : 0.0;
+        const double w = a.weight_mode == HPSP_HIST_WEIGHT_GENERATION ? wt
+                         : a.weight_mode == HPSP_HIST_WEIGHT_PHSP
+                             ? event_weight_f64<N>(p, a.d.m, a.d.maxw)
+                             : 1.0;
+        const uint64_t key = hist_key(a.h, x);
+        if (key != kDrop) {
+          if (a.use_lds)
+            atomicAdd(&bins[key], w);
+          else
+            unsafeAtomicAdd(&a.contents[key], w);
+        }
+      }
+      if (++g == g_end) break;
+      words.next();
     }
-    words.skip(a.a_stride);
   }
   if (a.use_lds) {
     __syncthreads();
-    for (uint64_t b = threadIdx.x; b < nslots; b += kRangeHistBlock) {
+    for (uint64_t b = threadIdx.x; b < nslots; b += blockDim.x) {
       const double v = bins[b];
       if (v != 0.0) unsafeAtomicAdd(&a.contents[b], v);
     }
@@ -183,15 +179,17 @@ void k_range_hist(const RangeArgs a) {
 
 // ---------------------------------------------------------------------------
 
-// Runs of the generation kernel as k_generate_f64's, dispatched in order
-// (bound by its stores up to 3 daughters); the events from a wave's run to its
-// next one are a power of a formed here.
+// One run per wave, dispatched in order.  The longest runs: 1 for 3 and 4 bodies,
+// whose stores bound them (4e6 3-body elements 72.7 us, runs of 2 78.4, of 4 81.5;
+// 2e6 35.5, 34.0, 34.0), 2 for 2 bodies (4e6: 55.5, 43.3, 44.0), 4 beyond (2e7
+// 6-body elements in runs of 1, 2, 4 and 16: 774, 738, 723, 776 us).
+constexpr uint32_t range_run_max(int N) { return N == 2 ? 2 : (N <= 4 ? 1 : 4); }
+
 template <int N>
 static void gen_one(RangeArgs a, hipStream_t s) {
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  a.run = run_groups(ngroups, N <= 3 ? kRunMaxStores : kRunMax);
-  const unsigned g = grid_for_runs((ngroups + a.run - 1) / a.run);
-  a.a_stride = minstd_pow((uint64_t)g * (kBlock / kWave) * a.run * kWave);
+  a.run = run_groups(ngroups, range_run_max(N));
+  const unsigned g = blocks_for_runs(ngroups, a.run);
   hipLaunchKernelGGL(k_range_generate<N>, dim3(g), dim3(kBlock), 0, s, a);
 }
 
@@ -203,17 +201,16 @@ static void hist_one(RangeArgs a, hipStream_t s) {
   // 8 waves per SIMD while the private bins are small, at least four groups per
   // wave beyond one block per CU
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  constexpr uint64_t kWaves = kRangeHistBlock / kWave;
+  const uint64_t block_waves =
+      ngroups <= range_few_groups(N) && nslots <= kRangeFewSlots ? kBlock / kWave
+                                                                 : kRangeHistBlock / kWave;
   const uint64_t cap = (a.use_lds && lds > 32768) ? 256 : 1024;
-  const uint64_t few = std::min<uint64_t>(256, (ngroups + kWaves - 1) / kWaves);
+  const uint64_t few = std::min<uint64_t>(256, (ngroups + block_waves - 1) / block_waves);
   const unsigned g = (unsigned)std::max(
-      few, std::min<uint64_t>(cap, (ngroups + 4 * kWaves - 1) / (4 * kWaves)));
-  // one run per wave: nothing is stored on the way
-  const uint64_t nwaves = g * kWaves;
-  const uint64_t per = (ngroups + nwaves - 1) / nwaves;
-  a.run = (uint32_t)(per < 1 ? 1 : (per < (1u << 20) ? per : (1u << 20)));
-  a.a_stride = minstd_pow(nwaves * a.run * kWave);
-  hipLaunchKernelGGL(k_range_hist<N>, dim3(g), dim3(kRangeHistBlock), lds, s, a);
+      few, std::min<uint64_t>(cap, (ngroups + 4 * block_waves - 1) / (4 * block_waves)));
+  const uint64_t nwaves = g * block_waves;
+  a.run = (uint32_t)((ngroups + nwaves - 1) / nwaves);
+  hipLaunchKernelGGL(k_range_hist<N>, dim3(g), dim3((unsigned)(block_waves * kWave)), lds, s, a);
 }
 
 template <int... I>

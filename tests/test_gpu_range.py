@@ -7,10 +7,13 @@ Bars: weights bit for bit (built from + - * / sqrt only); momenta within
 histogram puts every element in the bin of the oracle's element (unit-weight
 counts exact), weighted sums to rounding (1e-13 of the bin's sum of |w|).
 """
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
-from gpu_util import momentum_error, range_generate, range_histogram
+from gpu_util import DEV, momentum_error, range_generate, range_histogram
 from hydra_amd import capi
 from hydra_amd.capi import make_functor
 
@@ -179,3 +182,60 @@ def test_range_histogram_equals_fill_of_generated(oracle):
     torch.cuda.synchronize()
     assert np.array_equal(fused, out.cpu().numpy())
     assert fused.sum() == n
+
+
+@pytest.mark.parametrize("N,n", [(2, (1 << 20) + 77), (2, (1 << 22) + 4321), (3, (1 << 20) + 77),
+                                 (5, (1 << 20) + 77), (5, (1 << 21) + 4321),
+                                 (12, (1 << 21) + 4321)])
+def test_runs_equal_short_calls(N, n):
+    """A wave's runs of 1, 2 and 4 groups of 64 elements, which carry the engine's
+    words from group to group, against calls too short for them, at the run's
+    edges, beside them and at the ragged end."""
+    m4, m = random_range(np.random.default_rng(40 + N), N)
+    dec = capi.make_range(m4, m)
+    first = 987654321
+
+    def call(b, k):
+        cols = torch.empty((4 * N, k), dtype=torch.float64, device=DEV)
+        wt = torch.empty(k, dtype=torch.float64, device=DEV)
+        capi.check(capi.lib().hpsp_range_generate(ctypes.byref(dec), 5, first + b, k,
+                                                  capi.ptr(cols), k, capi.ptr(wt),
+                                                  capi.stream_handle()), "range")
+        return cols, wt
+
+    cols, wt = call(0, n)
+    mid = n // 2 // 1024 * 1024
+    for b, k in ((0, 1500), (mid - 300, 1500), (mid + 37, 700), (n - 1500, 1500)):
+        c, w = call(b, k)
+        assert torch.equal(cols[:, b:b + k], c)
+        assert torch.equal(wt[b:b + k], w)
+
+
+@pytest.mark.parametrize("N", [2, 3, 8])
+@pytest.mark.parametrize("n,bins", [(63, 50), (64 * 512, 4094), (64 * 512 + 1, 4094),
+                                    (64 * 512, 4095), (64 * 1024, 50), (64 * 1024 + 1, 50),
+                                    ((1 << 20) + 77, 50)])
+def test_range_histogram_blocks(N, n, bins):
+    """Blocks of 4 and of 8 waves, at the elements and bins where the launcher
+    changes between them, and runs of several groups: the counts of the generated
+    elements' masses as columns."""
+    m4, m = random_range(np.random.default_rng(60 + N), N)
+    dec = capi.make_range(m4, m)
+    axis = make_functor(capi.F_MASS, (0, N - 1))
+    lim = [0.9 * (m[0] + m[N - 1])], [1.05 * dec.mother_mass]
+    got = range_histogram([bins], *lim, dec, 9, [axis], n)
+    cols = torch.empty((4 * N, n), dtype=torch.float64, device=DEV)
+    capi.check(capi.lib().hpsp_range_generate(ctypes.byref(dec), 9, 0, n, capi.ptr(cols), n, None,
+                                              capi.stream_handle()), "range")
+    p = capi.Particles()
+    p.n = N
+    for i in range(N):
+        p.cols[i], p.ld[i] = cols.data_ptr() + 32 * n * i, n
+    x = torch.empty((1, n), dtype=torch.float64, device=DEV)
+    capi.check(capi.lib().hpsp_particles_evaluate(ctypes.byref(p), capi.functor_array([axis]), 1,
+                                                  n, capi.ptr(x), n, capi.stream_handle()), "axis")
+    h = capi.make_histogram([bins], *lim)
+    out = torch.empty(bins + 2, dtype=torch.float64, device=DEV)
+    capi.check(capi.lib().hpsp_histogram_fill(ctypes.byref(h), capi.ptr(x), n, n, None,
+                                              capi.ptr(out), capi.stream_handle()), "fill")
+    assert np.array_equal(got, out.cpu().numpy()) and got.sum() == n
