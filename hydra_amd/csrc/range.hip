@@ -179,16 +179,23 @@ void k_range_hist(const RangeArgs a) {
 
 // ---------------------------------------------------------------------------
 
-// One run per wave, dispatched in order.  The longest runs: 1 for 3 and 4 bodies,
-// whose stores bound them (4e6 3-body elements 72.7 us, runs of 2 78.4, of 4 81.5;
-// 2e6 35.5, 34.0, 34.0), 2 for 2 bodies (4e6: 55.5, 43.3, 44.0), 4 beyond (2e7
-// 6-body elements in runs of 1, 2, 4 and 16: 774, 738, 723, 776 us).
-constexpr uint32_t range_run_max(int N) { return N == 2 ? 2 : (N <= 4 ? 1 : 4); }
+// One run per wave, dispatched in order.  The longest runs: of 3 and 4 bodies, whose
+// stores bound them, 1 up to 2^25 elements (4e6 3-body elements 72.7 us, runs of 2
+// 78.4, of 4 81.5; 2e6 35.5, 34.0, 34.0; 2^25 620, of 4 621) and 4 or 16 beyond
+// (2^27 K+ -> 3 pi 2595 us in runs of 1, 2059 of 4; 4 bodies 3583, 3159 of 16); 2
+// for 2 bodies (4e6: 55.5, 43.3, 44.0); 4 for more than 4 (2e7 6-body elements in
+// runs of 1, 2, 4 and 16: 774, 738, 723, 776 us).
+constexpr uint64_t kRangeLongRuns = 1 << 25;  // elements
+inline uint32_t range_run_max(int N, uint64_t n) {
+  if (N == 2) return 2;
+  if (N >= 5) return 4;
+  return n <= kRangeLongRuns ? 1 : (N == 3 ? 4 : 16);
+}
 
 template <int N>
 static void gen_one(RangeArgs a, hipStream_t s) {
   const uint64_t ngroups = (a.n + kWave - 1) / kWave;
-  a.run = run_groups(ngroups, range_run_max(N));
+  a.run = run_groups(ngroups, range_run_max(N, a.n));
   const unsigned g = blocks_for_runs(ngroups, a.run);
   hipLaunchKernelGGL(k_range_generate<N>, dim3(g), dim3(kBlock), 0, s, a);
 }

@@ -186,9 +186,10 @@ def test_range_histogram_equals_fill_of_generated(oracle):
 
 @pytest.mark.parametrize("N,n", [(2, (1 << 20) + 77), (2, (1 << 22) + 4321), (3, (1 << 20) + 77),
                                  (5, (1 << 20) + 77), (5, (1 << 21) + 4321),
+                                 (3, (1 << 25) + 77), (4, (1 << 25) + 4321),
                                  (12, (1 << 21) + 4321)])
 def test_runs_equal_short_calls(N, n):
-    """A wave's runs of 1, 2 and 4 groups of 64 elements, which carry the engine's
+    """A wave's runs of 1, 2, 4 and 16 groups of 64 elements, which carry the engine's
     words from group to group, against calls too short for them, at the run's
     edges, beside them and at the ragged end."""
     m4, m = random_range(np.random.default_rng(40 + N), N)
