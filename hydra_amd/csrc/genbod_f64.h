@@ -21,10 +21,10 @@
 // model over 2^24 events from 239 to 221 us, Evaluate of 10^7 events from 174 to
 // 164 us.  gamma from gamma beta (one square root, no selects), the first
 // boost's back-to-back pair formed once and no guard on the energies' square
-// roots: 1e6 3-body events 20.1 -> 18.8 us, the 10-body Generate 1.47 -> 1.44 ms,
-// AverageOn 208 -> 199 us, Evaluate 145 -> 137 us.  The momenta's errors against
-// extended precision did not grow (3 bodies: 2.28 -> 2.24e-16 E RMS; 10: 1.51 ->
-// 1.47e-15).
+// roots: AverageOn 208 -> 199 us, the 10-body Generate and Evaluate 2-5%
+// in one run.  Now, in other runs, 1e6 3-body events 21-23 us, the 10-body Generate
+// 1.50 ms, AverageOn 197 us, Evaluate 143 us.  The momenta's errors against extended
+// precision did not grow (3 bodies: 2.28 -> 2.24e-16 E RMS; 10: 1.51 -> 1.47e-15).
 #pragma once
 
 #include <type_traits>

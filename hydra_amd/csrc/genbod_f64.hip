@@ -19,7 +19,7 @@ namespace hpsp {
 // (xcd_block).
 // COLS = false is the weights pass of a deferred Generate (no momentum columns).
 // Against runs of up to 16 groups per wave (91 registers and 5 waves per SIMD
-// for 3 bodies, 142 and 3 for 10; now 56 and 8, 120 and 4): 1e6 3-body events
+// for 3 bodies, 142 and 3 for 10; now 54 and 8, 118 and 4): 1e6 3-body events
 // 23.3 -> 20.1 us, 3e6 4-body Threefry ones 101 -> 86 us, 2^24 10-body ones 1.50
 // -> 1.47 ms, mixed near threshold 653 -> 608 us, Evaluate of 1e7 164 -> 148 us.
 template <int N, int ENGINE, bool MOTHERS, bool COLS = true>

@@ -319,7 +319,7 @@ void k_uw_flags_chain(const UnweightArgs a, uint64_t* dl_count, uint64_t* dl, co
   [[maybe_unused]] const double2* XY3 = reinterpret_cast<const double2*>(tab3);
   const uint64_t off = (uint64_t)wave * (kItems * kWave) + (uint64_t)lane;
   // key * (jump + k) of item 0 for the accept word and key * (gen_first + k +
-  // 3N) for the generation word; item j + 1 is kBlock events on
+  // 3N) for the generation word; item j + 1 is kWave events on
   uint64_t ykey = a.uw_key * (a.jump + tile * kUwTile + off);
   const uint64_t ystep = a.uw_key * (uint64_t)kWave;
   uint64_t ygen = a.d.key[0] * (a.gen_first + tile * kUwTile + off + 3 * (uint64_t)N);
